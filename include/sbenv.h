@@ -458,18 +458,18 @@ typedef struct {
     long long nnz_l, nnz_u;       /* off-diagonal factor entries */
     double bytes_per_step;        /* algorithmic HBM bytes of one batched step */
     double flops_per_step;        /* multiply-adds x 2 of the solves and the air-side combination */
-    int tail_rows_l, tail_rows_u;       /* rows of each sweep's LDS run (0: exact mode) */
-    int tail_levels_l, tail_levels_u;   /* levels of the LDS run */
-    int chunked_levels_l, chunked_levels_u;   /* levels after it solved chunked from HBM */
+    int tail_rows_l, tail_rows_u;       /* rows in fronts above the leaves (0: exact mode) */
+    int tail_levels_l, tail_levels_u;   /* heights of the tree of fronts above the leaves (0: exact mode) */
+    int chunked_levels_l, chunked_levels_u;   /* always 0 */
 } SbxFdmInfo;
-/* Flags of sbx_fdm_open. Default: each sweep's longest run of narrow levels
- * (at most 64 rows each: the separators at the top of the elimination tree,
- * as many as fit) runs with its rows in LDS, and the levels after it with
- * each row's terms spread over lanes; row sums are formed in another order,
- * so results agree with the reference to rounding, far inside 1e-9
- * relative. SBX_FDM_EXACT: every level from HBM in the reference's order,
- * bit-identical results. envs_per_block 0 picks 1 (default; 2 when there
- * are more envs than the GPU has compute units) or up to 64 (exact). The default mode also takes the air-side correction from the
+/* Flags of sbx_fdm_open. Default: the factors' rows grouped along their
+ * elimination tree into dense fronts, whose inverses and couplings are formed
+ * at open; a step's solve is one matrix product per front up the tree and one
+ * down it, so row sums are formed in another order and results agree with the
+ * reference to rounding, far inside 1e-9 relative. SBX_FDM_EXACT: every level
+ * in the reference's order, bit-identical results. envs_per_block (envs that
+ * share a block of the field's layout) 0 picks 1 (default) or up to 64
+ * (exact). The default mode also takes the air-side correction from the
  * responses of the applied columns (sbx_fdm_air_responses) instead of a
  * second solve per step. */
 #define SBX_FDM_EXACT 1

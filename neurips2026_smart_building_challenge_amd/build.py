@@ -36,11 +36,13 @@ HIP_FLAGS = [
 
 # the field step and the field envs' HVAC lanes are bit-exact to the reference
 # core only with products rounded before they are added
-EXTRA = {"fdm_kernel.hip": ["-ffp-contract=off"], "field_env_kernel.hip": ["-ffp-contract=off"]}
+EXTRA = {"fdm_kernel.hip": ["-ffp-contract=off"], "fdm_front_kernel.hip": ["-ffp-contract=off"],
+         "field_env_kernel.hip": ["-ffp-contract=off"]}
 
 
-HIP_SOURCES = ["step_kernel.hip", "policy_kernel.hip", "canon_kernel.hip", "fdm_kernel.hip", "field_env_kernel.hip"]
-HOST_SOURCES = ["vec.cpp", "plan.cpp", "sbb_reader.cpp", "fdm.cpp", "field_env.cpp"]
+HIP_SOURCES = ["step_kernel.hip", "policy_kernel.hip", "canon_kernel.hip", "fdm_kernel.hip", "fdm_front_kernel.hip",
+               "field_env_kernel.hip"]
+HOST_SOURCES = ["vec.cpp", "plan.cpp", "sbb_reader.cpp", "fdm.cpp", "fdm_front.cpp", "field_env.cpp"]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:

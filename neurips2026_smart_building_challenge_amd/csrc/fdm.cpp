@@ -1,6 +1,7 @@
 // Host side of the building-scale field step (sbx_fdm_*): reads a blob's
 // field sections (the ones complete_port/csim/sb_fdm.c:40-118 reads), checks
-// them, turns the baked CSC factors into level-ordered row solves, uploads
+// them, turns the baked CSC factors into level-ordered row solves (exact
+// mode, and the solves at open) and dense fronts (the default mode), uploads
 // every table once and owns the group's device buffers.
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
@@ -11,11 +12,14 @@
 #include <vector>
 
 #include "fdm.h"
+#include "fdm_front.h"
 #include "fdm_host.h"
 #include "sbb_reader.h"
 #include "sbenv.h"
 
-extern "C" int sbf_run_lds_limit(int bytes);
+extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, const int* front_of, const int* local,
+                                    const int* bperm, const long long* d0, const long long* s0, double* dense,
+                                    double* sol, double* ops);
 extern "C" int sbf_launch_solve_cols(const sbf::Tables* t, const sbf::Group* g, const double* b, double* x,
                                      double* S, hipStream_t s);
 
@@ -100,131 +104,6 @@ void level_order(const std::vector<std::vector<std::pair<int, double>>>& terms, 
     if (out->diag.empty()) out->diag.push_back(1.0);
 }
 
-// Runs of the default mode (see sbf::Tail and sbf::Sweep). The LDS run is the
-// longest run of consecutive levels with at most kTailRows rows each, cut from
-// its side that borders wider levels until its row values and one level's
-// chunk partials fit in kRunLds bytes for Gl envs.
-constexpr int kTailRows = 64;
-constexpr size_t kRunLds = 152 * 1024;
-constexpr int kWaveFinishRows = 16;   // levels with more rows (some long) finish one row per lane
-
-struct RunHost {
-    int lds = 0, lev0 = 0, m = 0, nlev = 0, max_chunks = 0;
-    std::vector<int> rows, hptr, hcol, trow, tchunk, tmode, rchunk, cpos;
-    std::vector<double> diag, hval, cval;
-    size_t need(int Gl) const { return (size_t)((lds ? m : 0) + max_chunks) * Gl * 8; }
-};
-
-struct LevelOf {
-    // level of a row (-1: not scheduled, final from the start), its position in level order
-    std::vector<int> lvl, q_of;
-    LevelOf(const TriHost& T, int n) : lvl(n, -1), q_of(n, -1) {
-        for (int l = 0; l < T.nlev; l++)
-            for (int q = T.lev[l]; q < T.lev[l + 1]; q++) lvl[T.rows[q]] = l;
-        for (size_t q = 0; q < T.rows.size(); q++) q_of[T.rows[q]] = (int)q;
-    }
-};
-
-void lay_run(const TriHost& T, const LevelOf& V, int lev0, int lev1, bool lds, int Gl, RunHost* out) {
-    const int nr = (int)T.rows.size();
-    const int q0 = T.lev[lev0];
-    RunHost& o = *out;
-    o = RunHost();
-    o.lds = lds;
-    o.lev0 = lev0;
-    o.m = T.lev[lev1] - q0;
-    o.nlev = lev1 - lev0;
-    o.hptr.push_back(0);
-    o.rchunk.push_back(0);
-    for (int t = 0; t < o.nlev; t++) {
-        o.trow.push_back(T.lev[lev0 + t] - q0);
-        o.tchunk.push_back((int)o.cpos.size() / sbf::kChunk);
-        int most = 0;
-        for (int q = T.lev[lev0 + t]; q < T.lev[lev0 + t + 1]; q++) {
-            o.rows.push_back(T.rows[q]);
-            if ((int)T.diag.size() == nr) o.diag.push_back(T.diag[q]);
-            int cnt = 0;
-            for (int e = T.ptr[q]; e < T.ptr[q + 1]; e++) {
-                const int j = T.col[e];
-                if (!lds) {
-                    o.cpos.push_back(j);
-                } else if (V.lvl[j] >= lev0) {   // a row reads earlier levels only: lvl[j] < lev0 + t
-                    o.cpos.push_back(V.q_of[j] - q0);
-                } else {
-                    o.hcol.push_back(j);
-                    o.hval.push_back(T.val[e]);
-                    continue;
-                }
-                o.cval.push_back(T.val[e]);
-                cnt++;
-            }
-            while (cnt % sbf::kChunk) {
-                o.cpos.push_back(0);
-                o.cval.push_back(0.0);
-                cnt++;
-            }
-            o.hptr.push_back((int)o.hcol.size());
-            o.rchunk.push_back((int)o.cpos.size() / sbf::kChunk);
-            most = std::max(most, cnt / sbf::kChunk);
-        }
-        const int nrows = T.lev[lev0 + t + 1] - T.lev[lev0 + t];
-        const int mode = most <= 1 ? 0 : nrows > kWaveFinishRows ? 1 : most > 64 / Gl ? 2 : 3;
-        o.tmode.push_back(mode);
-        if (mode == 1 || mode == 2)
-            o.max_chunks = std::max(o.max_chunks, (int)o.cpos.size() / sbf::kChunk - o.tchunk.back());
-    }
-    o.trow.push_back(o.m);
-    o.tchunk.push_back((int)o.cpos.size() / sbf::kChunk);
-    for (auto* v : {&o.rows, &o.hcol, &o.cpos, &o.tmode})
-        if (v->empty()) v->push_back(0);
-    for (auto* v : {&o.diag, &o.hval, &o.cval})
-        if (v->empty()) v->push_back(1.0);
-}
-
-struct SweepHost {
-    int pre_end = 0, post_begin = 0, pre_chunked = 0, post_chunked = 0;
-    RunHost pre, mid, post;
-};
-
-void plan_sweep(const TriHost& T, int n, int Gl, SweepHost* out) {
-    const LevelOf V(T, n);
-    auto narrow = [&](int l) { return T.lev[l + 1] - T.lev[l] <= kTailRows; };
-    int a = 0, b = 0;   // the longest run [a, b) of narrow levels
-    for (int l = 0; l < T.nlev;) {
-        if (!narrow(l)) { l++; continue; }
-        int e = l;
-        while (e < T.nlev && narrow(e)) e++;
-        if (e - l > b - a) { a = l; b = e; }
-        l = e;
-    }
-    RunHost& mid = out->mid;
-    auto need = [&](int lo, int hi) {
-        lay_run(T, V, lo, hi, true, Gl, &mid);
-        return mid.need(Gl);
-    };
-    if (b > a && need(a, b) > kRunLds) {
-        // cut the side that borders wider levels (for the L sweep the run ends
-        // the schedule, for the U sweep it starts it); fewer levels need less
-        // LDS, so bisect for the longest run that fits
-        const bool keep_end = b == T.nlev;
-        int lo = 0, hi = b - a;   // levels kept
-        while (lo < hi) {
-            const int mid_n = lo + (hi - lo + 1) / 2;
-            if (need(keep_end ? b - mid_n : a, keep_end ? b : a + mid_n) <= kRunLds) lo = mid_n;
-            else hi = mid_n - 1;
-        }
-        if (keep_end) a = b - lo;
-        else b = a + lo;
-    }
-    lay_run(T, V, a, b, true, Gl, &mid);
-    out->pre_end = a;
-    out->post_begin = b;
-    lay_run(T, V, 0, a, false, Gl, &out->pre);
-    out->pre_chunked = out->pre.nlev > 0 && out->pre.need(Gl) <= kRunLds;
-    lay_run(T, V, b, T.nlev, false, Gl, &out->post);
-    out->post_chunked = out->post.nlev > 0 && out->post.need(Gl) <= kRunLds;
-}
-
 bool csc_ok(const sbh::Blob& b, const char* name, int n_rows, int n_cols, const int32_t** p, const int32_t** ix,
             const double** x, uint64_t* nnz) {
     uint64_t np = 0, ni = 0, nx = 0;
@@ -266,6 +145,11 @@ void* dalloc(SbxFdm* f, size_t bytes) {
     return p;
 }
 
+bool hip_check(hipError_t e, const char* what) {
+    if (e == hipSuccess) return true;
+    return fail(std::string(what) + ": " + hipGetErrorString(e));
+}
+
 // Device buffers of a group of G envs in blocks of Gl lanes.
 bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     const sbf::Tables& t = f->tab;
@@ -273,9 +157,15 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     g->Gl = Gl;
     g->nblk = (G + Gl - 1) / Gl;
     const size_t lanes = (size_t)g->nblk * Gl;
-    g->W1 = (double*)dalloc(f, sizeof(double) * lanes * t.n);
-    const bool w2 = fields && !t.R;   // the second solve's vector (exact mode)
+    const bool fronts = fields && t.fast;   // the default mode's vectors, in tiles of envs
+    g->nt = (G + sbf::kEnvTile - 1) / sbf::kEnvTile;
+    const size_t tl = (size_t)g->nt * sbf::kEnvTile, c_rows = (size_t)t.ft.n_c + 1;
+    g->W1 = (double*)dalloc(f, sizeof(double) * (fronts ? tl : lanes) * t.n);
+    const bool w2 = fields && !t.fast;   // the second solve's vector (exact mode)
     g->W2 = w2 ? (double*)dalloc(f, sizeof(double) * lanes * t.n) : nullptr;
+    g->X = fronts ? (double*)dalloc(f, sizeof(double) * tl * t.n) : nullptr;
+    g->Y = fronts ? (double*)dalloc(f, sizeof(double) * tl * std::max(t.n - t.ft.n_leaf, 1)) : nullptr;
+    g->C = fronts ? (double*)dalloc(f, sizeof(double) * tl * c_rows) : nullptr;
     g->T = fields ? (double*)dalloc(f, sizeof(double) * lanes * t.n_cvs) : nullptr;
     g->M = fields ? (double*)dalloc(f, sizeof(double) * lanes * t.n) : nullptr;
     const size_t k = std::max(t.k, 1);
@@ -283,14 +173,11 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     g->mat = fields ? (double*)dalloc(f, sizeof(double) * G * k * k) : nullptr;
     g->eact = (int*)dalloc(f, sizeof(int) * G);
     g->bact = (int*)dalloc(f, sizeof(int) * g->nblk);
-    if (!g->W1 || !g->pw || !g->eact || !g->bact || (w2 && !g->W2) || (fields && (!g->T || !g->M || !g->mat)))
+    if (!g->W1 || !g->pw || !g->eact || !g->bact || (w2 && !g->W2) || (fields && (!g->T || !g->M || !g->mat))
+        || (fronts && (!g->X || !g->Y || !g->C)))
         return fail("hipMalloc failed for the field buffers");
-    return true;
-}
-
-bool hip_check(hipError_t e, const char* what) {
-    if (e == hipSuccess) return true;
-    return fail(std::string(what) + ": " + hipGetErrorString(e));
+    // C's zero rows (the contributions are written before they are read)
+    return !fronts || hip_check(hipMemset(g->C, 0, sizeof(double) * tl * c_rows), "clear the front contributions");
 }
 
 bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
@@ -371,6 +258,24 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     TriHost L, U;
     level_order(lt, nullptr, false, &L);
     level_order(ut, &udiag, true, &U);
+    const bool exact = (flags & SBX_FDM_EXACT) != 0;
+    sbf::FrontPlan fp;
+    std::vector<long double> rsum(exact ? 0 : n);   // L U 1 by row of the permuted system
+    if (!exact) {
+        sbf::plan_fronts(lt, ut, &fp);
+        // in 64-bit mantissas: a row's entries cancel to a tenth of the diagonal
+        std::vector<long double> u1(n);
+        for (int i = 0; i < n; i++) {
+            long double v = udiag[i];
+            for (const auto& e : ut[i]) v += e.second;
+            u1[i] = v;
+        }
+        for (int i = 0; i < n; i++) {
+            long double v = u1[i];
+            for (const auto& e : lt[i]) v += e.second * u1[e.first];
+            rsum[i] = v;
+        }
+    }
     lt.clear();
     ut.clear();
 
@@ -486,54 +391,49 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     };
     put_tri(&T.L, L);
     put_tri(&T.U, U);
-    // envs per block: as asked; by default one (the default mode keeps a run's
-    // rows in LDS per env), two once the group has more than 256 envs, the
-    // MI355X's compute-unit count (a block's level chain then serves two envs:
-    // 512 envs of a 205K-cell plan 18.6 -> 17.5 ms per step, 1,024 envs
-    // 28.2 ms; four were slower), or, in exact mode, up to 64. The threshold
-    // is a constant, not the device's count: the default mode's sums are
-    // reassociated by the block width, so an env's rounding depends on the
-    // group size only (both widths are held to the reference within 1e-9)
-    const bool exact = (flags & SBX_FDM_EXACT) != 0;
-    constexpr int kTwoPerBlockAbove = 256;
-    const int dflt = exact ? 64 : (G > kTwoPerBlockAbove ? 2 : 1);
-    const int gl = std::min(64, next_pow2(std::min(G, epb > 0 ? epb : dflt)));
+    // envs per block of the field's layout: as asked; by default one (the
+    // default mode's solve has its own layout), or, in exact mode, up to 64
+    const int gl = std::min(64, next_pow2(std::min(G, epb > 0 ? epb : exact ? 64 : 1)));
     T.fast = exact ? 0 : 1;
-    SweepHost sl, su;
+    size_t o_front = 0, o_local = 0, o_bperm = 0, o_d0 = 0, o_s0 = 0;   // for the operators, at open only
+    size_t dense_n = 0, sol_n = 0;
     if (T.fast) {
-        plan_sweep(L, n, gl, &sl);
-        plan_sweep(U, n, gl, &su);
-    }
-    auto put_run = [&](sbf::Tail* d, const RunHost& h) {
-        d->lds = h.lds;
-        d->lev0 = h.lev0;
-        d->m = h.m;
-        d->nlev = h.nlev;
-        d->max_chunks = h.max_chunks;
-        put((const void**)&d->rows, A.vec(h.rows));
-        put((const void**)&d->diag, A.vec(h.diag));
-        put((const void**)&d->hptr, A.vec(h.hptr));
-        put((const void**)&d->hcol, A.vec(h.hcol));
-        put((const void**)&d->hval, A.vec(h.hval));
-        put((const void**)&d->trow, A.vec(h.trow));
-        put((const void**)&d->tchunk, A.vec(h.tchunk));
-        put((const void**)&d->tmode, A.vec(h.tmode));
-        put((const void**)&d->rchunk, A.vec(h.rchunk));
-        put((const void**)&d->cpos, A.vec(h.cpos));
-        put((const void**)&d->cval, A.vec(h.cval));
-    };
-    auto put_sweep = [&](sbf::Sweep* d, const SweepHost& h) {
-        d->pre_end = h.pre_end;
-        d->post_begin = h.post_begin;
-        d->pre_chunked = h.pre_chunked;
-        d->post_chunked = h.post_chunked;
-        put_run(&d->mid, h.mid);
-        if (h.pre_chunked) put_run(&d->pre, h.pre);
-        if (h.post_chunked) put_run(&d->post, h.post);
-    };
-    if (T.fast) {
-        put_sweep(&T.SL, sl);
-        put_sweep(&T.SU, su);
+        sbf::FrontTab& ft = T.ft;
+        ft.n_fronts = (int)fp.fronts.size();
+        ft.n_levels = (int)fp.levels.size();
+        ft.n_leaf = fp.n_leaf;
+        ft.n_c = fp.n_c;
+        f->front_levels = fp.levels;
+        ft.levels = f->front_levels.data();
+        put((const void**)&ft.fronts, A.vec(fp.fronts));
+        put((const void**)&ft.brow, A.vec(fp.brow));
+        put((const void**)&ft.arow, A.vec(fp.arow));
+        put((const void**)&ft.xsrc, A.vec(fp.xsrc));
+        put((const void**)&ft.tasks, A.vec(fp.tasks));
+        std::vector<int> rf(n), rx(n), snf(snw.size());
+        std::vector<double> rst(n);
+        for (int i = 0; i < n; i++) {
+            rf[ir[i]] = fp.pos[i];
+            rst[ir[i]] = (double)(rsum[i] - cap[ir[i]] - mc[ir[i]]);
+        }
+        for (int t = 0; t < n; t++) rx[t] = fp.pos[pcv[t]];
+        for (size_t e = 0; e < snw.size(); e++) snf[e] = fp.pos[snw[e]];
+        put((const void**)&ft.rf, A.vec(rf));
+        put((const void**)&ft.rx, A.vec(rx));
+        put((const void**)&ft.sn_w, A.vec(snf));
+        put((const void**)&ft.rowsum, A.vec(rst));
+        std::vector<long long> d0, s0;
+        for (const sbf::Front& q : fp.fronts) {
+            d0.push_back((long long)dense_n);
+            s0.push_back((long long)sol_n);
+            dense_n += 2 * (size_t)q.w * ((size_t)q.w + q.r);
+            sol_n += (size_t)q.w * ((size_t)q.w + 2 * q.r);
+        }
+        o_front = A.vec(fp.front_of);
+        o_local = A.vec(fp.local);
+        o_bperm = A.vec(fp.bperm);
+        o_d0 = A.vec(d0);
+        o_s0 = A.vec(s0);
     }
     put((const void**)&T.sn_p, A.add(sp, 4 * (size_t)(k + 1)));
     put((const void**)&T.sn_w, A.vec(snw));
@@ -547,7 +447,25 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     if (!hip_check(hipMemcpy(f->d_tables, A.host.data(), A.host.size(), hipMemcpyHostToDevice), "upload field tables"))
         return false;
     for (auto& e : fix) *e.first = f->d_tables + e.second;
-    if (T.fast && !hip_check((hipError_t)sbf_run_lds_limit((int)kRunLds), "run LDS limit")) return false;
+    if (T.fast) {
+        // the fronts' operators, formed on the device from the factors' rows
+        double *dense = nullptr, *sol = nullptr, *ops = (double*)dalloc(f, 8 * fp.ops);
+        bool ok = ops && hip_check(hipMalloc(&dense, 8 * dense_n), "hipMalloc(front blocks)")
+                  && hip_check(hipMalloc(&sol, 8 * sol_n), "hipMalloc(front solutions)")
+                  && hip_check(hipMemset(dense, 0, 8 * dense_n), "clear front blocks");
+        T.ft.ops = ops;
+        auto at = [&](size_t off) { return (const void*)(f->d_tables + off); };
+        ok = ok
+             && hip_check((hipError_t)sbf_launch_front_ops(&T, (int)L.rows.size(), (int)U.rows.size(),
+                                                           (const int*)at(o_front), (const int*)at(o_local),
+                                                           (const int*)at(o_bperm), (const long long*)at(o_d0),
+                                                           (const long long*)at(o_s0), dense, sol, ops),
+                          "front operators")
+             && hip_check(hipDeviceSynchronize(), "front operators");
+        (void)hipFree(dense);
+        (void)hipFree(sol);
+        if (!ok) return ops ? false : fail("hipMalloc failed for the front operators");
+    }
     if (!hip_check(hipMalloc(&f->d_temp_init, 8 * (size_t)n_cvs), "hipMalloc(temp_init)")) return false;
     if (!hip_check(hipMalloc(&f->d_mass_init, 8 * (size_t)n), "hipMalloc(mass_temp_init)")) return false;
     if (!hip_check(hipMemcpy(f->d_temp_init, tinit, 8 * (size_t)n_cvs, hipMemcpyHostToDevice), "upload temp_init")
@@ -593,12 +511,9 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     I.levels_u = U.nlev;
     I.nnz_l = L.nnz;
     I.nnz_u = U.nnz;
-    I.tail_rows_l = T.fast ? sl.mid.m : 0;
-    I.tail_rows_u = T.fast ? su.mid.m : 0;
-    I.tail_levels_l = T.fast ? sl.mid.nlev : 0;
-    I.tail_levels_u = T.fast ? su.mid.nlev : 0;
-    I.chunked_levels_l = T.fast && sl.post_chunked ? sl.post.nlev : 0;
-    I.chunked_levels_u = T.fast && su.post_chunked ? su.post.nlev : 0;
+    I.tail_rows_l = I.tail_rows_u = T.fast ? n - T.ft.n_leaf : 0;
+    I.tail_levels_l = I.tail_levels_u = T.fast ? T.ft.n_levels - 1 : 0;
+    I.chunked_levels_l = I.chunked_levels_u = 0;
     // algorithmic HBM bytes of one batched step: both factors read once per
     // solve for the whole group (value + column per term, U's diagonal, row
     // ids and row pointers: shared by every env, however the blocks re-read

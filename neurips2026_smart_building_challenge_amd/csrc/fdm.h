@@ -6,7 +6,8 @@
 // into nblk blocks of Gl lanes (the last block may hold fewer envs), and every
 // per-env field array is block-major, env-minor: element (cell or row x, env
 // b * Gl + l) of array A sits at A[(b * rows + x) * Gl + l], so the envs of a
-// block read one row as Gl adjacent doubles. The solve works on the permuted
+// block read one row as Gl adjacent doubles. The default mode's solve has
+// vectors of its own, in tiles of kEnvTile envs. The solve works on the permuted
 // vector of the baked factorization (SuperLU convention, complete_port/csim/
 // sb_lu.c:38-63): w[i] = b[ir[i]], L w' = w, U z = w', x[t] = z[pc[t]].
 #pragma once
@@ -30,52 +31,77 @@ struct Tri {
     const double* diag;
 };
 
-// A run of consecutive levels lev0 .. lev0 + nlev - 1 of a factor's Tri,
-// solved level by level by one workgroup per block with each row's terms cut
-// into chunks of kChunk spread over the lanes (partial sums in LDS, then one
-// wavefront per row, or one lane per row where no row of the level has more
-// than one chunk, adds them and finishes the row). Two kinds:
-//   lds = 1: the run's own row values live in LDS for its duration (the narrow
-//     levels at the top of the elimination tree: the last levels of the L
-//     sweep, the first of the U sweep); terms on earlier levels ("head" terms,
-//     final before the run starts) per row in [hptr[r], hptr[r + 1]) of
-//     (hcol, hval) are applied first, and chunk positions index the run;
-//   lds = 0: values stay in HBM and chunk positions are row ids.
-// Rows in level order r = 0 .. m-1 (rows[r]); level t spans chunks
-// [tchunk[t], tchunk[t + 1]) and rows [trow[t], trow[t + 1]); row r's chunks
-// are [rchunk[r], rchunk[r + 1]). tmode[t]: 0 no row of the level has more
-// than one chunk (each lane finishes its rows directly, no partials); 1 and 2
-// chunks spread over all lanes, partials in LDS, rows finished one lane each
-// (1, wide levels) or one wavefront each (2, a few rows longer than a
-// wavefront's lanes); 3 one wavefront per row, no partials. Padding terms are
-// (0, 0.0).
-constexpr int kChunk = 8;
+// The default mode's form of the same two factors: dense fronts.
+//
+// The rows of the permuted system are grouped along the elimination tree of
+// the factors' union pattern (closed under fill): whole subtrees of at most
+// kLeafCols columns are one front each (the leaves), and above them chains of
+// columns are merged while the merged block stays nearly dense. A front with
+// columns C (w of them) and boundary B (the r later rows its columns reach)
+// needs two dense operators, formed once at open from L and U:
+//   F = -L_BC L_CC^-1                        [r][w]
+//   K = [U_CC^-1 L_CC^-1 | -U_CC^-1 U_CB]     [w][w + r]
+// A solve is then, up the tree, b' = b_C + the children's contributions and
+// c = the children's contributions on B + F b' (the front's own contribution),
+// and, down the tree, x_C = K [b'; x_B]: one matrix product a front and
+// direction, and as many dependent steps as the tree of fronts is high (17 on
+// a 205K-cell plan, against 2,288 levels of rows).
+//
+// Rows of W and X are in front order (leaves first, then by height), a front's
+// columns contiguous from `off`. Operators are stored for
+// v_mfma_f64_16x16x4: [tile of 16 rows][step of 4 columns][lane], lane l
+// holding row l % 16, column l / 16 of the step; the w and the r columns of K
+// are padded to whole steps separately (zeros).
+constexpr int kEnvTile = 16;    // envs of a tile: the columns of one MFMA
+constexpr int kLeafCols = 64;   // columns of a leaf front
+constexpr int kFrontCols = 256; // columns of a front above the leaves
 
-struct Tail {
-    int lds;
-    int lev0, m, nlev, max_chunks;
-    const int* rows;
-    const double* diag;     // [m] U's diagonal (unused for L)
-    const int* hptr;
-    const int* hcol;
-    const double* hval;
-    const int* trow;
-    const int* tchunk;
-    const int* tmode;
-    const int* rchunk;
-    const int* cpos;        // [chunks * kChunk]
-    const double* cval;     // [chunks * kChunk]
+struct Front {
+    int off, w, r;
+    int brow;               // its B rows (positions in X) in FrontTab::brow, padded to a multiple of 4
+    int c;                  // its contribution's first row in C
+    int arow;               // its first row in FrontTab::arow (w rows, then r; fronts above the leaves)
+    long long f, k;         // its operators' offsets in FrontTab::ops
 };
 
-// How one factor's sweep runs in the default (non-exact) mode: the levels
-// before the LDS run, the LDS run, the levels after it; the levels before and
-// after run chunked from HBM when one level's partials fit in LDS, else as
-// plain row solves.
-struct Sweep {
-    int pre_end;            // levels [0, pre_end) before the LDS run
-    int post_begin;         // levels [post_begin, nlev) after it
-    int pre_chunked, post_chunked;
-    Tail pre, mid, post;    // (mid.nlev may be 0)
+// The unknowns are the temperatures less the env's ambient temperature (the
+// right-hand side less ambient x row sum): forcing and solutions of some 10 K
+// instead of 300 K keep the products' rounding a digit below the field's own,
+// whatever the order of their sums.
+
+// The contributions added to one row of a front above the leaves: rows of C,
+// four at once (the zero row where there are fewer), then brow-style extras
+// [xb, xe) of FrontTab::xsrc.
+struct AsmRow {
+    int s[4];
+    int xb, xe, pad[2];
+};
+
+// One row tile of a front (16 rows from 16 * tile).
+struct FrontTask {
+    int front, tile;
+};
+
+// One height of the tree: its fronts' tasks up (F's row tiles, at least one a
+// front above the leaves) and down (K's), and the widest front's columns.
+struct FrontLevel {
+    int f0, nf, k0, nk;     // tasks [f0, f0 + nf) up and [k0, k0 + nk) down
+    int wmax;
+};
+
+struct FrontTab {
+    int n_fronts, n_levels, n_leaf, n_c;   // n_leaf: rows of the leaves; n_c: rows of C (row n_c is zero)
+    const Front* fronts;
+    const int* brow;
+    const AsmRow* arow;
+    const int* xsrc;
+    const FrontTask* tasks;
+    const double* ops;
+    const int* rf;          // [n] solved index t -> row of W (its right-hand side)
+    const int* rx;          // [n] solved index t -> row of X (its solution)
+    const int* sn_w;        // sensed entries -> row of X
+    const double* rowsum;   // [n] by t: the factored system's row sums (L U 1) less capacitance and mass coupling
+    const FrontLevel* levels;   // host memory (the launches read it), leaves first
 };
 
 struct Tables {
@@ -88,8 +114,8 @@ struct Tables {
     const double *cap, *dir, *mcoup, *mret, *mgain;   // [n] by t
     const double *a0, *a1, *hz, *vt, *cd;             // [n] by t: exterior face areas, half widths, conductivity
     Tri L, U;
-    int fast;               // chunked runs (reassociated sums) instead of every level in order
-    Sweep SL, SU;
+    int fast;               // dense fronts (reassociated sums) instead of every level in order
+    FrontTab ft;
     // sensed rows (k): entries p in [sn_p[i], sn_p[i + 1]) weigh row sn_w[p] of the solution
     const int* sn_p;
     const int* sn_w;
@@ -114,10 +140,16 @@ struct Tables {
 
 struct Group {
     int G, Gl, nblk;
+    int nt;                 // env tiles of the default mode's vectors
     double* T;              // [nblk][n_cvs][Gl]
     double* M;              // [nblk][n][Gl]
-    double* W1;             // [nblk][n][Gl] the forcing solve
-    double* W2;             // [nblk][n][Gl] the air-side correction (exact mode; null with Tables::R)
+    // exact mode: the forcing solve in place, [nblk][n][Gl]; default mode: the
+    // right-hand side in front order, [nt][n][kEnvTile]
+    double* W1;
+    double* W2;             // [nblk][n][Gl] the air-side correction (exact mode)
+    double* X;              // [nt][n][kEnvTile] the solution less the ambient temperature (default mode)
+    double* Y;              // [nt][n - n_leaf][kEnvTile] assembled right-hand sides above the leaves (default mode)
+    double* C;              // [nt][n_c + 1][kEnvTile] the fronts' contributions, then a zero row (default mode)
     double* pw;             // [G][k] air-side power, then the dense solve's result
     double* mat;            // [G][k][k] I + diag(g) S
     int* eact;              // [G] env has a nonzero air-side conductance this step
@@ -138,9 +170,9 @@ struct StepIn {
 
 // The host (g++) and the device (hipcc) compile these structs separately and
 // exchange them byte for byte: both builds check the same sizes and offsets.
-static_assert(sizeof(Tri) == 56 && sizeof(Tail) == 112 && sizeof(Sweep) == 352, "Tri / Tail / Sweep layout");
-static_assert(sizeof(Tables) == 1040 && offsetof(Tables, S) == 1008 && offsetof(Tables, R) == 1016
-              && offsetof(Tables, nz) == 1032, "Tables layout");
-static_assert(sizeof(Group) == 80 && sizeof(StepIn) == 48, "Group / StepIn layout");
+static_assert(sizeof(Tri) == 56 && sizeof(Front) == 40 && sizeof(AsmRow) == 32 && sizeof(FrontTab) == 104,
+              "Tri / Front / FrontTab layout");
+static_assert(sizeof(Tables) == 440 && offsetof(Tables, S) == 408 && offsetof(Tables, nz) == 432, "Tables layout");
+static_assert(sizeof(Group) == 104 && sizeof(StepIn) == 48, "Group / StepIn layout");
 
 }  // namespace sbf

@@ -1,0 +1,563 @@
+// The default mode's building-scale field step: dense fronts on the matrix
+// cores (sbf::FrontTab), envs in tiles of kEnvTile = 16, the columns of a
+// v_mfma_f64_16x16x4.
+//
+// Per step: forcing into W (sb_fdm.c:147-151), the solve up and down the tree
+// of fronts (sb_lu.c:38-63 in another order: results agree to rounding), the
+// sensed temperatures and air-side powers (sb_fdm.c:157-162), the dense solve
+// (fdm_kernel.hip), then the correction R^T q, the interior mass and the field
+// (sb_fdm.c:171-187). The field and the mass keep the group's own layout.
+//
+// MFMA operands: A lane l holds row l % 16, column l / 16 of the step (the
+// operators are stored that way, one 512-byte load a step and wavefront), B
+// lane l holds row l / 16 of the step, env l % 16 (a row of 16 envs is one
+// 128-byte line, so rows may be gathered), D register q holds row
+// l / 16 + 4 q, env l % 16.
+// What bounds it: the vectors' HBM traffic at 256 envs and more, the chain of
+// 2 x 17 dependent launches at a tile or two. Measured on the 205K-cell plan:
+// a step of 256 envs 13.1 -> 2.3 ms, of 16 envs 10.2 -> 0.8 ms against level
+// by level row solves, whose 4,577 dependent levels were the whole time.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "fdm.h"
+
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int E = sbf::kEnvTile;
+static_assert(E == 16, "one MFMA column per env of a tile");
+
+__device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// acc[r][e] += A (row tile r) B (env tile e) over the steps [k0, k1): A from
+// the operator's tiles, B through load(step, e). U steps' loads are issued
+// before their products.
+template <int RT, int NE, int U, class Load>
+__device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE]) {
+    int k = k0;
+    for (; k + U <= k1; k += U) {
+        double a[RT][U], b[NE][U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int e = 0; e < NE; e++) b[e][u] = load(k + u, e);
+#pragma unroll
+            for (int r = 0; r < RT; r++) a[r][u] = A[r][(size_t)(k + u) * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int e = 0; e < NE; e++) acc[r][e] = mfma(a[r][u], b[e][u], acc[r][e]);
+    }
+    for (; k < k1; k++) {
+        double a[RT], b[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) b[e] = load(k, e);
+#pragma unroll
+        for (int r = 0; r < RT; r++) a[r] = A[r][(size_t)k * 64];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int e = 0; e < NE; e++) acc[r][e] = mfma(a[r], b[e], acc[r][e]);
+    }
+}
+
+// The leaves, a wavefront per (RT row tiles of a front, NE env tiles): up
+// (DOWN false) c = F b, down x = K [b; x_B]. Env tiles of one task are
+// neighbouring wavefronts, so a workgroup's wavefronts share the operator.
+template <bool DOWN, int RT, int NE>
+__global__ __launch_bounds__(256) void leaf_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+                                                   const double* __restrict__ W, double* __restrict__ C,
+                                                   double* __restrict__ X) {
+    const int neg = (nt + NE - 1) / NE;
+    const unsigned x = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int eg = (int)(x % (unsigned)neg), task = (int)(x / (unsigned)neg) * RT;
+    if (task >= ntask) return;
+    const int lane = threadIdx.x & 63, j = lane & 15, kk = lane >> 4;
+    // RT consecutive tasks; those of another front are its own wavefront's
+    // work too (a front's tiles need not start at a multiple of RT)
+    for (int u = 0; u < RT;) {
+        if (task + u >= ntask) break;
+        const sbf::FrontTask tk = t.tasks[task0 + task + u];
+        const sbf::Front f = t.fronts[tk.front];
+        int m = 1;
+        while (u + m < RT && task + u + m < ntask && t.tasks[task0 + task + u + m].front == tk.front) m++;
+        const int kw = (f.w + 3) >> 2, ks = DOWN ? kw + ((f.r + 3) >> 2) : kw;
+        const double* A[RT];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+            A[r] = t.ops + (DOWN ? f.k : f.f) + (size_t)(tk.tile + (r < m ? r : 0)) * ks * 64 + lane;
+        const double* Wb[NE];
+        const double* Xb[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const size_t te = min(eg * NE + e, nt - 1);
+            Wb[e] = W + (te * n + f.off) * E + j;
+            Xb[e] = X + te * n * E + j;
+        }
+        d4 acc[RT][NE] = {};
+        product<RT, NE, 4>(A, 0, kw, [&](int k, int e) { return Wb[e][min(4 * k + kk, f.w - 1) * E]; }, acc);
+        if (DOWN) {
+            const int* br = t.brow + f.brow + kk - 4 * kw;
+            product<RT, NE, 4>(A, kw, ks, [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc);
+        }
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            if (r >= m) continue;
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const size_t te = eg * NE + e;
+                if ((int)te >= nt) continue;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int row = (tk.tile + r) * 16 + kk + 4 * q;
+                    if (row >= (DOWN ? f.w : f.r)) continue;
+                    if (DOWN) X[(te * n + f.off + row) * E + j] = acc[r][e][q];
+                    else C[(te * (t.n_c + 1) + f.c + row) * E + j] = acc[r][e][q];
+                }
+            }
+        }
+        u += m;
+    }
+}
+
+// The sum of the contributions to one row (FrontTab::arow) of one env.
+__device__ __forceinline__ double gathered(const sbf::FrontTab& t, int row, const double* Cb) {
+    const int4 s = *reinterpret_cast<const int4*>(t.arow[row].s);
+    const int2 xr = *reinterpret_cast<const int2*>(&t.arow[row].xb);
+    double v = (Cb[(size_t)s.x * E] + Cb[(size_t)s.y * E]) + (Cb[(size_t)s.z * E] + Cb[(size_t)s.w * E]);
+    for (int q = xr.x; q < xr.y; q++) v += Cb[(size_t)t.xsrc[q] * E];
+    return v;
+}
+
+// A height above the leaves, one workgroup per (RT row tiles of a front, NE
+// env tiles), its 4 wavefronts taking a quarter of the columns each, summed
+// in LDS in wavefront order. Up: the front's b' assembled into LDS by every
+// workgroup of the front (its first tile's writes it to Y), then c = the
+// children's contributions on B + F b'. Down: x = K [b'; x_B].
+template <bool DOWN, int RT, int NE>
+__global__ __launch_bounds__(256) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+                                                    const double* __restrict__ W, double* __restrict__ Y,
+                                                    double* C, double* X) {
+    extern __shared__ double lds[];
+    const int neg = (nt + NE - 1) / NE;
+    const int eg = (int)(blockIdx.x % (unsigned)neg), task = (int)(blockIdx.x / (unsigned)neg) * RT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, kk = lane >> 4;
+    const int ny = n - t.n_leaf;
+    for (int u = 0; u < RT;) {
+        if (task + u >= ntask) break;
+        const sbf::FrontTask tk = t.tasks[task0 + task + u];
+        const sbf::Front f = t.fronts[tk.front];
+        int m = 1;
+        while (u + m < RT && task + u + m < ntask && t.tasks[task0 + task + u + m].front == tk.front) m++;
+        const int kw = (f.w + 3) >> 2, ks = DOWN ? kw + ((f.r + 3) >> 2) : kw;
+        const double* A[RT];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+            A[r] = t.ops + (DOWN ? f.k : f.f) + (size_t)(tk.tile + (r < m ? r : 0)) * ks * 64 + lane;
+        d4 acc[RT][NE] = {};
+        const int rows = DOWN ? f.w : f.r;
+        if (DOWN) {
+            const double* Yb[NE];
+            const double* Xb[NE];
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const size_t te = min(eg * NE + e, nt - 1);
+                Yb[e] = Y + (te * ny + (f.off - t.n_leaf)) * E + j;
+                Xb[e] = X + te * n * E + j;
+            }
+            // the quarters cut where the columns are
+            const int q0 = ks * wave / 4, q1 = ks * (wave + 1) / 4;
+            product<RT, NE, 4>(A, min(q0, kw), min(q1, kw),
+                               [&](int k, int e) { return Yb[e][min(4 * k + kk, f.w - 1) * E]; }, acc);
+            const int* br = t.brow + f.brow + kk - 4 * kw;
+            product<RT, NE, 4>(A, max(q0, kw), max(q1, kw),
+                               [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc);
+        } else {
+            // b' [4 kw][NE][E], zero past w
+            for (int q = tid; q < 4 * kw * NE * E; q += 256) {
+                const int row = q / (NE * E), e = (q / E) % NE;
+                const size_t te = min(eg * NE + e, nt - 1);
+                double v = 0.0;
+                if (row < f.w) {
+                    v = W[(te * n + f.off + row) * E + q % E]
+                        + gathered(t, f.arow + row, C + te * (t.n_c + 1) * E + q % E);
+                    if (tk.tile == 0 && eg * NE + e < nt) Y[(te * ny + (f.off - t.n_leaf) + row) * E + q % E] = v;
+                }
+                lds[q] = v;
+            }
+            __syncthreads();
+            product<RT, NE, 4>(A, kw * wave / 4, rows > 0 ? kw * (wave + 1) / 4 : kw * wave / 4,
+                               [&](int k, int e) { return lds[((4 * k + kk) * NE + e) * E + j]; }, acc);
+            __syncthreads();
+        }
+        // [wavefront][row tile][env tile][register][lane]
+        double* red = lds;
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int e = 0; e < NE; e++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) red[(((wave * RT + r) * NE + e) * 4 + q) * 64 + lane] = acc[r][e][q];
+        __syncthreads();
+        // wavefront q' finishes register q' of every tile
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int row = (tk.tile + r) * 16 + kk + 4 * wave;
+            if (r >= m || row >= rows) continue;
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const size_t te = eg * NE + e;
+                if ((int)te >= nt) continue;
+                double v = 0.0;
+#pragma unroll
+                for (int w = 0; w < 4; w++) v += red[(((w * RT + r) * NE + e) * 4 + wave) * 64 + lane];
+                if (DOWN) {
+                    X[(te * n + f.off + row) * E + j] = v;
+                } else {
+                    double* Cb = C + te * (t.n_c + 1) * E + j;
+                    Cb[(size_t)(f.c + row) * E] = v + gathered(t, f.arow + f.w + row, Cb);
+                }
+            }
+        }
+        u += m;
+        if (u < RT) __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------ the operators, at open
+
+// Dense blocks of front f at dense + d0[f]: L_CC [w][w], U_CC [w][w], L_BC
+// [r][w], U_CB [w][r].
+struct OpsTab {
+    const int* front_of;
+    const int* local;
+    const int* bperm;
+    const long long* d0;
+    double* dense;
+    double* sol;            // per front at s0[f]: [w][w + r + r]: the columns of K, then those of F^T
+    const long long* s0;
+};
+
+__device__ int b_index(const sbf::Front& f, const int* bperm, int i) {
+    int lo = 0, hi = f.r - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (bperm[f.brow + mid] < i) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// One thread per scheduled row of a factor: its terms into the dense blocks.
+template <bool UPPER>
+__global__ void ops_scatter_kernel(sbf::Tri tri, int nrows, const sbf::Front* fronts, OpsTab o) {
+    const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (q >= nrows) return;
+    const int i = tri.rows[q], fi = o.front_of[i];
+    if (UPPER) {
+        const sbf::Front f = fronts[fi];
+        double* D = o.dense + o.d0[fi];
+        const int li = o.local[i];
+        D[(size_t)f.w * f.w + (size_t)li * f.w + li] = tri.diag[q];
+        for (int e = tri.ptr[q]; e < tri.ptr[q + 1]; e++) {
+            const int c = tri.col[e];
+            if (o.front_of[c] == fi) D[(size_t)f.w * f.w + (size_t)li * f.w + o.local[c]] = tri.val[e];
+            else D[2 * (size_t)f.w * f.w + (size_t)f.w * f.r + (size_t)li * f.r + b_index(f, o.bperm, c)] = tri.val[e];
+        }
+    } else {
+        for (int e = tri.ptr[q]; e < tri.ptr[q + 1]; e++) {
+            const int c = tri.col[e], fc = o.front_of[c], lc = o.local[c];
+            const sbf::Front f = fronts[fc];
+            double* D = o.dense + o.d0[fc];
+            if (fc == fi) D[(size_t)o.local[i] * f.w + lc] = tri.val[e];
+            else D[2 * (size_t)f.w * f.w + (size_t)b_index(f, o.bperm, i) * f.w + lc] = tri.val[e];
+        }
+    }
+}
+
+// One thread per column of a front's operators: column c < w of K solves
+// L U x = e_c, the next r solve U x = -U_CB, the last r (rows of F) z L = -L_BC.
+__global__ __launch_bounds__(64) void ops_solve_kernel(const sbf::Front* fronts, int n_fronts, OpsTab o) {
+    for (int fi = blockIdx.x; fi < n_fronts; fi += gridDim.x) {
+        const sbf::Front f = fronts[fi];
+        const int w = f.w, r = f.r, ld = w + 2 * r;
+        const double* L = o.dense + o.d0[fi];
+        const double* U = L + (size_t)w * w;
+        const double* LB = U + (size_t)w * w;
+        const double* UB = LB + (size_t)w * r;
+        double* S = o.sol + o.s0[fi];
+        for (int c = blockIdx.y * 64 + threadIdx.x; c < ld; c += gridDim.y * 64) {
+            double* x = S + c;   // x[m * ld]
+            if (c >= w + r) {
+                const int b = c - w - r;
+                for (int m = w - 1; m >= 0; m--) {
+                    double acc = -LB[(size_t)b * w + m];
+                    for (int q = m + 1; q < w; q++) acc = fma(-L[(size_t)q * w + m], x[(size_t)q * ld], acc);
+                    x[(size_t)m * ld] = acc;
+                }
+                continue;
+            }
+            if (c < w) {
+                for (int m = 0; m < c; m++) x[(size_t)m * ld] = 0.0;
+                x[(size_t)c * ld] = 1.0;
+                for (int m = c + 1; m < w; m++) {
+                    double acc = 0.0;
+                    for (int q = c; q < m; q++) acc = fma(-L[(size_t)m * w + q], x[(size_t)q * ld], acc);
+                    x[(size_t)m * ld] = acc;
+                }
+            } else {
+                for (int m = 0; m < w; m++) x[(size_t)m * ld] = -UB[(size_t)m * r + (c - w)];
+            }
+            for (int m = w - 1; m >= 0; m--) {
+                double acc = x[(size_t)m * ld];
+                for (int q = m + 1; q < w; q++) acc = fma(-U[(size_t)m * w + q], x[(size_t)q * ld], acc);
+                x[(size_t)m * ld] = acc / U[(size_t)m * w + m];
+            }
+        }
+    }
+}
+
+// The solutions into the operators' tiles (rows and columns past the front's are zero).
+__global__ void ops_pack_kernel(const sbf::Front* fronts, int n_fronts, OpsTab o, double* ops) {
+    for (int fi = blockIdx.x; fi < n_fronts; fi += gridDim.x) {
+        const sbf::Front f = fronts[fi];
+        const int w = f.w, r = f.r, ld = w + 2 * r, kw = (w + 3) / 4, ks = kw + (r + 3) / 4;
+        const double* S = o.sol + o.s0[fi];
+        const size_t nF = (size_t)((r + 15) / 16) * kw * 64, nK = (size_t)((w + 15) / 16) * ks * 64;
+        for (size_t x = threadIdx.x; x < nF + nK; x += blockDim.x) {
+            const bool up = x < nF;
+            const size_t y = up ? x : x - nF;
+            const int lane = (int)(y & 63), step = (int)((y >> 6) % (size_t)(up ? kw : ks));
+            const int row = (int)((y >> 6) / (size_t)(up ? kw : ks)) * 16 + (lane & 15);
+            int col = 4 * step + (lane >> 4);
+            double v = 0.0;
+            if (up) {
+                if (row < r && col < w) v = S[(size_t)col * ld + w + r + row];
+            } else if (row < w) {
+                if (step < kw) v = col < w ? S[(size_t)row * ld + col] : 0.0;
+                else if ((col -= 4 * kw) < r) v = S[(size_t)row * ld + w + col];
+            }
+            ops[(up ? f.f : f.k) + y] = v;
+        }
+    }
+}
+
+// ------------------------------------------------------------ the rest of the step
+
+// What the env's solution is taken relative to (FrontTab).
+__device__ __forceinline__ double base_of(double ambient) { return isfinite(ambient) ? ambient : 0.0; }
+
+// Forcing (sb_fdm.c:147-151, exposure :126-140) less base x row sum: a workgroup takes 64 solved
+// cells of one env tile, computes with lanes over cells (the field, the heat
+// and the mass are read in the cells' order) and stores rows of 16 envs
+// through LDS. Lanes past the group's envs get zeros. Clears the blocks'
+// air-side flags.
+__global__ __launch_bounds__(256) void front_forcing_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
+    __shared__ double fs[64][E + 1];
+    const int te = (int)(blockIdx.x % (unsigned)g.nt), t0 = (int)(blockIdx.x / (unsigned)g.nt) * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = t.n, Gl = g.Gl;
+    const int tt = min(t0 + lane, n - 1);
+    const int p = t.solved[tt];
+    const double a0 = t.a0[tt], a1 = t.a1[tt], hz = t.hz[tt], vt = t.vt[tt], cd = t.cd[tt];
+    const double cap = t.cap[tt], dir = t.dir[tt], mcoup = t.mcoup[tt], rs = t.ft.rowsum[tt];
+    const int z = in.q ? -1 : t.czone[tt];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int l = wave * 4 + q, env = te * E + l;
+        double v = 0.0;
+        if (env < g.G) {
+            const size_t b = env / Gl, gl = env % Gl;
+            const double h = in.h[env];
+            double e = 0.0;
+            if (a0 > 0.0) e += h * a0 / (1.0 + h * 0.5 * hz / cd);
+            if (a1 > 0.0) e += h * a1 / (1.0 + h * 0.5 * vt / cd);
+            double heat;
+            if (in.q) heat = in.q[(size_t)env * t.n_cvs + p];
+            else heat = z >= 0 ? in.qz[(size_t)env * t.nz + z] : 0.0;
+            const double amb = in.amb[env], base = base_of(amb);
+            v = fma(cap, g.T[(b * t.n_cvs + p) * Gl + gl] - base, heat);
+            if (mcoup != 0.0) v = fma(mcoup, g.M[(b * n + tt) * Gl + gl] - base, v);
+            v += fma(amb, dir + e, -base * rs);
+        }
+        fs[lane][l] = v;
+    }
+    __syncthreads();
+    double* Wt = g.W1 + (size_t)te * n * E;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int c = q * 16 + (threadIdx.x >> 4);
+        if (t0 + c < n) Wt[(size_t)t.ft.rf[t0 + c] * E + (threadIdx.x & 15)] = fs[c][threadIdx.x & 15];
+    }
+    const size_t x = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (x < (size_t)g.nblk) g.bact[x] = 0;
+}
+
+// Per sensed row and env tile: the sensed temperature of the solution and the
+// air-side power g (T_air - sensed) (sb_fdm.c:157-162), 32 entries at a time
+// by 32 x 16 threads, summed in a fixed order.
+constexpr int kSensedThreads = 512;
+__global__ __launch_bounds__(kSensedThreads) void front_sensed_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
+    constexpr int R = kSensedThreads / E;
+    __shared__ double part[R][E];
+    const int te = (int)(blockIdx.x % (unsigned)g.nt), i = (int)(blockIdx.x / (unsigned)g.nt);
+    const int j = threadIdx.x % E, s = threadIdx.x / E;
+    const double* Xb = g.X + (size_t)te * t.n * E + j;
+    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
+    double acc = 0.0;
+#pragma unroll 8
+    for (int p = t.sn_p[i] + s; p < t.sn_p[i + 1]; p += R) acc += t.sn_x[p] * (base + Xb[(size_t)t.ft.sn_w[p] * E]);
+    part[s][j] = acc;
+    __syncthreads();
+    for (int h = R / 2; h > 0; h >>= 1) {
+        if (s < h) part[s][j] += part[s + h][j];
+        __syncthreads();
+    }
+    const int env = te * E + j;
+    if (s == 0 && env < g.G) {
+        const size_t x = (size_t)env * t.k + i;
+        g.pw[x] = in.g[x] * (in.airT[x] - part[0][j]);
+    }
+}
+
+// y = the forcing solve + R^T q where the air side is on (R's rows the
+// solutions of the applied columns, q the dense solve's result: the same y as
+// the second solve of sb_fdm.c:171-178 up to rounding), then the interior
+// mass and the field (sb_fdm.c:183-187). A workgroup takes 64 solved cells of
+// one env tile: 16 cells a wavefront as one MFMA tile over the k columns,
+// then through LDS to lanes over cells.
+__global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
+    __shared__ double ys[E][64 + 1];
+    const int te = (int)(blockIdx.x % (unsigned)g.nt), t0 = (int)(blockIdx.x / (unsigned)g.nt) * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, kk = lane >> 4;
+    const int n = t.n, k = t.k, Gl = g.Gl;
+    const double* Xb = g.X + (size_t)te * n * E + j;
+    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
+    double y[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) y[q] = Xb[(size_t)t.ft.rx[min(t0 + wave * 16 + kk + 4 * q, n - 1)] * E];
+    if (t.R) {
+        const int env = min(te * E + j, g.G - 1);
+        const double* qv = g.pw + (size_t)env * k;
+        const double* Rb = t.R + min(t0 + wave * 16 + j, n - 1);   // A: row (cell) lane % 16
+        d4 acc = {};
+#pragma unroll 5
+        for (int c = 0; c < k; c += 4) {
+            const int col = c + kk;
+            const double a = col < k ? Rb[(size_t)min(col, k - 1) * n] : 0.0;
+            acc = mfma(a, qv[min(col, k - 1)], acc);
+        }
+        const bool on = g.eact[env] != 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) y[q] = on ? y[q] + acc[q] : y[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) ys[j][wave * 16 + kk + 4 * q] = base + y[q];
+    __syncthreads();
+    const int tt = t0 + lane;
+    if (tt < n) {
+        const int cell = t.solved[tt];
+        const double mr = t.mret[tt], mg = t.mgain[tt];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int l = wave * 4 + q, env = te * E + l;
+            if (env >= g.G) break;
+            const size_t b = env / Gl, gl = env % Gl, mi = (b * n + tt) * Gl + gl;
+            const double v = ys[l][lane];
+            g.M[mi] = g.M[mi] * mr + mg * v;
+            g.T[(b * t.n_cvs + cell) * Gl + gl] = v;
+        }
+    }
+    const size_t tu = (size_t)g.nblk * t.n_unsolved * Gl;
+    for (size_t x = (size_t)blockIdx.x * 256 + threadIdx.x; x < tu; x += (size_t)gridDim.x * 256) {
+        const size_t bu = x / Gl;
+        const int u = (int)(bu % t.n_unsolved);
+        const size_t b = bu / t.n_unsolved;
+        const int env = (int)(b * Gl + x % Gl);
+        if (env < g.G) g.T[(b * t.n_cvs + t.unsolved[u]) * Gl + x % Gl] = in.amb[env];
+    }
+}
+
+size_t front_lds(bool down, int rt, int ne, int wmax) {
+    const size_t red = (size_t)4 * rt * ne * 256, b = down ? 0 : (size_t)((wmax + 3) / 4 * 4) * ne * E;
+    return sizeof(double) * std::max(red, b);
+}
+
+// Workgroups below which a height runs on single row and env tiles: with 2 x 2
+// tiles a workgroup reads half as much per product, but a height of fewer
+// than two workgroups a CU leaves matrix cores idle.
+constexpr unsigned kWideGroups = 512;
+
+template <bool DOWN>
+void launch_level(const sbf::Tables& t, const sbf::Group& g, int h, hipStream_t s) {
+    const sbf::FrontLevel& L = t.ft.levels[h];
+    const int t0 = DOWN ? L.k0 : L.f0, m = DOWN ? L.nk : L.nf;
+    if (m == 0) return;
+    const unsigned nt = (unsigned)g.nt;
+    if (h == 0) {
+        if (nt > 1) {
+            const unsigned waves = (unsigned)((m + 1) / 2) * ((nt + 1) / 2);
+            hipLaunchKernelGGL((leaf_kernel<DOWN, 2, 2>), dim3((waves + 3) / 4), dim3(256), 0, s, t.ft, t0, m, t.n,
+                               g.nt, g.W1, g.C, g.X);
+        } else {
+            const unsigned waves = (unsigned)((m + 1) / 2);
+            hipLaunchKernelGGL((leaf_kernel<DOWN, 2, 1>), dim3((waves + 3) / 4), dim3(256), 0, s, t.ft, t0, m, t.n,
+                               g.nt, g.W1, g.C, g.X);
+        }
+        return;
+    }
+    const unsigned wide = (unsigned)((m + 1) / 2) * ((nt + 1) / 2);
+    if (nt > 1 && wide >= kWideGroups)
+        hipLaunchKernelGGL((front_kernel<DOWN, 2, 2>), dim3(wide), dim3(256), front_lds(DOWN, 2, 2, L.wmax), s, t.ft,
+                           t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
+    else
+        hipLaunchKernelGGL((front_kernel<DOWN, 1, 1>), dim3((unsigned)m * nt), dim3(256),
+                           front_lds(DOWN, 1, 1, L.wmax), s, t.ft, t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
+}
+
+}  // namespace
+
+extern "C" int sbf_launch_dense(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s);
+
+// One batched step of a group in the default mode.
+extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in,
+                                     hipStream_t s) {
+    const unsigned tiles = (unsigned)((t->n + 63) / 64) * (unsigned)g->nt;
+    hipLaunchKernelGGL(front_forcing_kernel, dim3(tiles), dim3(256), 0, s, *t, *g, *in);
+    for (int h = 0; h < t->ft.n_levels; h++) launch_level<false>(*t, *g, h, s);
+    for (int h = t->ft.n_levels; h-- > 0;) launch_level<true>(*t, *g, h, s);
+    if (t->k > 0) {
+        hipLaunchKernelGGL(front_sensed_kernel, dim3((unsigned)t->k * (unsigned)g->nt), dim3(kSensedThreads), 0, s,
+                           *t, *g, *in);
+        if (int e = sbf_launch_dense(t, g, in, s)) return e;
+    }
+    hipLaunchKernelGGL(front_update_kernel, dim3(tiles), dim3(256), 0, s, *t, *g, *in);
+    return (int)hipGetLastError();
+}
+
+// The fronts' operators from the factors (rows scheduled in L and U: nl, nu),
+// on the null stream; front_of, local, bperm: FrontPlan's, on the device;
+// d0, s0: per front the offsets of its dense blocks and solutions.
+extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, const int* front_of, const int* local,
+                                    const int* bperm, const long long* d0, const long long* s0, double* dense,
+                                    double* sol, double* ops) {
+    const OpsTab o{front_of, local, bperm, d0, dense, sol, s0};
+    const sbf::Front* fr = t->ft.fronts;
+    const int nf = t->ft.n_fronts;
+    if (nl > 0)
+        hipLaunchKernelGGL((ops_scatter_kernel<false>), dim3((nl + 255) / 256), dim3(256), 0, nullptr, t->L, nl, fr, o);
+    hipLaunchKernelGGL((ops_scatter_kernel<true>), dim3((nu + 255) / 256), dim3(256), 0, nullptr, t->U, nu, fr, o);
+    hipLaunchKernelGGL(ops_solve_kernel, dim3(nf, 4), dim3(64), 0, nullptr, fr, nf, o);
+    hipLaunchKernelGGL(ops_pack_kernel, dim3(nf), dim3(256), 0, nullptr, fr, nf, o, ops);
+    return (int)hipGetLastError();
+}

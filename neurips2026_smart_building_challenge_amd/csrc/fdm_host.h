@@ -15,6 +15,7 @@ struct SbxFdm {
     unsigned char* d_tables = nullptr;
     double* d_temp_init = nullptr;
     double* d_mass_init = nullptr;
+    std::vector<sbf::FrontLevel> front_levels;   // (tab.ft.levels points here)
     std::vector<void*> owned;     // device buffers of the group
 };
 
