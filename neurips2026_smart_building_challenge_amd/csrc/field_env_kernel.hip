@@ -30,9 +30,14 @@ constexpr double kPaPerBar = 100000.0;
 constexpr double kPi = 3.14159265358979323846;
 enum { MODE_OFF = 0, MODE_HEAT = 1, MODE_COOL = 2, MODE_PASSIVE = 3 };
 
-__device__ __forceinline__ int lane() { return (int)threadIdx.x; }
-// one-wavefront workgroups: orders the wavefront's LDS accesses across lanes
-__device__ __forceinline__ void wsync() { __syncthreads(); }
+__device__ __forceinline__ int lane() { return (int)threadIdx.x & (W - 1); }
+// orders a wavefront's memory accesses across its lanes (no workgroup barrier:
+// the convection plan's wavefronts run apart)
+__device__ __forceinline__ void wsync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
 
 __device__ __forceinline__ unsigned long long ballot(bool p) { return __ballot(p); }
 __device__ __forceinline__ int first_lane(unsigned long long m) { return __ffsll((long long)m) - 1; }
@@ -929,39 +934,42 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 // from the top) and swapped in order. None of this reads a temperature, so the
 // plan runs before the field step and leaves a list of moves.
 //
+// One workgroup per env. Its first wavefront walks the stream, which is one
+// serial chain over the rooms: the cells' swaps and candidates, then the
+// shuffle's draws. The others (appliers) each take every conv_appliers-th
+// room once its draws are posted: the candidates' cells, the shuffle and its
+// composition, the moves. What bounds it is the first wavefront's chain of
+// scalar instructions, one swap after another. At 256 envs of the 205K-cell
+// building (about 13,500 swaps a step): 10.4 ms with everything on one
+// wavefront, 4.1 ms with the shuffle's draws resolved 64 words at a time, the
+// rooms applied beside the stream and a swap loop of one straight line.
+//
 // Stream: raw blocks in LDS, two at a time (the current one and, once a read
-// reaches past it, the next), each with its tempered copy. A round reads the u
-// of up to 64 cells at the positions they have if no cell before them swaps,
-// and with it the word each would start its candidate draw with; the first
-// cell that swaps ends the round. Fisher-Yates draws take 64 words at a time
-// and resolve one draw per ballot. Each final pair t (known once the shuffle
-// has passed t, from the top) is composed into the room's inverse
-// permutation q (q <- q o (a b)), so after the room T_new[q[i]] = T_old[i]
-// for every cell i of the room: the moves are the cells with q[i] != i.
+// reaches past it, the next), each with its tempered copy, positions relative
+// to the current block.
 namespace {
 
 struct Stream {
     uint32_t* raw;     // [2][624]
     uint32_t* tw;      // [2][624] tempered
-    long long base;    // stream position of the current block's word 0
-    long long pos;     // next word to consume
-    int cur;
+    int pos;           // next word to consume, from the current block's word 0
+    int cur;           // which of the two is the current block
     bool have_next;
 
-    __device__ uint32_t word(long long q) const {
-        const int d = (int)(q - base);
-        const int b = d >= SBE_MT_N ? cur ^ 1 : cur;
-        return tw[b * SBE_MT_N + (d >= SBE_MT_N ? d - SBE_MT_N : d)];
+    // word q (from the current block's word 0)
+    __device__ uint32_t word(int q) const {
+        const int x = q + (cur ? SBE_MT_N : 0);
+        return tw[x >= 2 * SBE_MT_N ? x - 2 * SBE_MT_N : x];
     }
-    // words up to position q (q - pos < 624) readable
-    __device__ void ensure(long long q) {
-        while (q >= base + SBE_MT_N * (have_next ? 2 : 1)) {
+    // words up to pos + ahead (< 624) readable
+    __device__ void ensure(int ahead) {
+        while (pos + ahead >= SBE_MT_N * (have_next ? 2 : 1)) {
             if (!have_next) {
                 const int nb = cur ^ 1;
                 mt_next_block(raw + cur * SBE_MT_N, raw + nb * SBE_MT_N, tw + nb * SBE_MT_N);
                 have_next = true;
             } else {
-                base += SBE_MT_N;
+                pos -= SBE_MT_N;
                 cur ^= 1;
                 have_next = false;
             }
@@ -969,265 +977,313 @@ struct Stream {
     }
 };
 
-__device__ __forceinline__ uint32_t smear(uint32_t x) {
-    x |= x >> 1;
-    x |= x >> 2;
-    x |= x >> 4;
-    x |= x >> 8;
-    x |= x >> 16;
-    return x;
+__device__ __forceinline__ uint32_t smear(uint32_t x) { return x ? 0xffffffffu >> __clz((int)x) : 0u; }
+
+// A room's pairs and shuffle draws, from the stream wavefront to its applier:
+// in LDS up to `cap` of them, the rest in HBM. pr[i]: cell | candidate << 16
+// (first the candidate's place among the cell's, then its cell).
+struct RoomSlot {
+    uint32_t* pr;
+    uint16_t* jd;
+    uint16_t* qinv;
+    unsigned int *spill, *jspill;
+    int cap;
+
+    __device__ uint32_t pair(int i) const { return i < cap ? pr[i] : spill[i - cap]; }
+    __device__ void set_pair(int i, uint32_t v) const {
+        if (i < cap) pr[i] = v;
+        else spill[i - cap] = v;
+    }
+    __device__ uint32_t draw(int i) const { return i < cap ? (uint32_t)jd[i] : jspill[i - cap]; }
+    __device__ void set_draw(int i, uint32_t v) const {
+        if (i < cap) jd[i] = (uint16_t)v;
+        else jspill[i - cap] = v;
+    }
+};
+
+// Posts between the wavefronts of a workgroup, and the wait for one: every
+// post a wavefront waits for is made by another that never waits for it.
+__device__ __forceinline__ void slot_post(int* flag, int v) {
+    __builtin_amdgcn_wave_barrier();
+    if (lane() == 0) __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ int slot_wait(int* flag, bool full) {
+    int v;
+    while (((v = __hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) >= 0) != full)
+        __builtin_amdgcn_s_sleep(2);
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+// The room's pairs from the stream; returns their count. Windows of 128
+// words: lane l holds the words at offsets 2l, 2l + 1, 2l + 2 of the window.
+// The walk is at word x; the drift (what the window's swapping cells have
+// taken beyond two words each) has x's parity, so the swap bits of the cells
+// that start at x's parity are one ballot (P0, P1), the next swapping cell is
+// its next set bit, and that cell's candidate draw reads the low bytes of the
+// following words (a cell has at most 255 candidates).
+__device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n, uint64_t thr, bool never) {
+    int m = 0;
+    for (int j = 0; j < n;) {
+        S.ensure(2 * W);
+        const int p = S.pos + 2 * lane();
+        const uint32_t w0 = S.word(p), w1 = S.word(p + 1), w2 = S.word(p + 2);
+        const int nc = (j + lane() < n) ? ncand[j + lane()] : 0;
+        const uint64_t u0 = ((uint64_t)(w0 >> 5) << 26) | (uint64_t)(w1 >> 6);
+        const uint64_t u1 = ((uint64_t)(w1 >> 5) << 26) | (uint64_t)(w2 >> 6);
+        const unsigned long long P0 = never ? 0ull : ballot(u0 <= thr), P1 = never ? 0ull : ballot(u1 <= thr);
+        const uint32_t low = (w0 & 0xffu) | (w1 & 0xffu) << 8 | (w2 & 0xffu) << 16;
+        // each cell's candidate draw: mask << 16 | largest value; negative
+        // where it draws nothing (-1: one candidate, -2: none)
+        const int rule = nc > 1 ? (int)(smear((uint32_t)nc - 1u) << 16) | (nc - 1) : nc == 1 ? -1 : -2;
+        // the window's pairs collect in one register (lane k: its k-th pair)
+        uint32_t wp = 0;
+        int npair = 0, x = 0, drift = 0, c = 0, ru = 0;
+        bool slow = false;   // cell c's candidate draw runs past the window, at word x
+        while (x < 2 * W) {
+            // swaps whose draw takes one or two words inside the window, one
+            // straight line of scalar instructions each
+            unsigned long long bits;
+            for (;;) {
+                bits = ((x & 1) ? P1 : P0) >> (x >> 1);
+                const int xs = x + 2 * first_lane(bits), xd = xs + 2;
+                c = (xs - drift) >> 1;
+                ru = (int)lane_u32((uint32_t)rule, c & 63);
+                const uint32_t t = lane_u32(low, (xd >> 1) & 63) >> (8 * (xd & 1));
+                const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
+                const uint32_t v1 = t & mask, v2 = (t >> 8) & mask;
+                const uint32_t v = v1 <= mx ? v1 : v2;
+                const int xn = xd + (v1 <= mx ? 1 : 2);
+                if (!((int)(bits != 0ull) & (int)(ru >= 0) & (int)(v <= mx) & (int)(xn < 2 * W))) break;
+                wp = lane() == npair ? (uint32_t)(j + c) | (v << 16) : wp;
+                npair++;
+                x = xn;
+                drift = x - 2 * (c + 1);
+            }
+            // any other swap
+            if (bits == 0ull) break;
+            x += 2 * first_lane(bits) + 2;
+            if (ru == -2) continue;
+            uint32_t v = 0;
+            if (ru >= 0) {
+                const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
+                do {
+                    slow = x >= 2 * W;
+                    if (slow) break;
+                    v = (lane_u32(low, x >> 1) >> (8 * (x & 1))) & mask;
+                    x++;
+                } while (v > mx);
+                if (slow) break;
+            }
+            wp = lane() == npair ? (uint32_t)(j + c) | (v << 16) : wp;
+            npair++;
+            drift = x - 2 * (c + 1);
+        }
+        if (m + W <= R.cap) {
+            if (lane() < npair) R.pr[m + lane()] = wp;
+        } else if (lane() < npair) {
+            R.set_pair(m + lane(), wp);
+        }
+        m += npair;
+        if (slow) {
+            S.pos += x;
+            j += c;
+            const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
+            uint32_t pick = 0;
+            for (;;) {
+                S.ensure(W - 1);
+                const uint32_t y = S.word(S.pos + lane()) & mask;
+                const unsigned long long okm = ballot(y <= mx);
+                if (okm) {
+                    const int gl = first_lane(okm);
+                    pick = lane_u32(y, gl);
+                    S.pos += gl + 1;
+                    break;
+                }
+                S.pos += W;
+            }
+            if (lane() == 0) R.set_pair(m, (uint32_t)j | (pick << 16));
+            m++;
+            j += 1;
+            continue;
+        }
+        // the cells up to the window's end, or to the room's: those past it draw nothing
+        const int ce = min((max(x, 2 * W + (x & 1)) - drift) >> 1, n - j);
+        S.pos += 2 * ce + drift;
+        j += ce;
+    }
+    return m;
+}
+
+// The shuffle's draws (draw t below t + 1, t = m - 1 .. 1, into R's draw t):
+// 64 words at a time. A word is accepted by the draw it meets, t less the
+// words accepted before it, so the accepted set is the fixed point of
+// "v <= t - (accepted lanes below)": lane 0 is right after one pass and each
+// pass settles at least one more lane (two or three passes settle a window).
+// A window ends where the draws' mask changes.
+__device__ void room_draws(Stream& S, const RoomSlot& R, int m) {
+    for (int tt = m - 1; tt > 0;) {
+        S.ensure(W - 1);
+        const int mask = (int)smear((uint32_t)tt), low = (mask >> 1) + 1;
+        const int v = (int)(S.word(S.pos + lane()) & (uint32_t)mask);
+        unsigned long long acc = ballot(v <= tt);
+        int mine = tt;
+        for (int pass = 0; pass <= W; pass++) {
+            mine = tt - below_me(acc);
+            const unsigned long long a2 = ballot(mine >= low && v <= mine);
+            if (a2 == acc) break;
+            acc = a2;
+        }
+        if ((acc >> lane()) & 1ull) R.set_draw(mine, (uint32_t)v);
+        const int cnt = __popcll(acc);
+        S.pos += cnt == tt - low + 1 ? 64 - __clzll((long long)acc) : W;
+        tt -= cnt;
+    }
+}
+
+// The room's shuffle from the top, each final pair composed into its inverse
+// permutation q (q <- q o (a b); a pair is final once the shuffle has passed
+// it), so that T_new[q[i]] = T_old[i] for every cell i of the room. Lane 0
+// applies the draws; the composition of one pair overlaps the loads of the
+// next, one LDS round trip a draw. LDS: the room's pairs all fit the slot.
+template <bool LDS>
+__device__ void room_shuffle(const RoomSlot& R, int m) {
+    auto compose = [&](uint32_t y) {
+        const int ca = (int)(y & 0xffffu), cb = (int)(y >> 16);
+        const uint16_t qa = R.qinv[ca], qb = R.qinv[cb];
+        R.qinv[ca] = qb;
+        R.qinv[cb] = qa;
+    };
+    for (int top = m - 1; top > 0; top -= W) {
+        const int mine = top - lane();
+        const uint32_t jl = mine > 0 ? (LDS ? (uint32_t)R.jd[mine] : R.draw(mine)) : 0u;
+        if (lane() == 0) {
+            const int cnt = min(W, top);
+            uint32_t held = 0;
+            bool have = false;
+            for (int l = 0; l < cnt; l++) {
+                const int t2 = top - l, j2 = (int)lane_u32(jl, l);
+                const uint32_t x = LDS ? R.pr[t2] : R.pair(t2), y = LDS ? R.pr[j2] : R.pair(j2);
+                if (have) compose(held);
+                if (LDS) R.pr[j2] = x;
+                else R.set_pair(j2, x);
+                held = y;
+                have = true;
+            }
+            if (have) compose(held);
+        }
+        wsync();
+    }
+    if (m > 0 && lane() == 0) compose(LDS ? R.pr[0] : R.pair(0));
+    wsync();
 }
 
 }  // namespace
 
-__global__ __launch_bounds__(W) void fe_conv_plan_kernel(Args a) {
+__global__ __launch_bounds__(W * (1 + kConvAppliers)) void fe_conv_plan_kernel(Args a) {
     const int s = (int)blockIdx.x;
     if (s >= a.G) return;
     const Tabs& t = a.t;
     extern __shared__ __align__(16) unsigned char lds[];
-    Stream S;
-    S.raw = reinterpret_cast<uint32_t*>(lds);
-    S.tw = S.raw + 2 * SBE_MT_N;
-    uint32_t* pr = S.tw + 2 * SBE_MT_N;                           // [cv_lds_pairs]
-    uint16_t* qinv = reinterpret_cast<uint16_t*>(pr + a.cv_lds_pairs);   // [cv_max_room]
-    uint8_t* ncand = reinterpret_cast<uint8_t*>(qinv + t.cv_max_room);    // [cv_max_room]
-    unsigned char* g = a.state + (size_t)s * a.st.record;
-    uint32_t* gmt = reinterpret_cast<uint32_t*>(g + a.st.cmt);
-    int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
-    unsigned int* spill = a.cv_spill + (size_t)s * 2 * t.cv_max_room;
-    const int cap = a.cv_lds_pairs;
-    // the room's Fisher-Yates draws: u16 in LDS beside the pairs, past the
-    // LDS pairs in the HBM overflow area's second half
-    uint16_t* jd = reinterpret_cast<uint16_t*>(lds + ((ncand + t.cv_max_room - lds + 3) & ~3));
-    unsigned int* jspill = spill + t.cv_max_room;
-    auto jd_st = [&](int i, uint32_t v) {
-        if (i < cap) jd[i] = (uint16_t)v;
-        else jspill[i - cap] = v;
+    __shared__ int flag[kConvAppliers], total;   // flag: the slot's pairs + 0, or -1 where it is free
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W)), na = (int)(blockDim.x / W) - 1;
+    const ConvLds L = conv_lds(t.cv_max_room, a.cv_lds_pairs);
+    auto slot = [&](int i) {
+        unsigned char* b = lds + L.base + (size_t)i * L.slot;
+        unsigned int* sp = a.cv_spill + ((size_t)s * na + i) * 2 * t.cv_max_room;
+        return RoomSlot{reinterpret_cast<uint32_t*>(b), reinterpret_cast<uint16_t*>(b + L.jd),
+                        reinterpret_cast<uint16_t*>(b + L.q), sp, sp + t.cv_max_room, a.cv_lds_pairs};
     };
-    auto jd_ld = [&](int i) -> uint32_t { return i < cap ? (uint32_t)jd[i] : jspill[i - cap]; };
-    auto pr_ld = [&](int i) -> uint32_t { return i < cap ? pr[i] : spill[i - cap]; };
-    auto pr_st = [&](int i, uint32_t v) {
-        if (i < cap) pr[i] = v;
-        else spill[i - cap] = v;
-    };
-    for (int i = lane(); i < SBE_MT_N; i += W) {
-        const uint32_t w = gmt[i];
-        S.raw[i] = w;
-        S.tw[i] = mt_temper(w);
-    }
-    S.base = 0;
-    S.pos = *gidx;
-    S.cur = 0;
-    S.have_next = false;
-    wsync();
-    const uint64_t thr = ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo;
-    const bool never = t.cv_thr_hi == 0xFFFFFFFFu;
-    unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
-    int count = 0;
-    for (int rm = 0; rm < t.cv_rooms; rm++) {
-        const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
-        // the room's candidate counts, eight loads in flight per lane
-        for (int i0 = 0; i0 < n; i0 += 8 * W) {
-            uint8_t c8[8];
+    if (threadIdx.x < kConvAppliers) flag[threadIdx.x] = -1;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    if (wave == 0) {
+        Stream S;
+        S.raw = reinterpret_cast<uint32_t*>(lds);
+        S.tw = S.raw + 2 * SBE_MT_N;
+        uint8_t* nbuf = reinterpret_cast<uint8_t*>(S.tw + 2 * SBE_MT_N);   // [cv_max_room + 32]
+        unsigned char* g = a.state + (size_t)s * a.st.record;
+        uint32_t* gmt = reinterpret_cast<uint32_t*>(g + a.st.cmt);
+        int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
+        for (int i = lane(); i < SBE_MT_N; i += W) {
+            const uint32_t w = gmt[i];
+            S.raw[i] = w;
+            S.tw[i] = mt_temper(w);
+        }
+        S.pos = __builtin_amdgcn_readfirstlane(*gidx);
+        S.cur = 0;
+        S.have_next = false;
+        wsync();
+        const uint64_t thr = ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo;
+        const bool never = t.cv_thr_hi == 0xFFFFFFFFu;
+        for (int rm = 0; rm < t.cv_rooms; rm++) {
+            const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
+            // the room's candidate counts, 16 cells a lane (the section is
+            // padded and 256-byte aligned, so whole 16-byte words are its own)
+            const int skew = b0 & 15;
+            const uint4* src = reinterpret_cast<const uint4*>(t.cv_ncand + (b0 - skew));
+            for (int i = lane(); 16 * i < n + skew; i += W) reinterpret_cast<uint4*>(nbuf)[i] = src[i];
+            wsync();
+            const RoomSlot R = slot(rm % na);
+            slot_wait(&flag[rm % na], false);
+            const int m = room_pairs(S, R, nbuf + skew, n, thr, never);
+            room_draws(S, R, m);
+            slot_post(&flag[rm % na], m);
+            wsync();
+        }
+        // the stream state: the block holding the last word consumed
+        const int blkx = S.pos > SBE_MT_N ? (S.cur ^ 1) : S.cur;
+        for (int i = lane(); i < SBE_MT_N; i += W) gmt[i] = S.raw[blkx * SBE_MT_N + i];
+        if (lane() == 0) *gidx = S.pos > SBE_MT_N ? S.pos - SBE_MT_N : S.pos;
+    } else {
+        const RoomSlot R = slot(wave - 1);
+        unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
+        for (int rm = wave - 1; rm < t.cv_rooms; rm += na) {
+            const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
+            for (int i = 2 * lane(); i < n; i += 2 * W)
+                reinterpret_cast<uint32_t*>(R.qinv)[i >> 1] = (uint32_t)i | ((uint32_t)(i + 1) << 16);
+            const int m = slot_wait(&flag[wave - 1], true);
+            // each pair's candidate as a room-local cell
+            for (int i = lane(); i < m; i += W) {
+                const uint32_t x = R.pair(i);
+                const int cell = (int)(x & 0xffffu), pick = (int)(x >> 16);
+                const uint32_t right = t.cv_cidx[t.cv_coff[b0 + cell] + pick];
+                R.set_pair(i, (uint32_t)cell | (right << 16));
+            }
+            wsync();
+            if (m <= R.cap) room_shuffle<true>(R, m);
+            else room_shuffle<false>(R, m);
+            slot_post(&flag[wave - 1], -1);
+            // moves: cell i's value goes to cell q[i] (convection-cell indices;
+            // the move kernels map them to field cells), in any order: each
+            // reads and writes cells of its own
+            for (int i0 = 0; i0 < n; i0 += 4 * W) {
+                int q[4];
+                unsigned long long mm[4];
+                int cnt = 0;
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int i = i0 + u * W + lane();
-                c8[u] = i < n ? t.cv_ncand[b0 + i] : 0;
-            }
+                for (int u = 0; u < 4; u++) {
+                    const int i = i0 + u * W + lane();
+                    q[u] = i < n ? (int)R.qinv[i] : i;
+                    mm[u] = ballot(q[u] != i);
+                    cnt += __popcll(mm[u]);
+                }
+                if (cnt == 0) continue;
+                int at = 0;
+                if (lane() == 0) at = atomicAdd(&total, cnt);
+                at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int i = i0 + u * W + lane();
-                if (i < n) {
-                    ncand[i] = c8[u];
-                    qinv[i] = (uint16_t)i;
-                }
-            }
-        }
-        wsync();
-        // cells, in windows of 128 stream words: lane i holds the words at
-        // offsets 2i, 2i + 1, 2i + 2 of the window, so for either parity of the
-        // drift (the words the window's swapping cells have taken beyond two
-        // per cell) the swap bit of cell i is one ballot (P0, P1), and a drift
-        // of 2t + par shifts those bits by t cells; each swap's candidate
-        // draw reads its words from the same registers
-        int m = 0;
-        for (int j = 0; j < n;) {
-            S.ensure(S.pos + 2 * W);
-            const long long p = S.pos + 2 * lane();
-            const uint32_t w0 = S.word(p), w1 = S.word(p + 1), w2 = S.word(p + 2);
-            const int nc = (j + lane() < n) ? ncand[j + lane()] : 0;
-            const uint64_t u0 = ((uint64_t)(w0 >> 5) << 26) | (uint64_t)(w1 >> 6);
-            const uint64_t u1 = ((uint64_t)(w1 >> 5) << 26) | (uint64_t)(w2 >> 6);
-            const unsigned long long P0 = ballot(!never && u0 <= thr), P1 = ballot(!never && u1 <= thr);
-            const unsigned long long HC = ballot(nc > 0);
-            // the window's pairs collect in one register (lane k: its k-th pair)
-            uint32_t wp = 0;
-            int npair = 0;
-            int c = 0, drift = 0;
-            bool slow = false;           // a candidate draw ran past the window
-            uint32_t smax = 0;
-            while (true) {
-                const int tt = drift >> 1, par = drift & 1;
-                if (c + tt >= W) break;
-                const unsigned long long cand = ((par ? P1 : P0) >> tt) & HC & (~0ull << c);
-                if (cand == 0ull) {
-                    c = W - tt;
-                    break;
-                }
-                const int cc = first_lane(cand);
-                const uint32_t mx = (uint32_t)__builtin_amdgcn_readlane(nc, cc) - 1u;
-                int q = 2 * (cc + tt) + par + 2;   // the candidate draw's first word
-                uint32_t pick = 0;
-                if (mx != 0u) {
-                    const uint32_t mask = smear(mx);
-                    for (;;) {
-                        if (q >= 2 * W) {
-                            slow = true;
-                            break;
-                        }
-                        const uint32_t wa = lane_u32(w0, q >> 1), wb = lane_u32(w1, q >> 1);
-                        const uint32_t v = ((q & 1) ? wb : wa) & mask;
-                        q++;
-                        if (v <= mx) {
-                            pick = v;
-                            break;
-                        }
-                    }
-                }
-                if (slow) {
-                    // the draw continues past the window: finish it from LDS
-                    S.pos += q;
-                    j += cc;
-                    smax = mx;
-                    break;
-                }
-                wp = lane() == npair ? ((uint32_t)(j + cc) | (pick << 16)) : wp;
-                npair++;
-                drift = q - 2 * (cc + 1);
-                c = cc + 1;
-            }
-            if (npair > 0) {
-                if (m + W <= cap) {
-                    if (lane() < npair) pr[m + lane()] = wp;
-                } else if (lane() < npair) {
-                    pr_st(m + lane(), wp);
-                }
-                m += npair;
-            }
-            if (slow) {
-                const uint32_t mask = smear(smax);
-                uint32_t pick = 0;
-                for (;;) {
-                    S.ensure(S.pos + W - 1);
-                    const uint32_t v = S.word(S.pos + lane()) & mask;
-                    const unsigned long long okm = ballot(v <= smax);
-                    if (okm) {
-                        const int gl = first_lane(okm);
-                        pick = lane_u32(v, gl);
-                        S.pos += gl + 1;
-                        break;
-                    }
-                    S.pos += W;
-                }
-                if (lane() == 0) pr_st(m, (uint32_t)j | (pick << 16));
-                m++;
-                j += 1;
-                continue;
-            }
-            const int ce = min(c, n - j);   // the window's cells past the room draw nothing
-            S.pos += 2 * ce + drift;
-            j += ce;
-        }
-        wsync();
-        // each pair's candidate as a room-local cell
-        for (int i = lane(); i < m; i += W) {
-            const uint32_t x = pr_ld(i);
-            const int cell = (int)(x & 0xffffu), pick = (int)(x >> 16);
-            const uint32_t right = t.cv_cidx[t.cv_coff[b0 + cell] + pick];
-            pr_st(i, (uint32_t)cell | (right << 16));
-        }
-        wsync();
-        // Fisher-Yates from the top: every draw resolved first (64 stream
-        // words per ballot pass; draw t into jd[t]), then lane 0 applies them,
-        // each final pair composed into q (q <- q o (a b)); the composition of
-        // one pair overlaps the loads of the next, one LDS round trip a draw
-        for (int tt = m - 1; tt > 0;) {
-            S.ensure(S.pos + W - 1);
-            const uint32_t w = S.word(S.pos + lane());
-            int kx = 0;
-            while (tt > 0 && kx < W) {
-                const uint32_t mask = smear((uint32_t)tt);
-                const unsigned long long okm = ballot((w & mask) <= (uint32_t)tt) & (~0ull << kx);
-                if (okm == 0ull) {
-                    kx = W;
-                    break;
-                }
-                const int gl = first_lane(okm);
-                if (lane() == 0) jd_st(tt, (lane_u32(w, gl) & mask));
-                kx = gl + 1;
-                tt--;
-            }
-            S.pos += kx;
-        }
-        wsync();
-        for (int top = m - 1; top > 0; top -= W) {
-            const int mine = top - lane();
-            const uint32_t jl = mine > 0 ? jd_ld(mine) : 0u;
-            if (lane() == 0) {
-                const int cnt = min(W, top);
-                uint32_t held = 0;
-                bool have = false;
-                for (int l = 0; l < cnt; l++) {
-                    const int t2 = top - l;
-                    const int j2 = (int)lane_u32(jl, l);
-                    const uint32_t x = pr_ld(t2), y = pr_ld(j2);
-                    if (have) {
-                        const int ca = (int)(held & 0xffffu), cb = (int)(held >> 16);
-                        const uint16_t qa = qinv[ca], qb = qinv[cb];
-                        qinv[ca] = qb;
-                        qinv[cb] = qa;
-                    }
-                    pr_st(j2, x);
-                    held = y;
-                    have = true;
-                }
-                if (have) {
-                    const int ca = (int)(held & 0xffffu), cb = (int)(held >> 16);
-                    const uint16_t qa = qinv[ca], qb = qinv[cb];
-                    qinv[ca] = qb;
-                    qinv[cb] = qa;
+                for (int u = 0; u < 4; u++) {
+                    const int i = i0 + u * W + lane();
+                    if (q[u] != i)
+                        moves[at + below_me(mm[u])] = ((unsigned long long)(unsigned)(b0 + q[u]) << 32) | (unsigned)(b0 + i);
+                    at += __popcll(mm[u]);
                 }
             }
             wsync();
         }
-        if (m > 0 && lane() == 0) {
-            const uint32_t y = pr_ld(0);
-            const int ca = (int)(y & 0xffffu), cb = (int)(y >> 16);
-            const uint16_t qa = qinv[ca], qb = qinv[cb];
-            qinv[ca] = qb;
-            qinv[cb] = qa;
-        }
-        wsync();
-        // moves: cell i's value goes to cell q[i] (convection-cell indices;
-        // the move kernels map them to field cells)
-        for (int i0 = 0; i0 < n; i0 += W) {
-            const int i = i0 + lane();
-            const int q = i < n ? (int)qinv[i] : i;
-            const bool mv = i < n && q != i;
-            const unsigned long long mm = ballot(mv);
-            if (mv) moves[count + below_me(mm)] = ((unsigned long long)(unsigned)(b0 + q) << 32) | (unsigned)(b0 + i);
-            count += __popcll(mm);
-        }
-        wsync();
     }
-    // the stream state: the block holding the last word consumed
-    const long long d = S.pos - S.base;
-    const int blkx = d > SBE_MT_N ? (S.cur ^ 1) : S.cur;
-    for (int i = lane(); i < SBE_MT_N; i += W) gmt[i] = S.raw[blkx * SBE_MT_N + i];
-    if (lane() == 0) {
-        *gidx = (int)(d > SBE_MT_N ? d - SBE_MT_N : d);
-        a.cv_count[s] = count;
-    }
+    __syncthreads();
+    if (threadIdx.x == 0) a.cv_count[s] = total;
 }
 
 // The moves of the step, read then written (two launches: every value is read
@@ -1304,8 +1360,9 @@ extern "C" int sbe_launch(const sbe::Args* a, int which, hipStream_t s) {
     case 2: hipLaunchKernelGGL(fe_post_kernel, dim3(G), dim3(64), a->lds_bytes, s, *a); break;
     case 3: hipLaunchKernelGGL(fe_live_kernel, dim3(1), dim3(64), 0, s, *a); break;
     case 4: {
-        const size_t lds = 4 * 4 * SBE_MT_N + 6 * (size_t)a->cv_lds_pairs + 3 * (size_t)a->t.cv_max_room + 16;
-        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64), lds, s, *a);
+        const ConvLds L = conv_lds(a->t.cv_max_room, a->cv_lds_pairs);
+        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64 * (1 + a->cv_appliers)),
+                           L.base + (size_t)a->cv_appliers * L.slot, s, *a);
         break;
     }
     case 5: {

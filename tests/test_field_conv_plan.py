@@ -168,3 +168,99 @@ def test_composed_moves_equal_shuffled_swaps():
         for (dst, _), v in zip(moves, vals):
             got[dst] = v
         assert np.array_equal(got, ref), trial
+
+
+def test_draws_by_fixed_point_equal_sequential_draws():
+    """The shuffle's draws 64 words at a time: the accepted words of a window
+    as the fixed point of "v <= t - (accepted lanes below)", a window ending
+    where the draws' mask changes, against one masked rejection after another."""
+    rng = np.random.default_rng(31)
+    for m in list(range(0, 70)) + [127, 128, 129, 255, 256, 257, 600, 1025, 5000]:
+        words = [int(x) for x in rng.integers(0, 2 ** 32, size=8 * m + 256, dtype=np.uint64)]
+        start = int(rng.integers(0, 50))
+        want, pos = {}, start
+        for t in range(m - 1, 0, -1):
+            want[t], pos = interval(words, pos, t)
+        got, gpos, tt = {}, start, m - 1
+        while tt > 0:
+            mask = smear(tt)
+            low = (mask >> 1) + 1
+            v = [words[gpos + i] & mask for i in range(W)]
+            acc = [v[i] <= tt for i in range(W)]
+            for passes in range(W + 1):
+                mine = [tt - sum(acc[:i]) for i in range(W)]
+                a2 = [mine[i] >= low and v[i] <= mine[i] for i in range(W)]
+                if a2 == acc:
+                    break
+                acc = a2
+            assert a2 == acc
+            for i in range(W):
+                if acc[i]:
+                    assert mine[i] not in got
+                    got[mine[i]] = v[i]
+            cnt = sum(acc)
+            gpos += max(i for i in range(W) if acc[i]) + 1 if cnt == tt - low + 1 else W
+            tt -= cnt
+        assert got == want and gpos == pos, m
+
+
+def walk_pairs(words: list, pos: int, ncand, thr: int):
+    """The plan kernel's walk over a window of 128 words: the next swapping
+    cell as the next swap bit of the walk's parity."""
+    n, pairs, j = len(ncand), [], 0
+    while j < n:
+        w = words[pos:pos + 2 * W + 1]
+        swap = [(((w[i] >> 5) << 26) | (w[i + 1] >> 6)) <= thr for i in range(2 * W)]
+        nc = [int(ncand[j + i]) if j + i < n else 0 for i in range(W)]
+        x = drift = c = 0
+        slow, found = False, []
+        while x < 2 * W:
+            nxt = [q for q in range(x, 2 * W, 2) if swap[q]]
+            if not nxt:
+                break
+            c = (nxt[0] - drift) >> 1
+            x = nxt[0] + 2
+            v = 0
+            if nc[c] == 0:
+                continue
+            if nc[c] > 1:
+                while True:
+                    slow = x >= 2 * W
+                    if slow:
+                        break
+                    v = (w[x] & 0xFF) & smear(nc[c] - 1)
+                    x += 1
+                    if v <= nc[c] - 1:
+                        break
+                if slow:
+                    break
+            found.append((j + c, v))
+            drift = x - 2 * (c + 1)
+        pairs += found
+        if slow:
+            pos += x
+            j += c
+            pick, pos = interval(words, pos, nc[c] - 1)
+            pairs.append((j, pick))
+            j += 1
+            continue
+        ce = min((max(x, 2 * W + (x & 1)) - drift) >> 1, n - j)
+        pos += 2 * ce + drift
+        j += ce
+    return pairs, pos
+
+
+def test_walk_equals_sequential_draws():
+    rng = np.random.default_rng(77)
+    for trial in range(300):
+        n = int(rng.integers(1, 500))
+        p = float(rng.choice([0.0, 0.05, 0.1, 0.3, 0.6, 0.95, 1.0]))
+        thr = (1 << 53) if p >= 1 else int(np.floor(p * 2.0 ** 53))
+        ncand = rng.integers(0, 25, size=n)
+        ncand[rng.random(n) < 0.1] = 0
+        ncand[rng.random(n) < 0.1] = 1
+        if trial % 3 == 0:
+            ncand[:] = rng.choice([1, 2, 24, 129, 255])
+        words = [int(x) for x in rng.integers(0, 2 ** 32, size=7 * n + 1000, dtype=np.uint64)]
+        start = int(rng.integers(0, 50))
+        assert walk_pairs(words, start, ncand, thr) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
