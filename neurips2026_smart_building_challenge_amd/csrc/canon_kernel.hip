@@ -19,9 +19,6 @@
 //                      comfort guard's trust (sb_gpu_base.inc:230-265), and the
 //                      canonical observation into the trainer's row
 //                      (sb_gpu_base.inc:287-369).
-// One 64-lane workgroup per env: zone slots across lanes, one lane per AHU,
-// the building-wide hot-water reset on lane 0, features across lanes; the
-// env's proposal and trust are kept in LDS until they are written out.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -50,6 +47,21 @@ __device__ __forceinline__ T np_mean(const T* a, int n) {
     return r / (T)n;
 }
 
+// The same by a wavefront, the 8 accumulators on lanes 0..7 (every lane of the
+// wavefront calls it); the mean on lane 0.
+template <class T>
+__device__ __forceinline__ T np_mean_wave(const T* a, int n, int lane) {
+#pragma clang fp contract(off)
+    if (n < 8) return np_mean(a, n);
+    const int j = lane & 7;
+    T q = a[j];
+    int i = 8;
+    for (; i < n - (n % 8); i += 8) q = q + a[i + j];
+    for (int o = 1; o < 8; o <<= 1) q = q + __shfl_xor(q, o);
+    for (; i < n; i++) q = q + a[i];
+    return q / (T)n;
+}
+
 // pidw_base.py _cyclic_feature_to_index: float32 arctan2 (rounded from
 // float64), + 2 pi when negative, floor(period * angle / (2 pi)) in float32
 __device__ __forceinline__ int cyclic(float s, float c, int period) {
@@ -62,66 +74,109 @@ __device__ __forceinline__ int cyclic(float s, float c, int period) {
 
 __device__ __forceinline__ double clipd(double x, double lo, double hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
-__device__ __forceinline__ float nat(const CanonTab& C, const float* o, int i) {
+// One workgroup of 4 wavefronts per env. What bounds it is the chain of its
+// phases' latencies, so everything it reads goes out in one burst (the
+// observation row and its native values to LDS, each thread's own indices to
+// registers): wavefronts 0 and 1 take a zone slot per lane (its command, its
+// trust, its 9 features), wavefront 2 an AHU per lane (PID, 16 features),
+// wavefront 3 the hot-water loop and the global features; the observation row
+// is put together in LDS and written in one piece. 42 us as one wavefront
+// that looked each feature's fields up in turn, 8 us so (300 envs of 81
+// zones on 9 AHUs).
+constexpr int kPostThreads = 256;
+__global__ __launch_bounds__(kPostThreads) void canon_post_kernel(CanonArgs A) {
 #pragma clang fp contract(off)
-    return i >= 0 ? o[i] * C.fstd[i] + C.fmean[i] : 0.0f;
-}
-
-__global__ __launch_bounds__(64) void canon_post_kernel(CanonArgs A) {
-#pragma clang fp contract(off)
-    const int e = blockIdx.x, lane = (int)threadIdx.x;
+    const int e = blockIdx.x, tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (e >= A.n) return;
     const CanonTab& C = A.tabs[A.envs[e].layout];
     const float* o = A.raw_obs + (size_t)e * SB_OBS;
-    __shared__ float sb[SB_ACT], sw[SB_ACT], sT[SBC_ZS], st[SBC_ZS], sai[2 * SBC_K], swk[SBC_K];
-    __shared__ double spid[2 * SBC_K], seff[SBC_K];
-    __shared__ int sact[SBC_K], sheat[SBC_K];
+    // so: the env's observation; sn: its native values, then a zero for absent fields
+    __shared__ float so[SB_OBS], sn[SB_OBS + 1], sr[SB_OBS];
+    __shared__ float sb[SB_ACT], sw[SB_ACT], sT[SBC_ZS], st[SBC_ZS], sai[2 * SBC_K], swk[SBC_K], s32[SBC_ZS];
+    __shared__ double spid[2 * SBC_K], seff[SBC_K], s64[SBC_ZS];
+    __shared__ int sact[SBC_K], sheat[SBC_K], scold;
     const bool fresh = A.reset || A.terminals[e] == 1.0f;   // a new episode starts here
-    for (int i = lane; i < 2 * SBC_K; i += 64) {
-        spid[i] = fresh ? 0.0 : A.pid[(size_t)e * 2 * SBC_K + i];
-        sai[i] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < SB_OBS / kPostThreads; q++) {
+        const int i = q * kPostThreads + tid;
+        const float x = o[i];
+        so[i] = x;
+        sn[i] = x * C.fstd[i] + C.fmean[i];
+        sr[i] = 0.0f;
     }
-    for (int i = lane; i < SB_ACT; i += 64) {
+    for (int i = tid; i < SB_ACT; i += kPostThreads) {
         sb[i] = 0.0f;
         sw[i] = 1.0f;
     }
+    if (tid < 2 * SBC_K) {
+        spid[tid] = fresh ? 0.0 : A.pid[(size_t)e * 2 * SBC_K + tid];
+        sai[tid] = 0.0f;
+    }
+    if (tid == 0) {
+        sn[SB_OBS] = 0.0f;
+        scold = 1;
+    }
+    const int s = tid < SBC_ZS ? tid : 0;   // wavefronts 0 and 1: this lane's zone slot
+    const int zT = tid < SBC_ZS ? C.zT[s] : -1, zAd = C.zAd[s], zAr = C.zAr[s];
+    const int zH = C.zH[s], zC = C.zC[s], zD = C.zD[s], zR = C.zR[s];
+    int zpos = s % SBC_ZPA, ns = 0;         // its place among the building's zones, and their number
+#pragma unroll
+    for (int k = 0; k < SBC_K; k++) {
+        const int z = k < C.K ? C.zc[k] : 0;
+        if (k < s / SBC_ZPA) zpos += z;
+        ns += z;
+    }
+    const int ka = lane < SBC_K ? lane : 0;   // wavefront 2: this lane's AHU
+    int aq[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) aq[m] = C.aObs[ka][m];
+    const int aT = C.aT[ka], aP = C.aP[ka], aRec = C.aRec[ka], aRun = C.aRun[ka], azc = C.zc[ka];
+    const int hW = C.hW, hDPa = C.hDPa, hRun = C.hRun;
+    // hour of the day on even lanes, day of the week on odd ones
+    const int g0 = max(C.g[(lane & 1) * 8], 0), g1 = max(C.g[(lane & 1) * 8 + 4], 0);
     __syncthreads();
-    const int hour = cyclic(o[C.g[0]], o[C.g[4]], 24);
-    const int day = cyclic(o[C.g[8]], o[C.g[12]], 7);
+    auto nat = [&](int i) { return sn[i >= 0 ? i : SB_OBS]; };
+    const int cyc = cyclic(so[g0], so[g1], (lane & 1) ? 7 : 24);
+    const int hour = __builtin_amdgcn_readlane(cyc, 0), day = __builtin_amdgcn_readlane(cyc, 1);
     const bool work = day < 5 && C.morning <= hour && hour < C.evening;
     const double lo = work ? C.comfort_lo : C.eco_lo, hi = work ? C.comfort_hi : C.eco_hi;
     const float lof = (float)lo, hif = (float)hi;
     // zone commands (PIDProportionalReheatPolicy._command_zones) and the
-    // guard's trust per zone, one zone slot per lane
-    for (int s = lane; s < SBC_ZS; s += 64) {
-        if (C.zT[s] < 0) continue;
-        const float T = o[C.zT[s]] * C.tstd + C.tmean;
+    // guard's trust per zone
+    if (zT >= 0) {
+        const float T = so[zT] * C.tstd + C.tmean;
         sT[s] = T;
         float err = 0.0f;
         if (T < lof) err = lof - T;
         else if (T > hif) err = hif - T;
         const float damper = fminf(1.0f, fabsf(err) / 2.0f);
-        if (C.zAd[s] >= 0) sb[C.zAd[s]] = 2.0f * damper - 1.0f;
+        if (zAd >= 0) sb[zAd] = 2.0f * damper - 1.0f;
         const float opening = fminf(1.0f, fmaxf(0.0f, err) / 2.0f);
-        if (C.zAr[s] >= 0) sb[C.zAr[s]] = 2.0f * opening - 1.0f;
+        if (zAr >= 0) sb[zAr] = 2.0f * opening - 1.0f;
         if (A.guard) {
             const float dev = T < lof ? lof - T : (A.hot && T > hif ? T - hif : 0.0f);
             const float t = fminf(1.0f, fmaxf(0.0f, 1.0f - (dev - A.d0) / A.d1));
             st[s] = t;
-            if (C.zAd[s] >= 0) sw[C.zAd[s]] = t;
-            if (C.zAr[s] >= 0) sw[C.zAr[s]] = t;
+            if (zAd >= 0) sw[zAd] = t;
+            if (zAr >= 0) sw[zAr] = t;
         }
+        // the zones' shortfalls in order, for the hot-water reset
+        const float d = lof - T;
+        s32[zpos] = d;
+        s64[zpos] = d > 0.0f ? (double)d : 0.0;
+        if (!(d > 0.0f)) scold = 0;
     }
     __syncthreads();
     // one lane per AHU: its PID loop on the mean zone temperature, fan
     // pressure, run command and economiser (PIDWorstZonePolicy.get_action with
     // PIDEconomizerPolicy's average-zone error and recirculation)
-    if (lane < C.K) {
-        const int k = lane, nz = C.zc[k];
+    if (wave == 2 && lane < C.K) {
+        const int k = lane, nz = azc;
         sact[k] = 0;
         sheat[k] = 0;
         seff[k] = 0.0;
-        if (C.aRec[k] >= 0) sb[C.aRec[k]] = 1.0f;
+        if (aRec >= 0) sb[aRec] = 1.0f;
         if (nz > 0) {
             const double avg = (double)np_mean<float>(sT + SBC_ZPA * k, nz);
             sai[2 * k + 1] = (float)avg;
@@ -132,9 +187,9 @@ __global__ __launch_bounds__(64) void canon_post_kernel(CanonArgs A) {
             if (error == 0.0) {
                 ps[0] = ps[0] * 0.5;
                 ps[1] = 0.0;
-                if (C.aT[k] >= 0) sb[C.aT[k]] = -1.0f;
-                if (C.aP[k] >= 0) sb[C.aP[k]] = -1.0f;
-                if (C.aRun[k] >= 0) sb[C.aRun[k]] = 0.0f;
+                if (aT >= 0) sb[aT] = -1.0f;
+                if (aP >= 0) sb[aP] = -1.0f;
+                if (aRun >= 0) sb[aRun] = 0.0f;
             } else {
                 ps[0] = clipd(ps[0] + error, -10.0, 10.0);
                 const double deriv = error - ps[1];
@@ -145,14 +200,13 @@ __global__ __launch_bounds__(64) void canon_post_kernel(CanonArgs A) {
                 sact[k] = 1;
                 sheat[k] = error > 0.0;
                 const double pressure = clipd(2.0 * fabs(u) - 1.0, -1.0, 1.0);
-                if (C.aT[k] >= 0) sb[C.aT[k]] = (float)u;
-                if (C.aP[k] >= 0) sb[C.aP[k]] = (float)pressure;
-                if (C.aRun[k] >= 0) sb[C.aRun[k]] = 1.0f;
-                if (C.aRec[k] >= 0) {
+                if (aT >= 0) sb[aT] = (float)u;
+                if (aP >= 0) sb[aP] = (float)pressure;
+                if (aRun >= 0) sb[aRun] = 1.0f;
+                if (aRec >= 0) {
                     double rec = 1.0;
-                    const int oat = C.aObs[k][0];
-                    if (!(u >= 0.0) && oat >= 0) {
-                        const double outside = (double)o[oat], inside = avg;
+                    if (!(u >= 0.0) && aq[0] >= 0) {
+                        const double outside = (double)so[aq[0]], inside = avg;
                         if (isfinite(outside) && !(outside >= inside)) {
                             double pa = (pressure + 1.0) * 0.5 * 2000.0;
                             pa = pa > 200.0 ? pa : 200.0;
@@ -166,160 +220,134 @@ __global__ __launch_bounds__(64) void canon_post_kernel(CanonArgs A) {
                             }
                         }
                     }
-                    sb[C.aRec[k]] = (float)rec;
+                    sb[aRec] = (float)rec;
                 }
             }
         }
         if (A.guard) {
             float wk = 1.0f;
             for (int j = 0; j < nz; j++) wk = fminf(wk, st[SBC_ZPA * k + j]);
-            if (C.aT[k] >= 0) sw[C.aT[k]] = wk;
-            if (C.aP[k] >= 0) sw[C.aP[k]] = wk;
-            if (C.aRec[k] >= 0) sw[C.aRec[k]] = wk;
-            if (C.aRun[k] >= 0) sw[C.aRun[k]] = wk;
+            if (aT >= 0) sw[aT] = wk;
+            if (aP >= 0) sw[aP] = wk;
+            if (aRec >= 0) sw[aRec] = wk;
+            if (aRun >= 0) sw[aRun] = wk;
             swk[k] = wk;
         }
     }
+    // zone features (residual_policy.py _features), beside the AHUs
+    if (zT >= 0) {
+        const float T = nat(zT), Hs = nat(zH), Cs = nat(zC);
+        float* r = sr + SBC_FZ * s;
+        r[0] = 1.0f;
+        r[1] = (T - 295.0f) / 5.0f;
+        r[2] = (T - Hs) / 2.0f;
+        r[3] = (Cs - T) / 2.0f;
+        r[4] = (Hs - 294.0f) / 3.0f;
+        r[5] = zD >= 0 ? 2.0f * nat(zD) - 1.0f : 0.0f;
+        r[6] = zR >= 0 ? 2.0f * nat(zR) - 1.0f : 0.0f;
+        r[7] = zAd >= 0 ? sb[zAd] : 0.0f;
+        r[8] = zAr >= 0 ? sb[zAr] : 0.0f;
+    }
     __syncthreads();
-    // the hot-water loop (PIDPolicy's water actions, then PIDWaterResetPolicy's
-    // reset: the greater of the mean zone shortfall over 4 K and the 0.25
-    // quantile of the AHUs' heating effort)
-    if (lane == 0) {
-        int any_heat = 0, any_act = 0;
-        for (int k = 0; k < C.K; k++) {
-            any_heat |= sheat[k];
-            any_act |= sact[k];
-        }
-        if (C.hW >= 0) sb[C.hW] = any_heat ? 1.0f : -1.0f;
-        if (C.hDPa >= 0) sb[C.hDPa] = any_act ? 1.0f : -1.0f;
-        if (C.hRun >= 0) sb[C.hRun] = any_act ? 1.0f : 0.0f;
-        if (C.hW >= 0 && sb[C.hW] > 0.0f) {
+    if (wave == 3) {
+        // the hot-water loop (PIDPolicy's water actions, then
+        // PIDWaterResetPolicy's reset: the greater of the mean zone shortfall
+        // over 4 K and the 0.25 quantile of the AHUs' heating effort)
+        const bool mine = lane < C.K;
+        const bool act = mine && sact[ka] != 0;
+        const unsigned long long acts = __ballot(act);
+        const bool any_act = acts != 0ull, any_heat = __ballot(mine && sheat[ka] != 0) != 0ull;
+        float water = any_heat ? 1.0f : -1.0f;
+        if (hW >= 0 && any_heat) {
             // a shortfall of 0 is a Python 0.0 in the reference's list, which
             // makes numpy's mean float64; with none the mean is float32
-            float s32[SBC_ZS];
-            double s64[SBC_ZS];
-            int ns = 0;
-            bool all_pos = true;
-            for (int k = 0; k < C.K; k++)
-                for (int j = 0; j < C.zc[k]; j++) {
-                    const float d = lof - sT[SBC_ZPA * k + j];
-                    s32[ns] = d;
-                    s64[ns] = d > 0.0f ? (double)d : 0.0;
-                    all_pos = all_pos && d > 0.0f;
-                    ns++;
-                }
             double shortfall = 0.0;
-            if (ns > 0) shortfall = all_pos ? (double)np_mean<float>(s32, ns) : np_mean<double>(s64, ns);
+            if (ns > 0) shortfall = scold ? (double)np_mean_wave<float>(s32, ns, lane) : np_mean_wave<double>(s64, ns, lane);
             const double demand = shortfall / 4.0;
             double sat = 0.0;
-            double h[SBC_K];
-            int ne = 0;
-            for (int k = 0; k < C.K; k++)
-                if (sact[k]) h[ne++] = seff[k] > 0.0 ? seff[k] : 0.0;
+            const int ne = __popcll(acts);
             if (ne > 0) {
-                for (int i = 1; i < ne; i++) {
-                    const double x = h[i];
-                    int j = i - 1;
-                    while (j >= 0 && h[j] > x) {
-                        h[j + 1] = h[j];
-                        j--;
-                    }
-                    h[j + 1] = x;
+                // numpy quantile, method linear: virtual index (n - 1) q, numpy's
+                // _lerp; the sorted efforts by their ranks
+                const double h = act && seff[ka] > 0.0 ? seff[ka] : 0.0;
+                int rank = 0;
+#pragma unroll
+                for (int k = 0; k < SBC_K; k++) {
+                    const double x = __shfl(h, k);
+                    if ((acts >> k) & 1ull) rank += x < h || (x == h && k < lane);
                 }
-                // numpy quantile, method linear: virtual index (n - 1) q, numpy's _lerp
                 const double vi = (double)(ne - 1) * 0.25;
                 int i0 = (int)floor(vi), i1 = i0 + 1;
                 if (vi >= (double)(ne - 1)) i0 = i1 = ne - 1;
+                const double h0 = __shfl(h, __ffsll((long long)__ballot(act && rank == i0)) - 1);
+                const double h1 = __shfl(h, __ffsll((long long)__ballot(act && rank == i1)) - 1);
                 const double t = vi - floor(vi);
-                const double diff = h[i1] - h[i0];
-                sat = t >= 0.5 ? h[i1] - diff * (1.0 - t) : h[i0] + diff * t;
+                const double diff = h1 - h0;
+                sat = t >= 0.5 ? h1 - diff * (1.0 - t) : h0 + diff * t;
             }
             const double m = demand > sat ? demand : sat;
-            sb[C.hW] = (float)(2.0 * clipd(m + 0.0, 0.0, 1.0) - 1.0);
+            water = (float)(2.0 * clipd(m + 0.0, 0.0, 1.0) - 1.0);
         }
-        if (A.guard) {
-            float wb = 1.0f;
-            for (int k = 0; k < C.K; k++) wb = fminf(wb, swk[k]);
-            if (C.hW >= 0) sw[C.hW] = wb;
-            if (C.hDPa >= 0) sw[C.hDPa] = wb;
-            if (C.hRun >= 0) sw[C.hRun] = wb;
+        if (lane == 0) {
+            if (hW >= 0) sb[hW] = water;
+            if (hDPa >= 0) sb[hDPa] = any_act ? 1.0f : -1.0f;
+            if (hRun >= 0) sb[hRun] = any_act ? 1.0f : 0.0f;
+            if (A.guard) {
+                float wb = 1.0f;
+                for (int k = 0; k < C.K; k++) wb = fminf(wb, swk[k]);
+                if (hW >= 0) sw[hW] = wb;
+                if (hDPa >= 0) sw[hDPa] = wb;
+                if (hRun >= 0) sw[hRun] = wb;
+            }
+            const int* q = C.hObs;
+            float* r = sr + SBC_OH;
+            r[0] = 1.0f;
+            r[1] = (nat(q[0]) - 330.0f) / 20.0f;
+            r[2] = (nat(q[1]) - 330.0f) / 20.0f;
+            r[3] = nat(q[2]) / 10.0f;
+            r[4] = nat(q[3]) / 10.0f;
+            r[5] = 2.0f * nat(q[4]) - 1.0f;
+            r[6] = nat(q[5]) / 10.0f;
+            r[7] = hW >= 0 ? sb[hW] : 0.0f;
+            r[8] = hDPa >= 0 ? sb[hDPa] : 0.0f;
+            r[9] = hRun >= 0 ? 2.0f * sb[hRun] - 1.0f : 0.0f;
         }
+        if (lane < SBC_FG) {
+            const int i = C.g[lane];
+            sr[SBC_OG + lane] = i >= 0 ? so[i] : 0.0f;
+        }
+    } else if (wave == 2 && lane < C.K) {
+        const int k = lane;
+        float* r = sr + SBC_OA + SBC_FA * k;
+        r[0] = 1.0f;
+        r[1] = (nat(aq[0]) - 283.0f) / 15.0f;
+        r[2] = nat(aq[1]) / 1000.0f;
+        r[3] = nat(aq[2]) / 10.0f;
+        r[4] = nat(aq[3]) / 10.0f;
+        r[5] = aq[4] >= 0 ? (nat(aq[4]) - 295.0f) / 5.0f : 0.0f;
+        r[6] = 2.0f * nat(aq[5]) - 1.0f;
+        r[7] = nat(aq[6]) / 10.0f;
+        r[8] = 2.0f * nat(aq[7]) - 1.0f;
+        r[9] = aT >= 0 ? sb[aT] : 0.0f;
+        r[10] = aP >= 0 ? sb[aP] : 0.0f;
+        r[11] = aRec >= 0 ? sb[aRec] : 0.0f;
+        r[12] = aRun >= 0 ? 2.0f * sb[aRun] - 1.0f : 0.0f;
+        r[13] = azc > 0 ? (sai[2 * k + 1] - 295.0f) / 5.0f : 0.0f;
+        r[14] = (float)(spid[2 * k] / 10.0);
+        r[15] = sai[2 * k];
     }
     __syncthreads();
-    for (int i = lane; i < SB_ACT; i += 64) {
+    for (int i = tid; i < SB_ACT; i += kPostThreads) {
         A.base[(size_t)e * SB_ACT + i] = sb[i];
         A.trust[(size_t)e * SB_ACT + i] = sw[i];
     }
-    for (int i = lane; i < 2 * SBC_K; i += 64) {
-        A.pid[(size_t)e * 2 * SBC_K + i] = spid[i];
-        A.ainfo[(size_t)e * 2 * SBC_K + i] = sai[i];
+    if (tid < 2 * SBC_K) {
+        A.pid[(size_t)e * 2 * SBC_K + tid] = spid[tid];
+        A.ainfo[(size_t)e * 2 * SBC_K + tid] = sai[tid];
     }
-    // the canonical observation (residual_policy.py _features)
+    // the padding past the canonical features is zeroed by a reset only
     float* out = A.obs + (size_t)e * SB_OBS;
-    for (int f = lane; f < SBC_OBS; f += 64) {
-        float v = 0.0f;
-        if (f < SBC_OA) {
-            const int s = f / SBC_FZ, c = f % SBC_FZ;
-            if (C.zT[s] >= 0) {
-                const float T = nat(C, o, C.zT[s]), Hs = nat(C, o, C.zH[s]), Cs = nat(C, o, C.zC[s]);
-                switch (c) {
-                case 0: v = 1.0f; break;
-                case 1: v = (T - 295.0f) / 5.0f; break;
-                case 2: v = (T - Hs) / 2.0f; break;
-                case 3: v = (Cs - T) / 2.0f; break;
-                case 4: v = (Hs - 294.0f) / 3.0f; break;
-                case 5: v = C.zD[s] >= 0 ? 2.0f * nat(C, o, C.zD[s]) - 1.0f : 0.0f; break;
-                case 6: v = C.zR[s] >= 0 ? 2.0f * nat(C, o, C.zR[s]) - 1.0f : 0.0f; break;
-                case 7: v = C.zAd[s] >= 0 ? sb[C.zAd[s]] : 0.0f; break;
-                default: v = C.zAr[s] >= 0 ? sb[C.zAr[s]] : 0.0f; break;
-                }
-            }
-        } else if (f < SBC_OH) {
-            const int k = (f - SBC_OA) / SBC_FA, c = (f - SBC_OA) % SBC_FA;
-            if (k < C.K) {
-                const int* q = C.aObs[k];
-                switch (c) {
-                case 0: v = 1.0f; break;
-                case 1: v = (nat(C, o, q[0]) - 283.0f) / 15.0f; break;
-                case 2: v = nat(C, o, q[1]) / 1000.0f; break;
-                case 3: v = nat(C, o, q[2]) / 10.0f; break;
-                case 4: v = nat(C, o, q[3]) / 10.0f; break;
-                case 5: v = q[4] >= 0 ? (nat(C, o, q[4]) - 295.0f) / 5.0f : 0.0f; break;
-                case 6: v = 2.0f * nat(C, o, q[5]) - 1.0f; break;
-                case 7: v = nat(C, o, q[6]) / 10.0f; break;
-                case 8: v = 2.0f * nat(C, o, q[7]) - 1.0f; break;
-                case 9: v = C.aT[k] >= 0 ? sb[C.aT[k]] : 0.0f; break;
-                case 10: v = C.aP[k] >= 0 ? sb[C.aP[k]] : 0.0f; break;
-                case 11: v = C.aRec[k] >= 0 ? sb[C.aRec[k]] : 0.0f; break;
-                case 12: v = C.aRun[k] >= 0 ? 2.0f * sb[C.aRun[k]] - 1.0f : 0.0f; break;
-                case 13: v = C.zc[k] > 0 ? (sai[2 * k + 1] - 295.0f) / 5.0f : 0.0f; break;
-                case 14: v = (float)(spid[2 * k] / 10.0); break;
-                default: v = sai[2 * k]; break;
-                }
-            }
-        } else if (f < SBC_OG) {
-            const int c = f - SBC_OH;
-            const int* q = C.hObs;
-            switch (c) {
-            case 0: v = 1.0f; break;
-            case 1: v = (nat(C, o, q[0]) - 330.0f) / 20.0f; break;
-            case 2: v = (nat(C, o, q[1]) - 330.0f) / 20.0f; break;
-            case 3: v = nat(C, o, q[2]) / 10.0f; break;
-            case 4: v = nat(C, o, q[3]) / 10.0f; break;
-            case 5: v = 2.0f * nat(C, o, q[4]) - 1.0f; break;
-            case 6: v = nat(C, o, q[5]) / 10.0f; break;
-            case 7: v = C.hW >= 0 ? sb[C.hW] : 0.0f; break;
-            case 8: v = C.hDPa >= 0 ? sb[C.hDPa] : 0.0f; break;
-            default: v = C.hRun >= 0 ? 2.0f * sb[C.hRun] - 1.0f : 0.0f; break;
-            }
-        } else {
-            const int i = C.g[f - SBC_OG];
-            v = i >= 0 ? o[i] : 0.0f;
-        }
-        out[f] = v;
-    }
-    if (A.reset)
-        for (int f = SBC_OBS + lane; f < SB_OBS; f += 64) out[f] = 0.0f;
+    for (int f = tid; f < (A.reset ? SB_OBS : SBC_OBS); f += kPostThreads) out[f] = sr[f];
 }
 
 __global__ __launch_bounds__(64) void canon_pre_kernel(CanonArgs A) {
@@ -357,7 +385,7 @@ __global__ __launch_bounds__(64) void canon_pre_kernel(CanonArgs A) {
 
 extern "C" int sbk_launch_canon(const sbk::CanonArgs* a, int post, hipStream_t s) {
     if (a->n <= 0) return (int)hipErrorInvalidValue;
-    if (post) hipLaunchKernelGGL(sbk::canon_post_kernel, dim3(a->n), dim3(64), 0, s, *a);
+    if (post) hipLaunchKernelGGL(sbk::canon_post_kernel, dim3(a->n), dim3(sbk::kPostThreads), 0, s, *a);
     else hipLaunchKernelGGL(sbk::canon_pre_kernel, dim3(a->n), dim3(64), 0, s, *a);
     return (int)hipGetLastError();
 }
