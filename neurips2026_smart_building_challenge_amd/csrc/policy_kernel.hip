@@ -229,31 +229,25 @@ __global__ __launch_bounds__(256) void heads_layer_kernel(const float* __restric
         const bool live = e < n;
         const int ec = live ? e : n - 1;
         const bool used = live && (h < SB_CONT ? h < n_cont[ec] : h - SB_CONT < n_disc[ec]);
-        float gm = 1.0f;
+        float gm = 1.0f, a = 1.0f;
         if (used) {
-            const float a = beta_shape(ys[row][16 * which + k], floor);
+            a = beta_shape(ys[row][16 * which + k], floor);
             gm = gamma_mt(a, (uint32_t)e, step, 2u * (uint32_t)h + (uint32_t)which, (uint32_t)seed,
                           (uint32_t)(seed >> 32));
         }
         const float other = __shfl_xor(gm, 1, 64);
-        if (live && which == 0) {
-            float v = 0.0f, x = 0.0f;
-            if (used) {
-                x = gm / (gm + other);
-                v = h < SB_CONT ? 2.0f * x - 1.0f : (x > 0.5f ? 1.0f : 0.0f);
-            }
-            actions[(size_t)e * kActWidth + h] = v;
-            if (draws) {
-                const size_t o = (size_t)e * kActWidth + h;
+        const float ga = which ? other : gm, gb = which ? gm : other;
+        const float x = used ? ga / (ga + gb) : 0.0f;
+        const size_t o = (size_t)e * kActWidth + h;
+        if (live && which == 0)
+            actions[o] = used ? (h < SB_CONT ? 2.0f * x - 1.0f : (x > 0.5f ? 1.0f : 0.0f)) : 0.0f;
+        if (draws) {
+            const PairTerms t = beta_pair(a, __shfl_xor(a, 1, 64), which, x);
+            if (live && which == 0) {
                 draws[o] = x;
-                float lp = 0.0f, en = 0.0f;
-                if (used) {
-                    const BetaHead bh = beta_head(ys[row][k], ys[row][16 + k], x, floor);
-                    lp = (float)bh.logp;
-                    en = (float)bh.entropy;
-                }
-                hlp[o] = lp;
-                hent[o] = en;
+                hlp[o] = used ? (float)t.logp : 0.0f;
+            } else if (live) {
+                hent[o] = used ? (float)t.entropy : 0.0f;
             }
         }
     }
@@ -325,12 +319,11 @@ __global__ void beta_sample_kernel(const float* alpha, const float* beta, float*
 }
 
 constexpr int kPpoThreads = (kActWidth + 63) / 64 * 64;   // one thread per head
-static_assert(kPpoThreads <= 512, "the PPO reduction sums 512 slots");
 
 // The PPO side of the Beta heads for one minibatch row per env
 // (complete_port/patches/pufferlib_core.diff:1205-1252 ppo loss and its
-// ratio_per_dim, :539-543, :1008-1014 beta_kl): one workgroup per env, thread h takes
-// head h. Over the env's used heads (D of them), in f64 and a fixed summation
+// ratio_per_dim, :539-543, :1008-1014 beta_kl): one workgroup per env, a thread per
+// used head. Over the env's used heads (D of them), in f64 and a fixed summation
 // order: logp = sum log p_new(x), H = sum entropies under the new heads,
 // KL = sum KL(old head || new head). Then
 //   r = exp(clamp(lr, -20, 20)), lr = (logp - logp_old) / (D if per_dim else 1)
@@ -346,41 +339,48 @@ __global__ __launch_bounds__(kPpoThreads) void ppo_beta_kernel(const float* __re
                                                        const int* __restrict__ n_cont, const int* __restrict__ n_disc,
                                                        int n, float floor, float clip, float ent_coef, int per_dim,
                                                        float* __restrict__ out, float* __restrict__ grad) {
-    __shared__ double red[3][512];
+    __shared__ double red[3][kPpoThreads / 64];
     __shared__ float dlp;
     const int e = blockIdx.x, t = (int)threadIdx.x;
     if (e >= n) return;
     const int nc = n_cont[e], nd = n_disc[e];
-    const int h = t;
-    const bool used = h < kActWidth && (h < SB_CONT ? h < nc : h - SB_CONT < nd);
+    // the used heads on consecutive threads, so that the wavefronts past them
+    // (most envs use 89 to 181 of the 272 heads) do nothing
+    const bool used = t < nc + nd;
+    const int h = t < nc ? t : SB_CONT + t - nc;
     double lp = 0.0, en = 0.0, kl = 0.0;
     double g[4] = {0.0, 0.0, 0.0, 0.0};
     if (used) {
         const float* yn = y_new + (size_t)e * kPolicyHeads;
         const float* yo = y_old + (size_t)e * kPolicyHeads;
         const int cu = head_col(h, 0), cv = head_col(h, 1);
-        const BetaHead bh = beta_head(yn[cu], yn[cv], draws[(size_t)e * kActWidth + h], floor);
+        const BetaAt at = beta_at(yn[cu], yn[cv], floor);
+        const BetaHead bh = beta_head(at, yn[cu], yn[cv], draws[(size_t)e * kActWidth + h]);
         lp = bh.logp;
         en = bh.entropy;
 #pragma unroll
         for (int k = 0; k < 4; k++) g[k] = bh.g[k];
-        kl = beta_kl(beta_shape(yo[cu], floor), beta_shape(yo[cv], floor), beta_shape(yn[cu], floor),
-                     beta_shape(yn[cv], floor));
+        kl = beta_kl(beta_at(yo[cu], yo[cv], floor), at);
     }
-    for (int i = t; i < 512; i += (int)blockDim.x) {
-        const bool mine = i == t;
-        red[0][i] = mine ? lp : 0.0;
-        red[1][i] = mine ? en : 0.0;
-        red[2][i] = mine ? kl : 0.0;
+    // over the wavefront's lanes, then the wavefronts in order
+    for (int o = 32; o > 0; o >>= 1) {
+        lp += __shfl_xor(lp, o);
+        en += __shfl_xor(en, o);
+        kl += __shfl_xor(kl, o);
+    }
+    if ((t & 63) == 0) {
+        red[0][t >> 6] = lp;
+        red[1][t >> 6] = en;
+        red[2][t >> 6] = kl;
     }
     __syncthreads();
-    for (int w = 256; w > 0; w >>= 1) {
-        for (int i = t; i < w; i += (int)blockDim.x)
-            for (int q = 0; q < 3; q++) red[q][i] += red[q][i + w];
-        __syncthreads();
-    }
     if (t == 0) {
-        const double lps = red[0][0], ens = red[1][0], kls = red[2][0];
+        double lps = 0.0, ens = 0.0, kls = 0.0;
+        for (int w = 0; w < kPpoThreads / 64; w++) {
+            lps += red[0][w];
+            ens += red[1][w];
+            kls += red[2][w];
+        }
         const int D = nc + nd;
         double lr = lps - (double)logp_old[e];
         if (per_dim) lr /= (double)(D > 0 ? D : 1);
@@ -403,10 +403,16 @@ __global__ __launch_bounds__(kPpoThreads) void ppo_beta_kernel(const float* __re
         dlp = (float)(gr * r);
     }
     __syncthreads();
-    if (grad && h < kActWidth) {
+    if (grad) {
+        float* gu = grad + (size_t)e * 2 * kActWidth;
+        float* gv = gu + kActWidth;
         const double d = (double)dlp;
-        grad[((size_t)e * 2 + 0) * kActWidth + h] = used ? (float)(d * g[0] - (double)ent_coef * g[2]) : 0.0f;
-        grad[((size_t)e * 2 + 1) * kActWidth + h] = used ? (float)(d * g[1] - (double)ent_coef * g[3]) : 0.0f;
+        if (used) {
+            gu[h] = (float)(d * g[0] - (double)ent_coef * g[2]);
+            gv[h] = (float)(d * g[1] - (double)ent_coef * g[3]);
+        }
+        for (int q = t; q < kActWidth; q += kPpoThreads)
+            if (q < SB_CONT ? q >= nc : q - SB_CONT >= nd) gu[q] = gv[q] = 0.0f;
     }
 }
 

@@ -324,3 +324,53 @@ def test_gpu_beta_eval_floor_below_one(mixed_dir):
     act = vec.actions.cpu().numpy()
     assert np.all(np.abs(act[:, :256]) <= 1.0) and set(np.unique(act[:, 256:])) <= {0.0, 1.0}
     vec.close()
+
+
+@pytest.mark.parametrize("floor", [1.0, 0.05])
+@pytest.mark.parametrize("half", [0, 1])
+def test_gpu_beta_eval_across_shifts(mixed_dir, floor, half):
+    """The heads' density, entropy and gradients where their gamma functions
+    change form: shapes and shape sums on both sides of 8 (shifted below, not
+    above), next to the floor and in the hundreds, against scipy in float64 at
+    the float32 shapes. Outputs are float32 of 64-bit values, so each lies
+    within float32 rounding of it (half an ulp, 2^-24), and a sum of them
+    within that of its terms."""
+    from scipy import special
+
+    vec = E.VecEnv(1, blob_dir=str(mixed_dir), groups=1, max_steps=40)
+    vec.policy_bind(E.policy_weights(5), beta_floor=floor)
+    nc, nd = vec.envs[0].n_cont, vec.envs[0].n_disc
+    sh = np.array([floor + 1e-3, floor + 0.3, 2.0, 3.999, 4.001, 6.5, 7.999, 8.0, 8.001, 9.5, 40.0, 700.0])
+    pick = np.random.default_rng(2).permutation(sh.size ** 2)[half * 72:half * 72 + min(nc, 72)]
+    m = pick.size
+    a, b = np.ones(nc) * 2.0, np.ones(nc) * 2.0
+    a[:m], b[:m] = sh[pick // sh.size], sh[pick % sh.size]
+    raw = lambda s: np.where(s - floor < 15, np.log(np.expm1(np.minimum(s - floor, 15.0))), s - floor)
+    y = np.zeros((1, 2 * E.SB_ACT), np.float32)
+    y[0, :nc], y[0, E.SB_CONT:E.SB_CONT + nc] = raw(a), raw(b)
+    x = np.full((1, E.SB_ACT), 0.3, np.float32)
+    lp, en, g = (t.cpu().numpy().astype(np.float64) for t in
+                 vec.beta_eval(torch.from_numpy(y).cuda(), torch.from_numpy(x).cuda()))
+    u = np.concatenate([y[0, :nc], np.zeros(nd, np.float32)])   # (a discrete head's raw outputs are 0 here)
+    v = np.concatenate([y[0, E.SB_CONT:E.SB_CONT + nc], np.zeros(nd, np.float32)])
+    A = (_softplus32(u) + np.float32(floor)).astype(np.float64)
+    B = (_softplus32(v) + np.float32(floor)).astype(np.float64)
+    # (the device's float32 softplus may round the other way: a shape's half ulp moves each value by its derivative)
+    S, X = A + B, float(np.float32(0.3))
+    psi, tri = special.digamma, lambda t: special.polygamma(1, t)
+    lnb = special.gammaln(A) + special.gammaln(B) - special.gammaln(S)
+    wlp = (A - 1) * np.log(X) + (B - 1) * np.log1p(-X) - lnb
+    wen = lnb - (A - 1) * psi(A) - (B - 1) * psi(B) + (S - 2) * psi(S)
+    ga, gb = np.log(X) - psi(A) + psi(S), np.log1p(-X) - psi(B) + psi(S)
+    ha, hb = -(A - 1) * tri(A) + (S - 2) * tri(S), -(B - 1) * tri(B) + (S - 2) * tri(S)
+    ulp = 2.0 ** -22
+    assert abs(lp[0] - wlp.sum()) <= ulp * (np.abs(wlp) + np.abs(ga) * A + np.abs(gb) * B).sum()
+    assert abs(en[0] - wen.sum()) <= ulp * (np.abs(wen) + np.abs(ha) * A + np.abs(hb) * B).sum()
+    su, sv = special.expit(u.astype(np.float64)), special.expit(v.astype(np.float64))
+    t2 = lambda t: np.abs(special.polygamma(2, t))
+    move = [tri(A) * A + tri(S) * S, tri(B) * B + tri(S) * S,
+            (tri(A) + (A - 1) * t2(A)) * A + (tri(S) + S * t2(S)) * S, (tri(B) + (B - 1) * t2(B)) * B + (tri(S) + S * t2(S)) * S]
+    for k, want in enumerate([ga * su, gb * sv, ha * su, hb * sv]):
+        got = g[0, k, np.r_[0:nc, E.SB_CONT:E.SB_CONT + nd]]
+        assert np.all(np.abs(got - want) <= ulp * (np.abs(want) + np.abs(move[k]))), k
+    vec.close()
