@@ -17,7 +17,8 @@
 #include "sbb_reader.h"
 #include "sbenv.h"
 
-extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, const int* front_of, const int* local,
+extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, int leaf_fronts, const int* front_of,
+                                    const int* local,
                                     const int* bperm, const long long* d0, const long long* s0, double* dense,
                                     double* sol, double* ops);
 extern "C" int sbf_launch_solve_cols(const sbf::Tables* t, const sbf::Group* g, const double* b, double* x,
@@ -450,13 +451,16 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     if (T.fast) {
         // the fronts' operators, formed on the device from the factors' rows
         double *dense = nullptr, *sol = nullptr, *ops = (double*)dalloc(f, 8 * fp.ops);
+        const int leaf_fronts = (int)(std::partition_point(fp.fronts.begin(), fp.fronts.end(),
+                                                           [&](const sbf::Front& q) { return q.off < fp.n_leaf; })
+                                      - fp.fronts.begin());
         bool ok = ops && hip_check(hipMalloc(&dense, 8 * dense_n), "hipMalloc(front blocks)")
                   && hip_check(hipMalloc(&sol, 8 * sol_n), "hipMalloc(front solutions)")
                   && hip_check(hipMemset(dense, 0, 8 * dense_n), "clear front blocks");
         T.ft.ops = ops;
         auto at = [&](size_t off) { return (const void*)(f->d_tables + off); };
         ok = ok
-             && hip_check((hipError_t)sbf_launch_front_ops(&T, (int)L.rows.size(), (int)U.rows.size(),
+             && hip_check((hipError_t)sbf_launch_front_ops(&T, (int)L.rows.size(), (int)U.rows.size(), leaf_fronts,
                                                            (const int*)at(o_front), (const int*)at(o_local),
                                                            (const int*)at(o_bperm), (const long long*)at(o_d0),
                                                            (const long long*)at(o_s0), dense, sol, ops),
@@ -588,8 +592,13 @@ int sbx_fdm_get_state(SbxFdm* f, double* temp, double* mass_temp) {
     if (!f || !temp || !mass_temp) return -1;
     const sbf::Group& g = f->grp;
     const sbf::Tables& t = f->tab;
-    std::vector<double> buf((size_t)g.nblk * g.Gl * std::max(t.n_cvs, t.n));
     if (!hip_check(hipDeviceSynchronize(), "sbx_fdm_get_state")) return -1;
+    if (g.Gl == 1)   // env-major already: straight into the caller's arrays
+        return hip_check(hipMemcpy(temp, g.T, 8 * (size_t)g.G * t.n_cvs, hipMemcpyDeviceToHost), "copy T")
+                       && hip_check(hipMemcpy(mass_temp, g.M, 8 * (size_t)g.G * t.n, hipMemcpyDeviceToHost), "copy M")
+                   ? 0
+                   : -1;
+    std::vector<double> buf((size_t)g.nblk * g.Gl * std::max(t.n_cvs, t.n));
     if (!hip_check(hipMemcpy(buf.data(), g.T, 8 * (size_t)g.nblk * g.Gl * t.n_cvs, hipMemcpyDeviceToHost), "copy T"))
         return -1;
     for (int e = 0; e < g.G; e++) {

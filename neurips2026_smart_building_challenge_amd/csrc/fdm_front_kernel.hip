@@ -15,7 +15,7 @@
 // l / 16 + 4 q, env l % 16.
 // What bounds it: the vectors' HBM traffic at 256 envs and more, the chain of
 // 2 x 17 dependent launches at a tile or two. Measured on the 205K-cell plan:
-// a step of 256 envs 13.1 -> 2.3 ms, of 16 envs 10.2 -> 0.8 ms against level
+// a step of 256 envs 13.1 -> 2.0 ms, of 16 envs 10.2 -> 0.45 ms against level
 // by level row solves, whose 4,577 dependent levels were the whole time.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -36,36 +36,28 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
 
 // acc[r][e] += A (row tile r) B (env tile e) over the steps [k0, k1): A from
 // the operator's tiles, B through load(step, e). U steps' loads are issued
-// before their products.
+// before their products; the last U may run past k1 with zeros for A (a step
+// at a time there would be a memory latency each).
 template <int RT, int NE, int U, class Load>
 __device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE]) {
-    int k = k0;
-    for (; k + U <= k1; k += U) {
+    for (int k = k0; k < k1; k += U) {
         double a[RT][U], b[NE][U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            const int q = min(k + u, k1 - 1);
 #pragma unroll
-            for (int e = 0; e < NE; e++) b[e][u] = load(k + u, e);
+            for (int e = 0; e < NE; e++) b[e][u] = load(q, e);
 #pragma unroll
-            for (int r = 0; r < RT; r++) a[r][u] = A[r][(size_t)(k + u) * 64];
+            for (int r = 0; r < RT; r++) a[r][u] = A[r][(size_t)q * 64];
         }
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int r = 0; r < RT; r++)
+            for (int r = 0; r < RT; r++) {
+                const double x = k + u < k1 ? a[r][u] : 0.0;
 #pragma unroll
-                for (int e = 0; e < NE; e++) acc[r][e] = mfma(a[r][u], b[e][u], acc[r][e]);
-    }
-    for (; k < k1; k++) {
-        double a[RT], b[NE];
-#pragma unroll
-        for (int e = 0; e < NE; e++) b[e] = load(k, e);
-#pragma unroll
-        for (int r = 0; r < RT; r++) a[r] = A[r][(size_t)k * 64];
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-            for (int e = 0; e < NE; e++) acc[r][e] = mfma(a[r], b[e], acc[r][e]);
+                for (int e = 0; e < NE; e++) acc[r][e] = mfma(x, b[e][u], acc[r][e]);
+            }
     }
 }
 
@@ -137,15 +129,43 @@ __device__ __forceinline__ double gathered(const sbf::FrontTab& t, int row, cons
     return v;
 }
 
+// b' of the wide heights' fronts (those above the leaves with many
+// workgroups), a thread per (row, env): the right-hand side and the children's
+// contributions into Y.
+__global__ __launch_bounds__(256) void assemble_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+                                                       const double* __restrict__ W, double* __restrict__ Y,
+                                                       const double* __restrict__ C) {
+    const int ny = n - t.n_leaf, j = threadIdx.x % E, r = threadIdx.x / E;
+    const int te = (int)(blockIdx.x % (unsigned)nt), task = (int)(blockIdx.x / (unsigned)nt);
+    if (task >= ntask) return;
+    const sbf::FrontTask tk = t.tasks[task0 + task];   // (K's tasks: 16 of the front's columns each)
+    const sbf::Front f = t.fronts[tk.front];
+    const int row = tk.tile * 16 + r;
+    if (row >= f.w) return;
+    const double* Cb = C + (size_t)te * (t.n_c + 1) * E + j;
+    Y[((size_t)te * ny + (f.off - t.n_leaf) + row) * E + j] = W[((size_t)te * n + f.off + row) * E + j]
+                                                               + gathered(t, f.arow + row, Cb);
+}
+
 // A height above the leaves, one workgroup per (RT row tiles of a front, NE
-// env tiles), its 4 wavefronts taking a quarter of the columns each, summed
-// in LDS in wavefront order. Up: the front's b' assembled into LDS by every
-// workgroup of the front (its first tile's writes it to Y), then c = the
-// children's contributions on B + F b'. Down: x = K [b'; x_B].
-template <bool DOWN, int RT, int NE>
-__global__ __launch_bounds__(256) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
-                                                    const double* __restrict__ W, double* __restrict__ Y,
-                                                    double* C, double* X) {
+// env tiles), its KW wavefronts taking an equal share of the columns each,
+// summed in LDS in wavefront order. Down: x = K [b'; x_B]. Up: c = the
+// children's contributions on B + F b', with b' from Y (assemble_kernel), or,
+// FUSED, assembled into LDS by every workgroup of the front (its first tile's
+// writes it to Y).
+//
+// A narrow height (one to a few fronts: the upper 13 of 16 on a 205K-cell
+// plan) is a chain of memory latencies, so it runs FUSED with 8 wavefronts
+// and everything that does not wait for b' loaded before it: 18 and 11 us a
+// height with 4 wavefronts and 4 steps in flight, 9 and 8 so (16 envs). A wide
+// height (the lowest three) assembled by every workgroup took 188 us at 256
+// envs, from Y 47: there it
+// is bound by the products' operand traffic: 2 x 2 tiles.
+template <bool DOWN, bool FUSED, int RT, int NE, int KW, int U>
+__global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+                                                        const double* __restrict__ W, double* __restrict__ Y,
+                                                        double* C, double* X) {
+    static_assert(!FUSED || (RT == 1 && NE == 1), "the fused form takes single tiles");
     extern __shared__ double lds[];
     const int neg = (nt + NE - 1) / NE;
     const int eg = (int)(blockIdx.x % (unsigned)neg), task = (int)(blockIdx.x / (unsigned)neg) * RT;
@@ -163,41 +183,83 @@ __global__ __launch_bounds__(256) void front_kernel(sbf::FrontTab t, int task0, 
 #pragma unroll
         for (int r = 0; r < RT; r++)
             A[r] = t.ops + (DOWN ? f.k : f.f) + (size_t)(tk.tile + (r < m ? r : 0)) * ks * 64 + lane;
+        const double* Yb[NE];
+        const double* Xb[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const size_t te = min(eg * NE + e, nt - 1);
+            Yb[e] = Y + (te * ny + (f.off - t.n_leaf)) * E + j;
+            Xb[e] = X + te * n * E + j;
+        }
         d4 acc[RT][NE] = {};
         const int rows = DOWN ? f.w : f.r;
-        if (DOWN) {
-            const double* Yb[NE];
-            const double* Xb[NE];
+        // the shares cut where the columns are (none for a front without rows)
+        const int q0 = rows > 0 ? ks * wave / KW : 0, q1 = rows > 0 ? ks * (wave + 1) / KW : 0;
+        // the output's own gathered part, final before this height (up)
+        double own[RT][NE] = {};
+        if (!DOWN && wave < 4) {
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                const size_t te = min(eg * NE + e, nt - 1);
-                Yb[e] = Y + (te * ny + (f.off - t.n_leaf)) * E + j;
-                Xb[e] = X + te * n * E + j;
-            }
-            // the quarters cut where the columns are
-            const int q0 = ks * wave / 4, q1 = ks * (wave + 1) / 4;
-            product<RT, NE, 4>(A, min(q0, kw), min(q1, kw),
-                               [&](int k, int e) { return Yb[e][min(4 * k + kk, f.w - 1) * E]; }, acc);
-            const int* br = t.brow + f.brow + kk - 4 * kw;
-            product<RT, NE, 4>(A, max(q0, kw), max(q1, kw),
-                               [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc);
-        } else {
-            // b' [4 kw][NE][E], zero past w
-            for (int q = tid; q < 4 * kw * NE * E; q += 256) {
-                const int row = q / (NE * E), e = (q / E) % NE;
-                const size_t te = min(eg * NE + e, nt - 1);
-                double v = 0.0;
-                if (row < f.w) {
-                    v = W[(te * n + f.off + row) * E + q % E]
-                        + gathered(t, f.arow + row, C + te * (t.n_c + 1) * E + q % E);
-                    if (tk.tile == 0 && eg * NE + e < nt) Y[(te * ny + (f.off - t.n_leaf) + row) * E + q % E] = v;
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int e = 0; e < NE; e++) {
+                    const int row = min((tk.tile + r) * 16 + kk + 4 * wave, rows - 1);
+                    const size_t te = min(eg * NE + e, nt - 1);
+                    if (rows > 0) own[r][e] = gathered(t, f.arow + f.w + row, C + te * (t.n_c + 1) * E + j);
                 }
-                lds[q] = v;
+        }
+        if (FUSED && !DOWN) {
+            // b' [4 kw][E], zero past w; four rows' loads in flight a thread
+            constexpr int RS = 64 * KW / E;
+            const int col = tid % E;
+            const double* Wb = W + ((size_t)eg * n + f.off) * E + col;
+            const double* Cb = C + (size_t)eg * (t.n_c + 1) * E + col;
+            double* Yw = Y + ((size_t)eg * ny + (f.off - t.n_leaf)) * E + col;
+            // this wavefront's share of F, loaded meanwhile (a share has at most kFrontCols / 4 / KW steps)
+            constexpr int AU = (sbf::kFrontCols / 4 + KW - 1) / KW;
+            double a[AU];
+#pragma unroll
+            for (int k = 0; k < AU; k++) a[k] = A[0][(size_t)min(q0 + k, max(q1 - 1, 0)) * 64 * (rows > 0 ? 1 : 0)];
+            for (int r0 = tid / E; r0 < 4 * kw; r0 += 4 * RS) {
+                int4 src[4];
+                int2 more[4];
+                double v[4][5];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const sbf::AsmRow* ar = t.arow + f.arow + min(r0 + q * RS, f.w - 1);
+                    src[q] = *reinterpret_cast<const int4*>(ar->s);
+                    more[q] = *reinterpret_cast<const int2*>(&ar->xb);
+                    v[q][4] = Wb[(size_t)min(r0 + q * RS, f.w - 1) * E];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    v[q][0] = Cb[(size_t)src[q].x * E];
+                    v[q][1] = Cb[(size_t)src[q].y * E];
+                    v[q][2] = Cb[(size_t)src[q].z * E];
+                    v[q][3] = Cb[(size_t)src[q].w * E];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int row = r0 + q * RS;
+                    double x = (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
+                    for (int k = more[q].x; k < more[q].y; k++) x += Cb[(size_t)t.xsrc[k] * E];
+                    x += v[q][4];
+                    if (row < 4 * kw) lds[row * E + col] = row < f.w ? x : 0.0;
+                    if (tk.tile == 0 && row < f.w) Yw[(size_t)row * E] = x;
+                }
             }
             __syncthreads();
-            product<RT, NE, 4>(A, kw * wave / 4, rows > 0 ? kw * (wave + 1) / 4 : kw * wave / 4,
-                               [&](int k, int e) { return lds[((4 * k + kk) * NE + e) * E + j]; }, acc);
+#pragma unroll
+            for (int k = 0; k < AU; k++)
+                if (q0 + k < q1) acc[0][0] = mfma(a[k], lds[(4 * (q0 + k) + kk) * E + j], acc[0][0]);
             __syncthreads();
+        } else {
+            product<RT, NE, U>(A, min(q0, kw), min(q1, kw),
+                               [&](int k, int e) { return Yb[e][min(4 * k + kk, f.w - 1) * E]; }, acc);
+            if (DOWN) {
+                const int* br = t.brow + f.brow + kk - 4 * kw;
+                product<RT, NE, U>(A, max(q0, kw), max(q1, kw),
+                                   [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc);
+            }
         }
         // [wavefront][row tile][env tile][register][lane]
         double* red = lds;
@@ -208,23 +270,21 @@ __global__ __launch_bounds__(256) void front_kernel(sbf::FrontTab t, int task0, 
 #pragma unroll
                 for (int q = 0; q < 4; q++) red[(((wave * RT + r) * NE + e) * 4 + q) * 64 + lane] = acc[r][e][q];
         __syncthreads();
-        // wavefront q' finishes register q' of every tile
+        // wavefront q finishes register q of every tile
+        if (wave < 4) {
 #pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const int row = (tk.tile + r) * 16 + kk + 4 * wave;
-            if (r >= m || row >= rows) continue;
+            for (int r = 0; r < RT; r++) {
+                const int row = (tk.tile + r) * 16 + kk + 4 * wave;
+                if (r >= m || row >= rows) continue;
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                const size_t te = eg * NE + e;
-                if ((int)te >= nt) continue;
-                double v = 0.0;
+                for (int e = 0; e < NE; e++) {
+                    const size_t te = eg * NE + e;
+                    if ((int)te >= nt) continue;
+                    double v = 0.0;
 #pragma unroll
-                for (int w = 0; w < 4; w++) v += red[(((w * RT + r) * NE + e) * 4 + wave) * 64 + lane];
-                if (DOWN) {
-                    X[(te * n + f.off + row) * E + j] = v;
-                } else {
-                    double* Cb = C + te * (t.n_c + 1) * E + j;
-                    Cb[(size_t)(f.c + row) * E] = v + gathered(t, f.arow + f.w + row, Cb);
+                    for (int w = 0; w < KW; w++) v += red[(((w * RT + r) * NE + e) * 4 + wave) * 64 + lane];
+                    if (DOWN) X[(te * n + f.off + row) * E + j] = v;
+                    else C[(te * (t.n_c + 1) + f.c + row) * E + j] = v + own[r][e];
                 }
             }
         }
@@ -284,45 +344,59 @@ __global__ void ops_scatter_kernel(sbf::Tri tri, int nrows, const sbf::Front* fr
     }
 }
 
-// One thread per column of a front's operators: column c < w of K solves
+// One lane per column of a front's operators: column c < w of K solves
 // L U x = e_c, the next r solve U x = -U_CB, the last r (rows of F) z L = -L_BC.
-__global__ __launch_bounds__(64) void ops_solve_kernel(const sbf::Front* fronts, int n_fronts, OpsTab o) {
-    for (int fi = blockIdx.x; fi < n_fronts; fi += gridDim.x) {
-        const sbf::Front f = fronts[fi];
-        const int w = f.w, r = f.r, ld = w + 2 * r;
-        const double* L = o.dense + o.d0[fi];
-        const double* U = L + (size_t)w * w;
-        const double* LB = U + (size_t)w * w;
-        const double* UB = LB + (size_t)w * r;
-        double* S = o.sol + o.s0[fi];
-        for (int c = blockIdx.y * 64 + threadIdx.x; c < ld; c += gridDim.y * 64) {
-            double* x = S + c;   // x[m * ld]
-            if (c >= w + r) {
-                const int b = c - w - r;
-                for (int m = w - 1; m >= 0; m--) {
-                    double acc = -LB[(size_t)b * w + m];
-                    for (int q = m + 1; q < w; q++) acc = fma(-L[(size_t)q * w + m], x[(size_t)q * ld], acc);
-                    x[(size_t)m * ld] = acc;
-                }
-                continue;
+// A wavefront's 64 columns are kept in LDS; a row's coefficients are the same
+// for every lane (scalar loads), eight products a trip in four sums (columns
+// in global memory and one chain a row: 32 ms for a 205K-cell plan, 5 so).
+struct OpsCol {
+    double (*x)[64];
+    int lane;
+    // sum_q M[q * stride] x[q] over [q0, q1)
+    __device__ double dot(const double* M, size_t stride, int q0, int q1) const {
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        int q = q0;
+        for (; q + 8 <= q1; q += 8)
+#pragma unroll
+            for (int u = 0; u < 8; u++) s[u & 3] = fma(M[(size_t)(q + u) * stride], x[q + u][lane], s[u & 3]);
+        for (; q < q1; q++) s[0] = fma(M[(size_t)q * stride], x[q][lane], s[0]);
+        return (s[0] + s[1]) + (s[2] + s[3]);
+    }
+};
+
+__global__ __launch_bounds__(64) void ops_solve_kernel(const sbf::Front* fronts, OpsTab o) {
+    extern __shared__ double lds[];
+    const OpsCol X{reinterpret_cast<double (*)[64]>(lds), (int)threadIdx.x};
+    const int fi = blockIdx.x;
+    const sbf::Front f = fronts[fi];
+    const int w = f.w, r = f.r, ld = w + 2 * r;
+    const double* L = o.dense + o.d0[fi];
+    const double* U = L + (size_t)w * w;
+    const double* LB = U + (size_t)w * w;
+    const double* UB = LB + (size_t)w * r;
+    double* S = o.sol + o.s0[fi];
+    // columns of the three kinds apart, 64 at a time, so a wavefront runs one kind
+    const int nw = (w + 63) / 64, nr = (r + 63) / 64;
+    for (int g = blockIdx.y; g < nw + 2 * nr; g += gridDim.y) {
+        const int kind = g < nw ? 0 : g < nw + nr ? 1 : 2;
+        const int c = (kind == 0 ? g : kind == 1 ? g - nw : g - nw - nr) * 64 + X.lane;
+        const bool ok = c < (kind == 0 ? w : r);
+        const int cc = ok ? c : 0;
+        if (kind == 2) {
+            for (int m = w - 1; m >= 0; m--)
+                X.x[m][X.lane] = -LB[(size_t)cc * w + m] - X.dot(L + m, w, m + 1, w);
+        } else {
+            for (int m = 0; m < w; m++) {
+                double b = kind == 0 ? (m == cc ? 1.0 : 0.0) : -UB[(size_t)m * r + cc];
+                if (kind == 0) b -= X.dot(L + (size_t)m * w, 1, 0, m);
+                X.x[m][X.lane] = b;
             }
-            if (c < w) {
-                for (int m = 0; m < c; m++) x[(size_t)m * ld] = 0.0;
-                x[(size_t)c * ld] = 1.0;
-                for (int m = c + 1; m < w; m++) {
-                    double acc = 0.0;
-                    for (int q = c; q < m; q++) acc = fma(-L[(size_t)m * w + q], x[(size_t)q * ld], acc);
-                    x[(size_t)m * ld] = acc;
-                }
-            } else {
-                for (int m = 0; m < w; m++) x[(size_t)m * ld] = -UB[(size_t)m * r + (c - w)];
-            }
-            for (int m = w - 1; m >= 0; m--) {
-                double acc = x[(size_t)m * ld];
-                for (int q = m + 1; q < w; q++) acc = fma(-U[(size_t)m * w + q], x[(size_t)q * ld], acc);
-                x[(size_t)m * ld] = acc / U[(size_t)m * w + m];
-            }
+            for (int m = w - 1; m >= 0; m--)
+                X.x[m][X.lane] = (X.x[m][X.lane] - X.dot(U + (size_t)m * w, 1, m + 1, w)) / U[(size_t)m * w + m];
         }
+        const int at = kind == 0 ? c : kind == 1 ? w + c : w + r + c;
+        if (ok)
+            for (int m = 0; m < w; m++) S[(size_t)m * ld + at] = X.x[m][X.lane];
     }
 }
 
@@ -488,14 +562,14 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
     }
 }
 
-size_t front_lds(bool down, int rt, int ne, int wmax) {
-    const size_t red = (size_t)4 * rt * ne * 256, b = down ? 0 : (size_t)((wmax + 3) / 4 * 4) * ne * E;
+size_t front_lds(bool fused, int rt, int ne, int kw, int wmax) {
+    const size_t red = (size_t)kw * rt * ne * 256, b = fused ? (size_t)((wmax + 3) / 4 * 4) * E : 0;
     return sizeof(double) * std::max(red, b);
 }
 
-// Workgroups below which a height runs on single row and env tiles: with 2 x 2
-// tiles a workgroup reads half as much per product, but a height of fewer
-// than two workgroups a CU leaves matrix cores idle.
+// Workgroups (2 x 2 tiles) below which a height counts as narrow: with fewer
+// than two workgroups a CU the matrix cores idle and the chain of latencies is
+// what the height costs.
 constexpr unsigned kWideGroups = 512;
 
 template <bool DOWN>
@@ -517,12 +591,16 @@ void launch_level(const sbf::Tables& t, const sbf::Group& g, int h, hipStream_t 
         return;
     }
     const unsigned wide = (unsigned)((m + 1) / 2) * ((nt + 1) / 2);
-    if (nt > 1 && wide >= kWideGroups)
-        hipLaunchKernelGGL((front_kernel<DOWN, 2, 2>), dim3(wide), dim3(256), front_lds(DOWN, 2, 2, L.wmax), s, t.ft,
-                           t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
-    else
-        hipLaunchKernelGGL((front_kernel<DOWN, 1, 1>), dim3((unsigned)m * nt), dim3(256),
-                           front_lds(DOWN, 1, 1, L.wmax), s, t.ft, t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
+    if (nt > 1 && wide >= kWideGroups) {
+        if (!DOWN)
+            hipLaunchKernelGGL(assemble_kernel, dim3((unsigned)L.nk * nt), dim3(256), 0, s, t.ft, L.k0, L.nk, t.n, g.nt,
+                               g.W1, g.Y, g.C);
+        hipLaunchKernelGGL((front_kernel<DOWN, false, 2, 2, 4, 4>), dim3(wide), dim3(256),
+                           front_lds(false, 2, 2, 4, L.wmax), s, t.ft, t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
+    } else {
+        hipLaunchKernelGGL((front_kernel<DOWN, !DOWN, 1, 1, 8, 8>), dim3((unsigned)m * nt), dim3(512),
+                           front_lds(!DOWN, 1, 1, 8, L.wmax), s, t.ft, t0, m, t.n, g.nt, g.W1, g.Y, g.C, g.X);
+    }
 }
 
 }  // namespace
@@ -545,10 +623,11 @@ extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* g, 
     return (int)hipGetLastError();
 }
 
-// The fronts' operators from the factors (rows scheduled in L and U: nl, nu),
+// The fronts' operators from the factors (rows scheduled in L and U: nl, nu;
+// the first leaf_fronts fronts are the leaves),
 // on the null stream; front_of, local, bperm: FrontPlan's, on the device;
 // d0, s0: per front the offsets of its dense blocks and solutions.
-extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, const int* front_of, const int* local,
+extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, int leaf_fronts, const int* front_of, const int* local,
                                     const int* bperm, const long long* d0, const long long* s0, double* dense,
                                     double* sol, double* ops) {
     const OpsTab o{front_of, local, bperm, d0, dense, sol, s0};
@@ -557,7 +636,24 @@ extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, const 
     if (nl > 0)
         hipLaunchKernelGGL((ops_scatter_kernel<false>), dim3((nl + 255) / 256), dim3(256), 0, nullptr, t->L, nl, fr, o);
     hipLaunchKernelGGL((ops_scatter_kernel<true>), dim3((nu + 255) / 256), dim3(256), 0, nullptr, t->U, nu, fr, o);
-    hipLaunchKernelGGL(ops_solve_kernel, dim3(nf, 4), dim3(64), 0, nullptr, fr, nf, o);
+    int wmax = 1;
+    for (int h = 0; h < t->ft.n_levels; h++) wmax = std::max(wmax, t->ft.levels[h].wmax);
+    const size_t lds = sizeof(double) * 64 * (size_t)wmax;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute((const void*)ops_solve_kernel,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    // leaves (the fronts before the first one above them) have at most 64 columns
+    const int leaves = t->ft.n_levels > 1 ? leaf_fronts : nf;
+    const size_t small = sizeof(double) * 64 * (size_t)sbf::kLeafCols;
+    hipLaunchKernelGGL(ops_solve_kernel, dim3(leaves, 3), dim3(64), small, nullptr, fr, o);
+    if (nf > leaves) {
+        OpsTab up = o;
+        up.d0 += leaves;
+        up.s0 += leaves;
+        hipLaunchKernelGGL(ops_solve_kernel, dim3(nf - leaves, 16), dim3(64), lds, nullptr, fr + leaves, up);
+    }
     hipLaunchKernelGGL(ops_pack_kernel, dim3(nf), dim3(256), 0, nullptr, fr, nf, o, ops);
     return (int)hipGetLastError();
 }
