@@ -215,20 +215,53 @@ __global__ __launch_bounds__(64) void dense_kernel(sbf::Tables t, sbf::Group g, 
     }
 }
 
-// The same solve per env with M, the power row and the step's row factors in
-// LDS, one workgroup of kDenseThreads per env (k <= kDenseLdsK). Every value
-// sees the operations of sb_fdm.c:9-38 in their order: the pivot is the first
-// row reaching the largest |M[r][c]| over r >= c (NaNs never win; row c stays
-// when |M[c][c]| is NaN), as the sequential strictly-greater scan picks it;
-// the rows' factors f = M[r][c] / d are taken before the step's updates;
-// M[r][j] -= f M[c][j] for j >= c (the product rounded: this file is built
-// without contraction) and b[r] -= f b[c], rows with f == 0 skipped; then
-// lane 0 back-substitutes row by row, each row's terms in ascending column.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ double dpp_d(double v) {
+    const unsigned long long x = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp((int)(unsigned)x, (int)(unsigned)x, CTRL, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(unsigned)(x >> 32), (int)(unsigned)(x >> 32), CTRL, ROWS, 0xF, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ __forceinline__ double lane_d(double v, int l) {
+    const unsigned long long x = __double_as_longlong(v);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), l) << 32)
+                                            | (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, l)));
+}
+// The largest value over the wavefront's lanes (no NaN among them).
+__device__ __forceinline__ double lane_max(double v) {
+    v = fmax(v, dpp_d<0xB1>(v));          // quad_perm [1,0,3,2]
+    v = fmax(v, dpp_d<0x4E>(v));          // quad_perm [2,3,0,1]
+    v = fmax(v, dpp_d<0x141>(v));         // row_half_mirror
+    v = fmax(v, dpp_d<0x140>(v));         // row_mirror
+    v = fmax(v, dpp_d<0x142, 0xA>(v));    // row_bcast:15
+    v = fmax(v, dpp_d<0x143, 0xC>(v));    // row_bcast:31
+    return lane_d(v, 63);
+}
+
+// The same solve per env with M and the power row in LDS (k <= kDenseLdsK),
+// columns apart: M[j][r], column k the power row; one workgroup of 4
+// wavefronts per env, lane l row l (and l + 64 for k > 64: RW 2). Every wavefront finds the
+// step's pivot and its own rows' factors from column c by itself (lane moves
+// and one division), then swaps and updates every fourth later column, so a
+// step needs one barrier (a pivot search, a swap, factors and updates of all
+// elements with a barrier after each: 83 us for k = 39; this form 44, what is
+// left is the chain of the k steps). Every value sees the operations of
+// sb_fdm.c:9-38 in their order: the pivot is the first row reaching the largest
+// |M[r][c]| over r >= c (NaNs never win; row c stays when |M[c][c]| is NaN), as
+// the sequential strictly-greater scan picks it; f = M[r][c] / d;
+// M[r][j] -= f M[c][j] (the product rounded: this file is built without
+// contraction) and b[r] -= f b[c], rows with f == 0 skipped. The back
+// substitution takes each row's terms in ascending column on one lane (EXACT),
+// or each column's terms of all rows at once.
 constexpr int kDenseThreads = 256, kDenseLdsK = 89;
+constexpr size_t dense_lds_bytes(int k) { return sizeof(double) * ((size_t)k * (k + 1) + k); }
+
+template <bool EXACT, int RW>
 __global__ __launch_bounds__(kDenseThreads) void dense_lds_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
-    extern __shared__ __align__(16) double dl[];
-    __shared__ int s_piv, s_sing;
-    const int env = blockIdx.x, k = t.k, tid = threadIdx.x;
+    extern __shared__ __align__(16) double M[];   // [k + 1][k], then the pivots [k]
+    const int env = blockIdx.x, k = t.k, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = kDenseThreads / 64;
     const double* gv = in.g + (size_t)env * k;
     int any = 0;
     for (int i = tid; i < k; i += kDenseThreads) any |= gv[i] != 0.0;
@@ -238,82 +271,108 @@ __global__ __launch_bounds__(kDenseThreads) void dense_lds_kernel(sbf::Tables t,
         if (any) atomicOr(&g.bact[env / g.Gl], 1);
     }
     if (!any) return;   // workgroup-uniform
-    double* M = dl;             // [k][k]
-    double* bv = dl + k * k;    // [k]
-    double* fr = bv + k;        // [k]: the step's row factors
+    double* bv = M + k * k;
+    double* dv = bv + k;
     double* pw = g.pw + (size_t)env * k;
     for (int x = tid; x < k * k; x += kDenseThreads) {
         const int i = x / k, j = x % k;
-        M[x] = (i == j ? 1.0 : 0.0) + gv[i] * t.S[x];
+        M[j * k + i] = (i == j ? 1.0 : 0.0) + gv[i] * t.S[x];
     }
     for (int i = tid; i < k; i += kDenseThreads) bv[i] = pw[i];
     __syncthreads();
+    int row[RW], q[RW];   // this lane's rows, and as readable ones
+#pragma unroll
+    for (int u = 0; u < RW; u++) {
+        row[u] = lane + 64 * u;
+        q[u] = min(row[u], k - 1);
+    }
     for (int c = 0; c < k; c++) {
-        if (tid < 64) {
-            double m = -1.0;
-            for (int r = c + tid; r < k; r += 64) {
-                const double v = fabs(M[r * k + c]);
-                if (v > m) m = v;
-            }
-            for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-            int first = k;
-            for (int r = c + tid; r < k; r += 64)
-                if (fabs(M[r * k + c]) == m) {
-                    first = r;
-                    break;
-                }
-            for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o));
-            if (tid == 0) {
-                const double vc = fabs(M[c * k + c]);
-                const bool nan_c = vc != vc;
-                s_piv = nan_c ? c : first;
-                s_sing = !nan_c && m == 0.0;
-            }
+        const double vc = M[c * k + c];
+        double v[RW], a[RW], m = -1.0;
+#pragma unroll
+        for (int u = 0; u < RW; u++) {
+            v[u] = M[c * k + q[u]];
+            a[u] = row[u] >= c && row[u] < k && fabs(v[u]) >= 0.0 ? fabs(v[u]) : -1.0;
+            m = a[u] > m ? a[u] : m;
         }
-        __syncthreads();
-        if (s_sing) {
+        m = lane_max(m);
+        const bool nan_c = vc != vc;
+        int first = -1;
+#pragma unroll
+        for (int u = RW - 1; u >= 0; u--) {
+            const unsigned long long eq = __ballot(a[u] == m);
+            if (eq) first = 64 * u + __ffsll((long long)eq) - 1;
+        }
+        if (!nan_c && m == 0.0) {
             // the reference returns here, leaving the partly reduced row
             for (int i = tid; i < k; i += kDenseThreads) pw[i] = bv[i];
             return;
         }
-        const int piv = s_piv;
-        if (piv != c) {
-            for (int j = c + tid; j < k; j += kDenseThreads) {
-                const double x = M[c * k + j];
-                M[c * k + j] = M[piv * k + j];
-                M[piv * k + j] = x;
-            }
-            if (tid == 0) {
-                const double x = bv[c];
-                bv[c] = bv[piv];
-                bv[piv] = x;
-            }
-            __syncthreads();
+        const int piv = __builtin_amdgcn_readfirstlane(nan_c ? c : first);
+        const double d = lane_d(piv < 64 ? v[0] : v[RW - 1], piv & 63);
+        double f[RW];
+        bool on[RW], is_p[RW], is_c[RW];
+#pragma unroll
+        for (int u = 0; u < RW; u++) {
+            is_p[u] = row[u] == piv;
+            is_c[u] = row[u] == c;
+            f[u] = (is_p[u] ? vc : v[u]) / d;
+            on[u] = row[u] > c && f[u] != 0.0;
         }
-        const double d = M[c * k + c];
-        for (int r = c + 1 + tid; r < k; r += kDenseThreads) fr[r] = M[r * k + c] / d;
-        __syncthreads();
-        const int nc = k - c, nx = (k - c - 1) * nc;
-        for (int x = tid; x < nx; x += kDenseThreads) {
-            const int r = c + 1 + x / nc, j = c + x % nc;
-            const double f = fr[r];
-            if (f != 0.0) M[r * k + j] -= f * M[c * k + j];
-        }
-        for (int r = c + 1 + tid; r < k; r += kDenseThreads) {
-            const double f = fr[r];
-            if (f != 0.0) bv[r] -= f * bv[c];
+        if (tid == 0) dv[c] = d;
+        for (int j0 = c + 1 + wave; j0 <= k; j0 += 4 * NW) {
+            // four columns' loads in flight; rows past c's swap are written
+            // back as they were
+            double p[4], oc[4], z[4][RW];
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const double* col = M + min(j0 + w * NW, k) * k;
+                p[w] = col[piv];
+                oc[w] = col[c];
+#pragma unroll
+                for (int u = 0; u < RW; u++) z[w][u] = col[q[u]];
+            }
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                double* col = M + min(j0 + w * NW, k) * k;
+#pragma unroll
+                for (int u = 0; u < RW; u++) {
+                    double x = is_p[u] ? oc[w] : z[w][u];
+                    const double y = x - f[u] * p[w];
+                    x = is_c[u] ? p[w] : on[u] ? y : x;
+                    if (row[u] < k && j0 + w * NW <= k) col[row[u]] = x;
+                }
+            }
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        for (int r = k - 1; r >= 0; r--) {
-            double s = bv[r];
-            for (int j = r + 1; j < k; j++) s -= M[r * k + j] * bv[j];
-            bv[r] = s / M[r * k + r];
+    if (wave != 0) return;
+    if (EXACT) {
+        if (lane == 0) {
+            for (int r = k - 1; r >= 0; r--) {
+                double s = bv[r];
+                for (int j = r + 1; j < k; j++) s -= M[j * k + r] * bv[j];
+                bv[r] = s / dv[r];
+            }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        for (int i = lane; i < k; i += 64) pw[i] = bv[i];
+    } else {
+        double b[RW];
+#pragma unroll
+        for (int u = 0; u < RW; u++) b[u] = bv[q[u]];
+        for (int j = k - 1; j >= 0; j--) {
+            const double x = lane_d(j < 64 ? b[0] : b[RW - 1], j & 63) / dv[j];
+#pragma unroll
+            for (int u = 0; u < RW; u++) {
+                const double y = b[u] - M[j * k + q[u]] * x;
+                b[u] = row[u] == j ? x : row[u] < j ? y : b[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < RW; u++)
+            if (row[u] < k) pw[row[u]] = b[u];
     }
-    __syncthreads();
-    for (int i = tid; i < k; i += kDenseThreads) pw[i] = bv[i];
 }
 
 // The applied heat of the solved powers (sb_fdm.c:171-177), permuted into the
@@ -454,9 +513,15 @@ int solve(const sbf::Tables& t, const sbf::Group& g, double* W, const int* bact,
 
 // Whether each env's air side is on and, where it is, its power row solved.
 extern "C" int sbf_launch_dense(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s) {
-    if (t->k <= kDenseLdsK)
-        hipLaunchKernelGGL(dense_lds_kernel, dim3(g->G), dim3(kDenseThreads),
-                           sizeof(double) * ((size_t)t->k * t->k + 2 * (size_t)t->k), s, *t, *g, *in);
+    const size_t lds = dense_lds_bytes(t->k);
+    if (t->k <= 64 && t->fast)
+        hipLaunchKernelGGL((dense_lds_kernel<false, 1>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
+    else if (t->k <= 64)
+        hipLaunchKernelGGL((dense_lds_kernel<true, 1>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
+    else if (t->k <= kDenseLdsK && t->fast)
+        hipLaunchKernelGGL((dense_lds_kernel<false, 2>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
+    else if (t->k <= kDenseLdsK)
+        hipLaunchKernelGGL((dense_lds_kernel<true, 2>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
     else
         hipLaunchKernelGGL(dense_kernel, dim3(g->G), dim3(64), 0, s, *t, *g, *in);
     return (int)hipGetLastError();
