@@ -614,7 +614,7 @@ bool field_attach(FieldScen* f, const std::string& path, const std::vector<sbe::
         // leave half of a compute unit's LDS to the field's workgroups
         const int mr_lds = f->t.cv_max_room;
         const double expect = 1.5 * std::min(std::max(f->conv_p, 0.0), 1.0) * mr_lds;
-        f->lds_pairs = std::min(mr_lds, std::max(512, (int)expect));
+        f->lds_pairs = std::max(512, (int)expect);
         auto need = [&](int pairs, int n) {
             const sbe::ConvLds L = sbe::conv_lds(mr_lds, pairs);
             return L.base + n * L.slot;

@@ -186,17 +186,17 @@ struct Slot {
 
 enum { FE_STEP = 0, FE_RESET = 1 };
 
-// The convection plan kernel's LDS for rooms of up to `room` cells: two MT
-// blocks (raw and tempered) and the room's candidate counts (with up to 15
-// cells before and after it), then per applier `pairs` pairs (u32) and shuffle
-// draws (u16) and the room's inverse permutation (u16).
+// The convection plan kernel's LDS for rooms of up to `room` cells: four MT
+// blocks, a record and the low byte of each of their words, the room's
+// candidate counts (with up to 15 cells before and after it), then per applier `pairs` pairs
+// (u32) and shuffle draws (u16) and the room's inverse permutation (u16).
 struct ConvLds {
     size_t base, slot, jd, q;
 };
-constexpr int kConvAppliers = 3;
+constexpr int kConvAppliers = 2;
 constexpr ConvLds conv_lds(int room, int pairs) {
     const size_t jd = 4 * (size_t)pairs, q = (jd + 2 * (size_t)pairs + 3) & ~(size_t)3;
-    return ConvLds{16 * (size_t)SBE_MT_N + (((size_t)room + 47) & ~(size_t)15),
+    return ConvLds{(36 * (size_t)SBE_MT_N + 16 + (size_t)room + 47) & ~(size_t)15,
                    (q + 2 * ((size_t)room + 1) + 15) & ~(size_t)15, jd, q};
 }
 
@@ -238,7 +238,7 @@ struct Args {
     double* cv_vals;              // [G][cv_cells]
     unsigned int* cv_spill;       // [G][cv_appliers][2][cv_max_room]: pairs, then shuffle draws, past the LDS
     int cv_lds_pairs;             // pairs the plan kernel keeps in LDS per applier
-    int cv_appliers;              // its wavefronts beside the stream's
+    int cv_appliers;              // its wavefronts that take rooms from the stream's
     int exact;                    // the field group runs in exact mode (SBX_FDM_EXACT): sums in the reference's order
 };
 

@@ -115,9 +115,8 @@ __device__ __forceinline__ uint32_t mt_temper(uint32_t y) {
 }
 
 // Each range: every lane's loads (at most four words per lane) issued before
-// its first store, so a range costs one LDS round trip. `tw`, if given,
-// receives the tempered words of the new block as well.
-__device__ void mt_next_block(const uint32_t* src, uint32_t* dst, uint32_t* tw = nullptr) {
+// its first store, so a range costs one LDS round trip.
+__device__ void mt_next_block(const uint32_t* src, uint32_t* dst) {
     auto range = [&](int lo, int hi, bool far_new) {
         uint32_t a[4], b[4], f[4];
 #pragma unroll
@@ -132,11 +131,7 @@ __device__ void mt_next_block(const uint32_t* src, uint32_t* dst, uint32_t* tw =
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int i = lo + u * W + lane();
-            if (i < hi) {
-                const uint32_t x = mt_mix(a[u], b[u], f[u]);
-                dst[i] = x;
-                if (tw) tw[i] = mt_temper(x);
-            }
+            if (i < hi) dst[i] = mt_mix(a[u], b[u], f[u]);
         }
         wsync();
     };
@@ -936,46 +931,113 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 //
 // One workgroup per env. Its first wavefront walks the stream, which is one
 // serial chain over the rooms: the cells' swaps and candidates, then the
-// shuffle's draws. The others (appliers) each take every conv_appliers-th
-// room once its draws are posted: the candidates' cells, the shuffle and its
-// composition, the moves. What bounds it is the first wavefront's chain of
-// scalar instructions, one swap after another. At 256 envs of the 205K-cell
-// building (about 13,500 swaps a step): 10.4 ms with everything on one
-// wavefront, 4.1 ms with the shuffle's draws resolved 64 words at a time, the
-// rooms applied beside the stream and a swap loop of one straight line.
-//
-// Stream: raw blocks in LDS, two at a time (the current one and, once a read
-// reaches past it, the next), each with its tempered copy, positions relative
-// to the current block.
+// shuffle's draws. The second (the producer) runs up to three MT blocks ahead
+// of it: the words and, for every word position, where the next swap would be
+// and its draw's first bytes, none of which depends on the walk. The others (appliers) each take every
+// n-th room once its draws are posted: the candidates' cells, the shuffle and
+// its composition, the moves. What bounds it is the walk's chain of scalar
+// instructions, one swap after another. At 256 envs of the 205K-cell building
+// (about 14,500 swaps a step): 10.4 ms with everything on one wavefront, 4.0 ms
+// with the rooms applied beside the stream, 3.5 ms with the producer (the
+// walk's windows had cost as much as its swaps).
 namespace {
 
-struct Stream {
-    uint32_t* raw;     // [2][624]
-    uint32_t* tw;      // [2][624] tempered
-    int pos;           // next word to consume, from the current block's word 0
-    int cur;           // which of the two is the current block
-    bool have_next;
+constexpr int kWin = 96;             // words of a walk window
+constexpr int kRing = 4;             // MT blocks in LDS
+constexpr int kRingWords = kRing * SBE_MT_N;
+constexpr int kRingPad = 8;          // the ring's first words again, so that reads past a window need no wrap
+static_assert(kRingWords % kWin == 0 && kWin % 2 == 0 && kWin / 2 <= W, "windows tile the ring, two words a lane");
 
-    // word q (from the current block's word 0)
-    __device__ uint32_t word(int q) const {
-        const int x = q + (cur ? SBE_MT_N : 0);
-        return tw[x >= 2 * SBE_MT_N ? x - 2 * SBE_MT_N : x];
-    }
-    // words up to pos + ahead (< 624) readable
-    __device__ void ensure(int ahead) {
-        while (pos + ahead >= SBE_MT_N * (have_next ? 2 : 1)) {
-            if (!have_next) {
-                const int nb = cur ^ 1;
-                mt_next_block(raw + cur * SBE_MT_N, raw + nb * SBE_MT_N, tw + nb * SBE_MT_N);
-                have_next = true;
-            } else {
-                pos -= SBE_MT_N;
-                cur ^= 1;
-                have_next = false;
-            }
+// The stream's LDS, shared by the walk and the producer. Positions are words
+// from the step's first block, which sits at the ring's start.
+//
+// rec[p]: what the walk needs to know at word p, if a cell's draw starts there.
+// Byte 0: words to the next position of p's parity (p itself included) in p's
+// window where a cell would swap, kNone if there is none; bytes 1..3: the low
+// bytes of that position's words + 2, + 3, + 4, the candidate draw's first.
+struct Words {
+    uint32_t* raw;                 // [kRingWords]
+    uint32_t* rec;                 // [kRingWords]
+    uint8_t* low;                  // [kRingWords + kRingPad]: the tempered words' low bytes
+    int* ready;                    // windows prepared
+    int* used;                     // the block that holds the last word consumed; -1 once the walk is done
+};
+constexpr uint32_t kNone = 0xffu;
+
+// A post and the wait for one: every post that a wavefront waits for is made
+// by another that never waits for it meanwhile.
+__device__ __forceinline__ void post(int* flag, int v) {
+    __builtin_amdgcn_wave_barrier();
+    if (lane() == 0) __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ int peek(int* flag) {
+    return __builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+
+// The walk's side of the stream.
+struct Stream {
+    Words w;
+    int pos;       // next word to consume
+    int ready;     // blocks known to be prepared
+    int used;      // posted last
+
+    // window b prepared, so every word up to word q in it readable; what lies
+    // before the walk's word (q or before) is given back first (the producer
+    // needs the room for the next two blocks past it)
+    __device__ void need_window(int b, int q) {
+        if (q - 1 >= (used + 1) * SBE_MT_N) post(w.used, ++used);
+        while (ready <= b) {
+            ready = peek(w.ready);
+            if (ready <= b) __builtin_amdgcn_s_sleep(1);
         }
     }
+    // words up to pos + ahead readable
+    __device__ void need(int ahead) {
+        const int u = pos > 0 ? (pos - 1) / SBE_MT_N : 0;
+        if (u > used) post(w.used, used = u);
+        need_window((pos + ahead) / kWin, 0);
+    }
+    __device__ uint32_t word(int q) const { return mt_temper(w.raw[q % kRingWords]); }
 };
+
+// The producer: MT blocks while the ring has room, and behind them the
+// windows' records. A window's last swap draw reads the word after it and its
+// records bytes up to four words past it, so a window is prepared once the
+// words 8 past it are there.
+__device__ void produce(const Words& w, uint64_t thr, bool never) {
+    const int l2 = 2 * min(lane(), kWin / 2 - 1);
+    int win = 0;   // next window to prepare
+    for (int b = 0;; b++) {
+        int u;
+        while ((u = peek(w.used)) >= 0 && b > u + kRing - 1) __builtin_amdgcn_s_sleep(2);
+        if (u < 0) return;
+        const int r = (b % kRing) * SBE_MT_N;
+        if (b > 0) mt_next_block(w.raw + (b + kRing - 1) % kRing * SBE_MT_N, w.raw + r);
+        for (int i = lane(); i < SBE_MT_N; i += W) {
+            const uint8_t x = (uint8_t)mt_temper(w.raw[r + i]);
+            w.low[r + i] = x;
+            if (r + i < kRingPad) w.low[kRingWords + r + i] = x;
+        }
+        wsync();
+        for (; (win + 1) * kWin + kRingPad <= (b + 1) * SBE_MT_N; win++) {
+            const int x0 = win * kWin % kRingWords, p = x0 + l2;
+            const uint32_t w0 = mt_temper(w.raw[p]), w1 = mt_temper(w.raw[p + 1]);
+            const uint32_t w2 = mt_temper(w.raw[p + 2 == kRingWords ? 0 : p + 2]);
+            const uint64_t u0 = ((uint64_t)(w0 >> 5) << 26) | (uint64_t)(w1 >> 6);
+            const uint64_t u1 = ((uint64_t)(w1 >> 5) << 26) | (uint64_t)(w2 >> 6);
+            const unsigned long long in = ~0ull >> (64 - kWin / 2);
+            const unsigned long long P0 = ballot(!never && u0 <= thr) & in, P1 = ballot(!never && u1 <= thr) & in;
+            const unsigned long long n0 = P0 >> (l2 >> 1), n1 = P1 >> (l2 >> 1);
+            const int d0 = n0 ? 2 * first_lane(n0) : 0, d1 = n1 ? 2 * first_lane(n1) : 0;
+            const uint8_t *c0 = w.low + p + d0 + 2, *c1 = w.low + p + 1 + d1 + 2;
+            const uint32_t e0 = (uint32_t)c0[0] << 8 | (uint32_t)c0[1] << 16 | (uint32_t)c0[2] << 24;
+            const uint32_t e1 = (uint32_t)c1[0] << 8 | (uint32_t)c1[1] << 16 | (uint32_t)c1[2] << 24;
+            if (lane() < kWin / 2)
+                *reinterpret_cast<uint2*>(w.rec + p) = make_uint2(e0 | (n0 ? (uint32_t)d0 : kNone), e1 | (n1 ? (uint32_t)d1 : kNone));
+        }
+        post(w.ready, win);
+    }
+}
 
 __device__ __forceinline__ uint32_t smear(uint32_t x) { return x ? 0xffffffffu >> __clz((int)x) : 0u; }
 
@@ -1001,116 +1063,101 @@ struct RoomSlot {
     }
 };
 
-// Posts between the wavefronts of a workgroup, and the wait for one: every
-// post a wavefront waits for is made by another that never waits for it.
-__device__ __forceinline__ void slot_post(int* flag, int v) {
-    __builtin_amdgcn_wave_barrier();
-    if (lane() == 0) __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
+// Waits until a slot's flag holds a room (its pairs, 0 or more) or is free (-1).
 __device__ __forceinline__ int slot_wait(int* flag, bool full) {
     int v;
-    while (((v = __hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) >= 0) != full)
-        __builtin_amdgcn_s_sleep(2);
-    return __builtin_amdgcn_readfirstlane(v);
+    while (((v = peek(flag)) >= 0) != full) __builtin_amdgcn_s_sleep(2);
+    return v;
 }
 
-// The room's pairs from the stream; returns their count. Windows of 128
-// words: lane l holds the words at offsets 2l, 2l + 1, 2l + 2 of the window.
-// The walk is at word x; the drift (what the window's swapping cells have
-// taken beyond two words each) has x's parity, so the swap bits of the cells
-// that start at x's parity are one ballot (P0, P1), the next swapping cell is
-// its next set bit, and that cell's candidate draw reads the low bytes of the
-// following words (a cell has at most 255 candidates).
-__device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n, uint64_t thr, bool never) {
-    int m = 0;
-    for (int j = 0; j < n;) {
-        S.ensure(2 * W);
-        const int p = S.pos + 2 * lane();
-        const uint32_t w0 = S.word(p), w1 = S.word(p + 1), w2 = S.word(p + 2);
-        const int nc = (j + lane() < n) ? ncand[j + lane()] : 0;
-        const uint64_t u0 = ((uint64_t)(w0 >> 5) << 26) | (uint64_t)(w1 >> 6);
-        const uint64_t u1 = ((uint64_t)(w1 >> 5) << 26) | (uint64_t)(w2 >> 6);
-        const unsigned long long P0 = never ? 0ull : ballot(u0 <= thr), P1 = never ? 0ull : ballot(u1 <= thr);
-        const uint32_t low = (w0 & 0xffu) | (w1 & 0xffu) << 8 | (w2 & 0xffu) << 16;
-        // each cell's candidate draw: mask << 16 | largest value; negative
-        // where it draws nothing (-1: one candidate, -2: none)
-        const int rule = nc > 1 ? (int)(smear((uint32_t)nc - 1u) << 16) | (nc - 1) : nc == 1 ? -1 : -2;
-        // the window's pairs collect in one register (lane k: its k-th pair)
-        uint32_t wp = 0;
-        int npair = 0, x = 0, drift = 0, c = 0, ru = 0;
-        bool slow = false;   // cell c's candidate draw runs past the window, at word x
-        while (x < 2 * W) {
-            // swaps whose draw takes one or two words inside the window, one
-            // straight line of scalar instructions each
-            unsigned long long bits;
-            for (;;) {
-                bits = ((x & 1) ? P1 : P0) >> (x >> 1);
-                const int xs = x + 2 * first_lane(bits), xd = xs + 2;
+// The room's pairs from the stream; returns their count. The walk is at word
+// x of a window; the record there holds the distance to the next swapping
+// cell and the first words of its candidate draw (low bytes: a cell has at
+// most 255 candidates). drift: what x is ahead of two words a cell from the
+// window's first cell. The walk is a chain of scalar instructions at about
+// five cycles each, so the common swap (a draw that ends in the window after
+// one or two words) is as few of them as possible.
+template <bool LDS>
+__device__ void room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n, int& m, int& j) {
+    // the window's first word, its place in the ring, its number, the walk's
+    // word in it, and what that is ahead of two words a cell from cell j
+    int win = S.pos / kWin, x0 = win * kWin, ring = x0 % kRingWords;
+    int x = S.pos - x0, drift = x;
+    for (;;) {
+        S.need_window(win, x0);
+        const uint2 rec = *reinterpret_cast<const uint2*>(S.w.rec + ring + 2 * min(lane(), kWin / 2 - 1));
+        const int nc = ncand[min(j + lane(), n - 1)];
+        // each cell's candidate draw: mask << 16 | largest value; where it
+        // draws nothing a value no byte is below (one candidate: -1, none, or
+        // past the room: -2)
+        const int rule = j + lane() >= n || nc == 0 ? 0xfffe
+                         : nc > 1 ? (int)(smear((uint32_t)nc - 1u) << 16) | (nc - 1) : 0xffff;
+        while (x < kWin) {
+            uint32_t rc;
+            int xs, c, ru, at;
+            do {
+                uint32_t ra = lane_u32(rec.x, x >> 1), rb = lane_u32(rec.y, x >> 1);
+                asm volatile("" : "+s"(ra), "+s"(rb));   // (both read: a select, not a branch)
+                rc = (x & 1) ? rb : ra;
+                xs = x + (int)(rc & 0xffu);
                 c = (xs - drift) >> 1;
                 ru = (int)lane_u32((uint32_t)rule, c & 63);
-                const uint32_t t = lane_u32(low, (xd >> 1) & 63) >> (8 * (xd & 1));
-                const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
-                const uint32_t v1 = t & mask, v2 = (t >> 8) & mask;
-                const uint32_t v = v1 <= mx ? v1 : v2;
-                const int xn = xd + (v1 <= mx ? 1 : 2);
-                if (!((int)(bits != 0ull) & (int)(ru >= 0) & (int)(v <= mx) & (int)(xn < 2 * W))) break;
-                wp = lane() == npair ? (uint32_t)(j + c) | (v << 16) : wp;
-                npair++;
-                x = xn;
-                drift = x - 2 * (c + 1);
+                const int mask = ru >> 16, mx = (int)(int16_t)ru;
+                const int v1 = (int)(rc >> 8) & mask, v2 = (int)(rc >> 16) & mask;
+                const int v = v1 <= mx ? v1 : v2;
+                at = v1 <= mx ? xs + 3 : xs + 4;
+                at = v <= mx ? at : kWin;
+                // (stored whether or not it is a swap: the next one overwrites it)
+                if (LDS) R.pr[m] = (uint32_t)(j + c) | ((uint32_t)v << 16);
+                else R.set_pair(m, (uint32_t)(j + c) | ((uint32_t)v << 16));
+                const bool ok = at < kWin;
+                m += ok ? 1 : 0;
+                drift = ok ? at - 2 * (c + 1) : drift;
+                x = ok ? at : x;
+            } while (at < kWin);
+            // any other swap, or none in the rest of the window
+            if ((rc & 0xffu) == kNone) break;
+            x = xs + 2;
+            const int mask = ru >> 16, mx = (int)(int16_t)ru;
+            if (mx == -2) continue;
+            int v = 0;
+            while (mx >= 0) {
+                S.need_window((x0 + x) / kWin, x0 + x);
+                v = __builtin_amdgcn_readfirstlane((int)S.w.low[(x0 + x) % kRingWords]) & mask;
+                x++;
+                if (v <= mx) break;
             }
-            // any other swap
-            if (bits == 0ull) break;
-            x += 2 * first_lane(bits) + 2;
-            if (ru == -2) continue;
-            uint32_t v = 0;
-            if (ru >= 0) {
-                const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
-                do {
-                    slow = x >= 2 * W;
-                    if (slow) break;
-                    v = (lane_u32(low, x >> 1) >> (8 * (x & 1))) & mask;
-                    x++;
-                } while (v > mx);
-                if (slow) break;
-            }
-            wp = lane() == npair ? (uint32_t)(j + c) | (v << 16) : wp;
-            npair++;
+            if (LDS) R.pr[m] = (uint32_t)(j + c) | ((uint32_t)v << 16);
+            else R.set_pair(m, (uint32_t)(j + c) | ((uint32_t)v << 16));
+            m++;
             drift = x - 2 * (c + 1);
         }
-        if (m + W <= R.cap) {
-            if (lane() < npair) R.pr[m + lane()] = wp;
-        } else if (lane() < npair) {
-            R.set_pair(m + lane(), wp);
+        // the cells up to the window's end; the room may end before (the cells
+        // past it draw nothing), or the pairs may be about to outgrow the slot
+        const int xe = max(x, kWin + (x & 1)), ce = (xe - drift) >> 1;
+        if (ce >= n - j || (LDS && m + kWin / 2 >= R.cap)) {
+            const int cells = min(ce, n - j);
+            S.pos = x0 + 2 * cells + drift;
+            j += cells;
+            return;
         }
-        m += npair;
-        if (slow) {
-            S.pos += x;
-            j += c;
-            const uint32_t mask = (uint32_t)ru >> 16, mx = (uint32_t)ru & 0xffffu;
-            uint32_t pick = 0;
-            for (;;) {
-                S.ensure(W - 1);
-                const uint32_t y = S.word(S.pos + lane()) & mask;
-                const unsigned long long okm = ballot(y <= mx);
-                if (okm) {
-                    const int gl = first_lane(okm);
-                    pick = lane_u32(y, gl);
-                    S.pos += gl + 1;
-                    break;
-                }
-                S.pos += W;
-            }
-            if (lane() == 0) R.set_pair(m, (uint32_t)j | (pick << 16));
-            m++;
-            j += 1;
-            continue;
-        }
-        // the cells up to the window's end, or to the room's: those past it draw nothing
-        const int ce = min((max(x, 2 * W + (x & 1)) - drift) >> 1, n - j);
-        S.pos += 2 * ce + drift;
         j += ce;
+        x = xe;
+        do {   // (a candidate draw may run past a whole window)
+            x -= kWin;
+            x0 += kWin;
+            win++;
+            ring = ring + kWin == kRingWords ? 0 : ring + kWin;
+        } while (x >= kWin);
+        drift = x;
     }
+}
+
+// Every pair of the room: in the slot's LDS, then in HBM should they outgrow it.
+__device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n) {
+    int m = 0, j = 0;
+    while (j < n && m + kWin / 2 < R.cap) room_pairs<true>(S, R, ncand, n, m, j);
+    if (j < n) room_pairs<false>(S, R, ncand, n, m, j);
     return m;
 }
 
@@ -1122,7 +1169,7 @@ __device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, in
 // A window ends where the draws' mask changes.
 __device__ void room_draws(Stream& S, const RoomSlot& R, int m) {
     for (int tt = m - 1; tt > 0;) {
-        S.ensure(W - 1);
+        S.need(W - 1);
         const int mask = (int)smear((uint32_t)tt), low = (mask >> 1) + 1;
         const int v = (int)(S.word(S.pos + lane()) & (uint32_t)mask);
         unsigned long long acc = ballot(v <= tt);
@@ -1179,13 +1226,14 @@ __device__ void room_shuffle(const RoomSlot& R, int m) {
 
 }  // namespace
 
-__global__ __launch_bounds__(W * (1 + kConvAppliers)) void fe_conv_plan_kernel(Args a) {
+__global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(Args a) {
     const int s = (int)blockIdx.x;
     if (s >= a.G) return;
     const Tabs& t = a.t;
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ int flag[kConvAppliers], total;   // flag: the slot's pairs + 0, or -1 where it is free
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W)), na = (int)(blockDim.x / W) - 1;
+    // flag: the slot's pairs, or -1 where it is free
+    __shared__ int flag[kConvAppliers], total, ready, used;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W)), na = (int)(blockDim.x / W) - 2;
     const ConvLds L = conv_lds(t.cv_max_room, a.cv_lds_pairs);
     auto slot = [&](int i) {
         unsigned char* b = lds + L.base + (size_t)i * L.slot;
@@ -1193,55 +1241,58 @@ __global__ __launch_bounds__(W * (1 + kConvAppliers)) void fe_conv_plan_kernel(A
         return RoomSlot{reinterpret_cast<uint32_t*>(b), reinterpret_cast<uint16_t*>(b + L.jd),
                         reinterpret_cast<uint16_t*>(b + L.q), sp, sp + t.cv_max_room, a.cv_lds_pairs};
     };
+    Words w;
+    w.raw = reinterpret_cast<uint32_t*>(lds);
+    w.rec = w.raw + kRingWords;
+    w.low = reinterpret_cast<uint8_t*>(w.rec + kRingWords);
+    uint8_t* nbuf = w.low + kRingWords + kRingPad + 8;   // [cv_max_room + 32]
+    w.ready = &ready;
+    w.used = &used;
+    unsigned char* g = a.state + (size_t)s * a.st.record;
+    uint32_t* gmt = reinterpret_cast<uint32_t*>(g + a.st.cmt);
+    int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
+    for (int i = (int)threadIdx.x; i < SBE_MT_N; i += (int)blockDim.x) w.raw[i] = gmt[i];
     if (threadIdx.x < kConvAppliers) flag[threadIdx.x] = -1;
-    if (threadIdx.x == 0) total = 0;
+    if (threadIdx.x == 0) total = ready = used = 0;
     __syncthreads();
     if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);   // the field step's wavefronts share the SIMD
         Stream S;
-        S.raw = reinterpret_cast<uint32_t*>(lds);
-        S.tw = S.raw + 2 * SBE_MT_N;
-        uint8_t* nbuf = reinterpret_cast<uint8_t*>(S.tw + 2 * SBE_MT_N);   // [cv_max_room + 32]
-        unsigned char* g = a.state + (size_t)s * a.st.record;
-        uint32_t* gmt = reinterpret_cast<uint32_t*>(g + a.st.cmt);
-        int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
-        for (int i = lane(); i < SBE_MT_N; i += W) {
-            const uint32_t w = gmt[i];
-            S.raw[i] = w;
-            S.tw[i] = mt_temper(w);
-        }
+        S.w = w;
         S.pos = __builtin_amdgcn_readfirstlane(*gidx);
-        S.cur = 0;
-        S.have_next = false;
-        wsync();
-        const uint64_t thr = ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo;
-        const bool never = t.cv_thr_hi == 0xFFFFFFFFu;
+        S.ready = 0;
+        S.used = 0;
         for (int rm = 0; rm < t.cv_rooms; rm++) {
             const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
-            // the room's candidate counts, 16 cells a lane (the section is
-            // padded and 256-byte aligned, so whole 16-byte words are its own)
+            // the room's candidate counts, 16 cells a lane (whole 16-byte words:
+            // the section starts 256-byte aligned and others follow it)
             const int skew = b0 & 15;
             const uint4* src = reinterpret_cast<const uint4*>(t.cv_ncand + (b0 - skew));
             for (int i = lane(); 16 * i < n + skew; i += W) reinterpret_cast<uint4*>(nbuf)[i] = src[i];
             wsync();
             const RoomSlot R = slot(rm % na);
             slot_wait(&flag[rm % na], false);
-            const int m = room_pairs(S, R, nbuf + skew, n, thr, never);
+            const int m = room_pairs(S, R, nbuf + skew, n);
             room_draws(S, R, m);
-            slot_post(&flag[rm % na], m);
+            post(&flag[rm % na], m);
             wsync();
         }
         // the stream state: the block holding the last word consumed
-        const int blkx = S.pos > SBE_MT_N ? (S.cur ^ 1) : S.cur;
-        for (int i = lane(); i < SBE_MT_N; i += W) gmt[i] = S.raw[blkx * SBE_MT_N + i];
-        if (lane() == 0) *gidx = S.pos > SBE_MT_N ? S.pos - SBE_MT_N : S.pos;
+        const int u = S.pos > 0 ? (S.pos - 1) / SBE_MT_N : 0;
+        for (int i = lane(); i < SBE_MT_N; i += W) gmt[i] = w.raw[(u % kRing) * SBE_MT_N + i];
+        if (lane() == 0) *gidx = S.pos - u * SBE_MT_N;
+        wsync();
+        post(&used, -1);
+    } else if (wave == 1) {
+        produce(w, ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo, t.cv_thr_hi == 0xFFFFFFFFu);
     } else {
-        const RoomSlot R = slot(wave - 1);
+        const RoomSlot R = slot(wave - 2);
         unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
-        for (int rm = wave - 1; rm < t.cv_rooms; rm += na) {
+        for (int rm = wave - 2; rm < t.cv_rooms; rm += na) {
             const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
             for (int i = 2 * lane(); i < n; i += 2 * W)
                 reinterpret_cast<uint32_t*>(R.qinv)[i >> 1] = (uint32_t)i | ((uint32_t)(i + 1) << 16);
-            const int m = slot_wait(&flag[wave - 1], true);
+            const int m = slot_wait(&flag[wave - 2], true);
             // each pair's candidate as a room-local cell
             for (int i = lane(); i < m; i += W) {
                 const uint32_t x = R.pair(i);
@@ -1252,7 +1303,7 @@ __global__ __launch_bounds__(W * (1 + kConvAppliers)) void fe_conv_plan_kernel(A
             wsync();
             if (m <= R.cap) room_shuffle<true>(R, m);
             else room_shuffle<false>(R, m);
-            slot_post(&flag[wave - 1], -1);
+            post(&flag[wave - 2], -1);
             // moves: cell i's value goes to cell q[i] (convection-cell indices;
             // the move kernels map them to field cells), in any order: each
             // reads and writes cells of its own
@@ -1361,7 +1412,7 @@ extern "C" int sbe_launch(const sbe::Args* a, int which, hipStream_t s) {
     case 3: hipLaunchKernelGGL(fe_live_kernel, dim3(1), dim3(64), 0, s, *a); break;
     case 4: {
         const ConvLds L = conv_lds(a->t.cv_max_room, a->cv_lds_pairs);
-        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64 * (1 + a->cv_appliers)),
+        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64 * (2 + a->cv_appliers)),
                            L.base + (size_t)a->cv_appliers * L.slot, s, *a);
         break;
     }

@@ -204,18 +204,22 @@ def test_draws_by_fixed_point_equal_sequential_draws():
         assert got == want and gpos == pos, m
 
 
+CHUNK = 96
+
+
 def walk_pairs(words: list, pos: int, ncand, thr: int):
-    """The plan kernel's walk over a window of 128 words: the next swapping
-    cell as the next swap bit of the walk's parity."""
+    """The plan kernel's walk: windows are the stream's chunks of 96 words,
+    entered at any word; the next swapping cell is the next swap bit of the
+    walk's parity (a cell's swap draw is words x and x + 1)."""
     n, pairs, j = len(ncand), [], 0
     while j < n:
-        w = words[pos:pos + 2 * W + 1]
-        swap = [(((w[i] >> 5) << 26) | (w[i + 1] >> 6)) <= thr for i in range(2 * W)]
+        x0 = pos // CHUNK * CHUNK
+        w = words[x0:]
+        swap = [(((w[i] >> 5) << 26) | (w[i + 1] >> 6)) <= thr for i in range(CHUNK)]
         nc = [int(ncand[j + i]) if j + i < n else 0 for i in range(W)]
-        x = drift = c = 0
-        slow, found = False, []
-        while x < 2 * W:
-            nxt = [q for q in range(x, 2 * W, 2) if swap[q]]
+        x = drift = pos - x0
+        while x < CHUNK:
+            nxt = [q for q in range(x, CHUNK, 2) if swap[q]]
             if not nxt:
                 break
             c = (nxt[0] - drift) >> 1
@@ -223,29 +227,15 @@ def walk_pairs(words: list, pos: int, ncand, thr: int):
             v = 0
             if nc[c] == 0:
                 continue
-            if nc[c] > 1:
-                while True:
-                    slow = x >= 2 * W
-                    if slow:
-                        break
-                    v = (w[x] & 0xFF) & smear(nc[c] - 1)
-                    x += 1
-                    if v <= nc[c] - 1:
-                        break
-                if slow:
+            while nc[c] > 1:
+                v = (w[x] & 0xFF) & smear(nc[c] - 1)
+                x += 1
+                if v <= nc[c] - 1:
                     break
-            found.append((j + c, v))
+            pairs.append((j + c, v))
             drift = x - 2 * (c + 1)
-        pairs += found
-        if slow:
-            pos += x
-            j += c
-            pick, pos = interval(words, pos, nc[c] - 1)
-            pairs.append((j, pick))
-            j += 1
-            continue
-        ce = min((max(x, 2 * W + (x & 1)) - drift) >> 1, n - j)
-        pos += 2 * ce + drift
+        ce = min((max(x, CHUNK + (x & 1)) - drift) >> 1, n - j)
+        pos = x0 + 2 * ce + drift
         j += ce
     return pairs, pos
 
@@ -262,5 +252,5 @@ def test_walk_equals_sequential_draws():
         if trial % 3 == 0:
             ncand[:] = rng.choice([1, 2, 24, 129, 255])
         words = [int(x) for x in rng.integers(0, 2 ** 32, size=7 * n + 1000, dtype=np.uint64)]
-        start = int(rng.integers(0, 50))
+        start = int(rng.integers(0, 700))
         assert walk_pairs(words, start, ncand, thr) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
