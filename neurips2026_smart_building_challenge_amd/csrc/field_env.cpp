@@ -66,7 +66,7 @@ struct FieldScen {
     int* d_count = nullptr;
     double* d_vals = nullptr;
     unsigned int* d_spill = nullptr;
-    int lds_pairs = 0, appliers = 1;   // of the convection plan kernel
+    int lds_pairs = 0, nc_lds = 1;   // of the convection plan kernel
     double conv_p = 0.0;
     // the plan kernel runs on its own stream, forked from the bound stream at
     // the start of a step and joined before the moves (it reads no field)
@@ -555,7 +555,7 @@ sbe::Args base_args(const FieldScen* f) {
     a.cv_vals = f->d_vals;
     a.cv_spill = f->d_spill;
     a.cv_lds_pairs = f->lds_pairs;
-    a.cv_appliers = f->appliers;
+    a.cv_nc_lds = f->nc_lds;
     a.exact = f->exact;
     return a;
 }
@@ -609,29 +609,22 @@ bool field_attach(FieldScen* f, const std::string& path, const std::vector<sbe::
     int lds = f->lds_bytes;
     if (f->t.cv_rooms > 0) {
         // pairs in LDS for 1.5 times the expected count of the largest room,
-        // at least 512 (the rest go to HBM), and as many appliers (the
-        // wavefronts that shuffle and compose rooms beside the stream's) as
-        // leave half of a compute unit's LDS to the field's workgroups
+        // at least 512 (the rest go to HBM)
         const int mr_lds = f->t.cv_max_room;
         const double expect = 1.5 * std::min(std::max(f->conv_p, 0.0), 1.0) * mr_lds;
         f->lds_pairs = std::max(512, (int)expect);
-        auto need = [&](int pairs, int n) {
-            const sbe::ConvLds L = sbe::conv_lds(mr_lds, pairs);
-            return L.base + n * L.slot;
-        };
         const size_t all = 160 * 1024 - 64;   // (a few words are the kernel's own)
         if (4 * 4 * SBE_MT_N + 3 * mr_lds + 16 > 154 * 1024)
             return (*err = "a convection room is too large for the plan kernel's LDS"), false;
-        while (need(f->lds_pairs, 1) > all) f->lds_pairs = std::max(512, f->lds_pairs * 3 / 4);
-        f->appliers = 1;
-        while (f->appliers < sbe::kConvAppliers && need(f->lds_pairs, f->appliers + 1) <= 80 * 1024) f->appliers++;
-        lds = std::max(lds, (int)need(f->lds_pairs, f->appliers));
+        f->nc_lds = sbe::conv_lds(mr_lds, 512, 1).bytes <= all;   // (rooms of up to some 45,000 cells)
+        while (sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes > all) f->lds_pairs -= 64;
+        lds = std::max(lds, (int)sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes);
         const size_t cells = (size_t)std::max(f->t.cv_cells, 1), mr = (size_t)std::max(f->t.cv_max_room, 1);
         if (!hip_ok(hipMalloc(&f->d_moves, 8 * cells * G), "hipMalloc(convection moves)", err)
             || !hip_ok(hipMalloc(&f->d_vals, 8 * cells * G), "hipMalloc(convection values)", err)
             || !hip_ok(hipMalloc(&f->d_count, 4 * (size_t)G), "hipMalloc", err)
             || !hip_ok(hipMemset(f->d_count, 0, 4 * (size_t)G), "clear", err)
-            || !hip_ok(hipMalloc(&f->d_spill, 8 * mr * f->appliers * G), "hipMalloc(convection pairs)", err)
+            || !hip_ok(hipMalloc(&f->d_spill, 2 * 8 * mr * G), "hipMalloc(convection pairs)", err)
             || !hip_ok(hipStreamCreateWithFlags(&f->side, hipStreamNonBlocking), "convection stream", err)
             || !hip_ok(hipEventCreateWithFlags(&f->fork, hipEventDisableTiming), "event", err)
             || !hip_ok(hipEventCreateWithFlags(&f->join, hipEventDisableTiming), "event", err))

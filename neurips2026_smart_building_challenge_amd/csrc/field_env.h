@@ -187,17 +187,18 @@ struct Slot {
 enum { FE_STEP = 0, FE_RESET = 1 };
 
 // The convection plan kernel's LDS for rooms of up to `room` cells: four MT
-// blocks, a record and the low byte of each of their words, the room's
-// candidate counts (with up to 15 cells before and after it), then per applier `pairs` pairs
-// (u32) and shuffle draws (u16) and the room's inverse permutation (u16).
+// blocks, a record and the low byte of each of their words, with nc_lds the
+// room's candidate counts (and up to 15 cells before and after it; else they
+// are read from HBM), the inverse permutation of the room being applied (u16),
+// then two slots of `pairs` pairs (u32) and shuffle draws (u16).
 struct ConvLds {
-    size_t base, slot, jd, q;
+    size_t q, slot0, slot, jd, bytes;
 };
-constexpr int kConvAppliers = 2;
-constexpr ConvLds conv_lds(int room, int pairs) {
-    const size_t jd = 4 * (size_t)pairs, q = (jd + 2 * (size_t)pairs + 3) & ~(size_t)3;
-    return ConvLds{(36 * (size_t)SBE_MT_N + 16 + (size_t)room + 47) & ~(size_t)15,
-                   (q + 2 * ((size_t)room + 1) + 15) & ~(size_t)15, jd, q};
+constexpr ConvLds conv_lds(int room, int pairs, int nc_lds) {
+    const size_t q = (36 * (size_t)SBE_MT_N + 16 + (nc_lds ? (size_t)room + 47 : 15)) & ~(size_t)15;
+    const size_t slot0 = (q + 2 * ((size_t)room + 1) + 15) & ~(size_t)15;
+    const size_t slot = (6 * (size_t)pairs + 15) & ~(size_t)15;
+    return ConvLds{q, slot0, slot, 4 * (size_t)pairs, slot0 + 2 * slot};
 }
 
 struct Args {
@@ -236,9 +237,9 @@ struct Args {
     unsigned long long* cv_moves; // [G][cv_cells]
     int* cv_count;                // [G]
     double* cv_vals;              // [G][cv_cells]
-    unsigned int* cv_spill;       // [G][cv_appliers][2][cv_max_room]: pairs, then shuffle draws, past the LDS
-    int cv_lds_pairs;             // pairs the plan kernel keeps in LDS per applier
-    int cv_appliers;              // its wavefronts that take rooms from the stream's
+    unsigned int* cv_spill;       // [G][2][2][cv_max_room]: per slot pairs, then shuffle draws, past the LDS
+    int cv_lds_pairs;             // pairs the plan kernel keeps in LDS per slot
+    int cv_nc_lds;                // it keeps a room's candidate counts in LDS
     int exact;                    // the field group runs in exact mode (SBX_FDM_EXACT): sums in the reference's order
 };
 

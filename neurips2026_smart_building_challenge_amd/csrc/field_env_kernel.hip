@@ -933,13 +933,18 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 // serial chain over the rooms: the cells' swaps and candidates, then the
 // shuffle's draws. The second (the producer) runs up to three MT blocks ahead
 // of it: the words and, for every word position, where the next swap would be
-// and its draw's first bytes, none of which depends on the walk. The others (appliers) each take every
-// n-th room once its draws are posted: the candidates' cells, the shuffle and
-// its composition, the moves. What bounds it is the walk's chain of scalar
-// instructions, one swap after another. At 256 envs of the 205K-cell building
+// and its draw's first bytes, none of which depends on the walk. The third
+// (the applier) takes the rooms once their draws are posted, through two
+// slots: the candidates' cells, the shuffle and its composition, the moves.
+// What bounds it is the walk's chain of scalar instructions, one swap after
+// another. At 256 envs of the 205K-cell building
 // (about 14,500 swaps a step): 10.4 ms with everything on one wavefront, 4.0 ms
-// with the rooms applied beside the stream, 3.5 ms with the producer (the
-// walk's windows had cost as much as its swaps).
+// with the rooms applied beside the stream, 3.8 ms with the producer (the
+// walk's windows had cost as much as its swaps) and one applier. One applier
+// keeps up with the walk, and its LDS is what the field step running beside
+// the plan is left with: at 512 envs (two workgroups per CU) four appliers on
+// 64 KB each held the wide up heights at 531 us, one on 51 KB leaves them
+// 103 us, and the env step went from 13.3 to 9.7 ms.
 namespace {
 
 constexpr int kWin = 96;             // words of a walk window
@@ -1226,20 +1231,20 @@ __device__ void room_shuffle(const RoomSlot& R, int m) {
 
 }  // namespace
 
-__global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(Args a) {
+__global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
     const int s = (int)blockIdx.x;
     if (s >= a.G) return;
     const Tabs& t = a.t;
     extern __shared__ __align__(16) unsigned char lds[];
     // flag: the slot's pairs, or -1 where it is free
-    __shared__ int flag[kConvAppliers], total, ready, used;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W)), na = (int)(blockDim.x / W) - 2;
-    const ConvLds L = conv_lds(t.cv_max_room, a.cv_lds_pairs);
+    __shared__ int flag[2], total, ready, used;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W));
+    const ConvLds L = conv_lds(t.cv_max_room, a.cv_lds_pairs, a.cv_nc_lds);
     auto slot = [&](int i) {
-        unsigned char* b = lds + L.base + (size_t)i * L.slot;
-        unsigned int* sp = a.cv_spill + ((size_t)s * na + i) * 2 * t.cv_max_room;
+        unsigned char* b = lds + L.slot0 + (size_t)i * L.slot;
+        unsigned int* sp = a.cv_spill + ((size_t)s * 2 + i) * 2 * t.cv_max_room;
         return RoomSlot{reinterpret_cast<uint32_t*>(b), reinterpret_cast<uint16_t*>(b + L.jd),
-                        reinterpret_cast<uint16_t*>(b + L.q), sp, sp + t.cv_max_room, a.cv_lds_pairs};
+                        reinterpret_cast<uint16_t*>(lds + L.q), sp, sp + t.cv_max_room, a.cv_lds_pairs};
     };
     Words w;
     w.raw = reinterpret_cast<uint32_t*>(lds);
@@ -1252,7 +1257,7 @@ __global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(A
     uint32_t* gmt = reinterpret_cast<uint32_t*>(g + a.st.cmt);
     int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
     for (int i = (int)threadIdx.x; i < SBE_MT_N; i += (int)blockDim.x) w.raw[i] = gmt[i];
-    if (threadIdx.x < kConvAppliers) flag[threadIdx.x] = -1;
+    if (threadIdx.x < 2) flag[threadIdx.x] = -1;
     if (threadIdx.x == 0) total = ready = used = 0;
     __syncthreads();
     if (wave == 0) {
@@ -1264,17 +1269,19 @@ __global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(A
         S.used = 0;
         for (int rm = 0; rm < t.cv_rooms; rm++) {
             const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
-            // the room's candidate counts, 16 cells a lane (whole 16-byte words:
-            // the section starts 256-byte aligned and others follow it)
             const int skew = b0 & 15;
-            const uint4* src = reinterpret_cast<const uint4*>(t.cv_ncand + (b0 - skew));
-            for (int i = lane(); 16 * i < n + skew; i += W) reinterpret_cast<uint4*>(nbuf)[i] = src[i];
-            wsync();
-            const RoomSlot R = slot(rm % na);
-            slot_wait(&flag[rm % na], false);
-            const int m = room_pairs(S, R, nbuf + skew, n);
+            if (a.cv_nc_lds) {
+                // the room's candidate counts, 16 cells a lane (whole 16-byte
+                // words: the section starts 256-byte aligned and others follow it)
+                const uint4* src = reinterpret_cast<const uint4*>(t.cv_ncand + (b0 - skew));
+                for (int i = lane(); 16 * i < n + skew; i += W) reinterpret_cast<uint4*>(nbuf)[i] = src[i];
+                wsync();
+            }
+            const RoomSlot R = slot(rm & 1);
+            slot_wait(&flag[rm & 1], false);
+            const int m = a.cv_nc_lds ? room_pairs(S, R, nbuf + skew, n) : room_pairs(S, R, t.cv_ncand + b0, n);
             room_draws(S, R, m);
-            post(&flag[rm % na], m);
+            post(&flag[rm & 1], m);
             wsync();
         }
         // the stream state: the block holding the last word consumed
@@ -1286,13 +1293,13 @@ __global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(A
     } else if (wave == 1) {
         produce(w, ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo, t.cv_thr_hi == 0xFFFFFFFFu);
     } else {
-        const RoomSlot R = slot(wave - 2);
         unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
-        for (int rm = wave - 2; rm < t.cv_rooms; rm += na) {
+        for (int rm = 0; rm < t.cv_rooms; rm++) {
+            const RoomSlot R = slot(rm & 1);
             const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
             for (int i = 2 * lane(); i < n; i += 2 * W)
                 reinterpret_cast<uint32_t*>(R.qinv)[i >> 1] = (uint32_t)i | ((uint32_t)(i + 1) << 16);
-            const int m = slot_wait(&flag[wave - 2], true);
+            const int m = slot_wait(&flag[rm & 1], true);
             // each pair's candidate as a room-local cell
             for (int i = lane(); i < m; i += W) {
                 const uint32_t x = R.pair(i);
@@ -1303,7 +1310,7 @@ __global__ __launch_bounds__(W * (2 + kConvAppliers)) void fe_conv_plan_kernel(A
             wsync();
             if (m <= R.cap) room_shuffle<true>(R, m);
             else room_shuffle<false>(R, m);
-            post(&flag[wave - 2], -1);
+            post(&flag[rm & 1], -1);
             // moves: cell i's value goes to cell q[i] (convection-cell indices;
             // the move kernels map them to field cells), in any order: each
             // reads and writes cells of its own
@@ -1411,9 +1418,8 @@ extern "C" int sbe_launch(const sbe::Args* a, int which, hipStream_t s) {
     case 2: hipLaunchKernelGGL(fe_post_kernel, dim3(G), dim3(64), a->lds_bytes, s, *a); break;
     case 3: hipLaunchKernelGGL(fe_live_kernel, dim3(1), dim3(64), 0, s, *a); break;
     case 4: {
-        const ConvLds L = conv_lds(a->t.cv_max_room, a->cv_lds_pairs);
-        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64 * (2 + a->cv_appliers)),
-                           L.base + (size_t)a->cv_appliers * L.slot, s, *a);
+        const ConvLds L = conv_lds(a->t.cv_max_room, a->cv_lds_pairs, a->cv_nc_lds);
+        hipLaunchKernelGGL(fe_conv_plan_kernel, dim3(G), dim3(64 * 3), L.bytes, s, *a);
         break;
     }
     case 5: {
