@@ -280,6 +280,10 @@ bool build_plan(const Blob& b, int width, SolvePlan* out, std::string* err) {
         // for the pivot; its readers multiply by the reciprocal)
         for (int i : Lcol[r]) {
             intersect(Lrow[i], Ucol[r], r, ks);
+            // without terms and unscaled the slot already holds its value (81
+            // zones: 378 of 3,231 tasks and 4 of 120 passes; 960 envs of every
+            // scenario: 449 -> 443 us a pass of four steps)
+            if (ks.empty() && defer) continue;
             std::vector<Term> terms;
             for (int m : ks) terms.push_back({slot[key(i, m)], slot[key(m, r)], defer ? ib + m : kSlotOne});
             add_task(slot[key(i, r)], defer ? kSlotOne : ib + r, kSlotSink, std::move(terms), 0);
