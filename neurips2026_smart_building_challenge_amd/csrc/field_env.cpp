@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <map>
 #include <string>
 #include <vector>
@@ -250,6 +251,11 @@ FieldScen* field_open(const sbh::Blob& b, std::string* err) {
             cv_off.push_back(r1);
         }
         cv_coff.assign(cf, cf + cells + 1);
+        std::array<int, 65> has{};
+        for (uint8_t c : cv_ncand)
+            if (c >= 2 && c <= 64) has[c]++;
+        const auto top = std::max_element(has.begin(), has.end());
+        f.t.cv_usual = *top ? (int)(top - has.begin()) : 0;
         f.t.cv_rooms = rooms;
         f.t.cv_cells = cells;
         // csim swaps when its 53-bit draw u / 2^53 <= p (sb_convect.c:47)
@@ -616,7 +622,7 @@ bool field_attach(FieldScen* f, const std::string& path, const std::vector<sbe::
         const size_t all = 160 * 1024 - 64;   // (a few words are the kernel's own)
         if (4 * 4 * SBE_MT_N + 3 * mr_lds + 16 > 154 * 1024)
             return (*err = "a convection room is too large for the plan kernel's LDS"), false;
-        f->nc_lds = sbe::conv_lds(mr_lds, 512, 1).bytes <= all;   // (rooms of up to some 45,000 cells)
+        f->nc_lds = sbe::conv_lds(mr_lds, 512, 1).bytes <= all;   // (rooms of up to some 46,000 cells)
         while (sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes > all) f->lds_pairs -= 64;
         lds = std::max(lds, (int)sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes);
         const size_t cells = (size_t)std::max(f->t.cv_cells, 1), mr = (size_t)std::max(f->t.cv_max_room, 1);

@@ -170,6 +170,7 @@ struct Tabs {
     const uint8_t* cv_ncand;
     const int* cv_coff;
     const uint16_t* cv_cidx;
+    int cv_usual;                 // the commonest candidate count of 2..64 (0: none), the walk's fast case
 };
 
 // One env of a field group: its index in the vec, its calendar start, episode
@@ -195,7 +196,7 @@ struct ConvLds {
     size_t q, slot0, slot, jd, bytes;
 };
 constexpr ConvLds conv_lds(int room, int pairs, int nc_lds) {
-    const size_t q = (36 * (size_t)SBE_MT_N + 16 + (nc_lds ? (size_t)room + 47 : 15)) & ~(size_t)15;
+    const size_t q = (28 * (size_t)SBE_MT_N + 16 + (nc_lds ? (size_t)room + 47 : 15)) & ~(size_t)15;
     const size_t slot0 = (q + 2 * ((size_t)room + 1) + 15) & ~(size_t)15;
     const size_t slot = (6 * (size_t)pairs + 15) & ~(size_t)15;
     return ConvLds{q, slot0, slot, 4 * (size_t)pairs, slot0 + 2 * slot};
@@ -248,8 +249,8 @@ struct Args {
 static_assert(sizeof(StateLayout) == 144 && offsetof(StateLayout, cmt) == 140, "StateLayout layout");
 static_assert(sizeof(Slot) == 32, "Slot layout");
 static_assert(offsetof(Tabs, gas_co2) == 528 && offsetof(Tabs, temp_init) == 536 && offsetof(Tabs, cv_off) == 576
-              && sizeof(Tabs) == 616, "Tabs layout");
-static_assert(offsetof(Args, st) == 616 && offsetof(Args, state) == 760 && offsetof(Args, qz) == 840
-              && offsetof(Args, live) == 904 && sizeof(Args) == 968, "Args layout");
+              && sizeof(Tabs) == 624, "Tabs layout");
+static_assert(offsetof(Args, st) == 624 && offsetof(Args, state) == 768 && offsetof(Args, qz) == 848
+              && offsetof(Args, live) == 912 && sizeof(Args) == 976, "Args layout");
 
 }  // namespace sbe

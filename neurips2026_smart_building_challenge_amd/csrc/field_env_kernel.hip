@@ -933,18 +933,19 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 // serial chain over the rooms: the cells' swaps and candidates, then the
 // shuffle's draws. The second (the producer) runs up to three MT blocks ahead
 // of it: the words and, for every word position, where the next swap would be
-// and its draw's first bytes, none of which depends on the walk. The third
+// and its candidate for the commonest count, which do not depend on the walk. The third
 // (the applier) takes the rooms once their draws are posted, through two
 // slots: the candidates' cells, the shuffle and its composition, the moves.
 // What bounds it is the walk's chain of scalar instructions, one swap after
 // another. At 256 envs of the 205K-cell building
 // (about 14,500 swaps a step): 10.4 ms with everything on one wavefront, 4.0 ms
 // with the rooms applied beside the stream, 3.8 ms with the producer (the
-// walk's windows had cost as much as its swaps) and one applier. One applier
+// walk's windows had cost as much as its swaps) and one applier, 3.4 ms with
+// whole swaps in the producer's records. One applier
 // keeps up with the walk, and its LDS is what the field step running beside
 // the plan is left with: at 512 envs (two workgroups per CU) four appliers on
 // 64 KB each held the wide up heights at 531 us, one on 51 KB leaves them
-// 103 us, and the env step went from 13.3 to 9.7 ms.
+// 103 us, and two env steps went from 13.3 to 9.7 ms.
 namespace {
 
 constexpr int kWin = 96;             // words of a walk window
@@ -956,18 +957,21 @@ static_assert(kRingWords % kWin == 0 && kWin % 2 == 0 && kWin / 2 <= W, "windows
 // The stream's LDS, shared by the walk and the producer. Positions are words
 // from the step's first block, which sits at the ring's start.
 //
-// rec[p]: what the walk needs to know at word p, if a cell's draw starts there.
-// Byte 0: words to the next position of p's parity (p itself included) in p's
-// window where a cell would swap, kNone if there is none; bytes 1..3: the low
-// bytes of that position's words + 2, + 3, + 4, the candidate draw's first.
+// hop[p]: what the walk needs to know at word p, if a cell's draw starts there.
+// Bits 1..7: words + 2 to the next position of p's parity (p itself included)
+// in p's window where a cell would swap, kNoHop if there is none. Bit 0: for a
+// cell of the building's commonest candidate count the draw of the candidate
+// ends in the window, after at most three words; bits 8..9: its words, bits
+// 10..15: the candidate.
 struct Words {
     uint32_t* raw;                 // [kRingWords]
-    uint32_t* rec;                 // [kRingWords]
+    uint16_t* hop;                 // [kRingWords]
     uint8_t* low;                  // [kRingWords + kRingPad]: the tempered words' low bytes
     int* ready;                    // windows prepared
     int* used;                     // the block that holds the last word consumed; -1 once the walk is done
 };
-constexpr uint32_t kNone = 0xffu;
+constexpr uint32_t kNoHop = 0xfeu;
+__device__ __forceinline__ uint32_t smear(uint32_t x) { return x ? 0xffffffffu >> __clz((int)x) : 0u; }
 
 // A post and the wait for one: every post that a wavefront waits for is made
 // by another that never waits for it meanwhile.
@@ -985,6 +989,7 @@ struct Stream {
     int pos;       // next word to consume
     int ready;     // blocks known to be prepared
     int used;      // posted last
+    int usual;     // the commonest candidate count
 
     // window b prepared, so every word up to word q in it readable; what lies
     // before the walk's word (q or before) is given back first (the producer
@@ -1009,8 +1014,17 @@ struct Stream {
 // windows' records. A window's last swap draw reads the word after it and its
 // records bytes up to four words past it, so a window is prepared once the
 // words 8 past it are there.
-__device__ void produce(const Words& w, uint64_t thr, bool never) {
+__device__ void produce(const Words& w, uint64_t thr, bool never, int usual) {
     const int l2 = 2 * min(lane(), kWin / 2 - 1);
+    const int umax = usual - 1, umask = (int)smear((uint32_t)max(umax, 0));
+    // the hop at word x of a window, its next swap d words on with the low bytes e after it
+    auto hop = [&](int x, int d, const uint8_t* e, bool swaps) {
+        const int v1 = (int)e[0] & umask, v2 = (int)e[1] & umask, v3 = (int)e[2] & umask;
+        const int k = v1 <= umax ? 1 : v2 <= umax ? 2 : 3;
+        const int v = v1 <= umax ? v1 : v2 <= umax ? v2 : v3;
+        const bool ok = v <= umax && x + d + 2 + k < kWin;
+        return !swaps ? kNoHop : (uint32_t)(d + 2) << 1 | (ok ? 1u | (uint32_t)k << 8 | (uint32_t)v << 10 : 0u);
+    };
     int win = 0;   // next window to prepare
     for (int b = 0;; b++) {
         int u;
@@ -1035,16 +1049,12 @@ __device__ void produce(const Words& w, uint64_t thr, bool never) {
             const unsigned long long n0 = P0 >> (l2 >> 1), n1 = P1 >> (l2 >> 1);
             const int d0 = n0 ? 2 * first_lane(n0) : 0, d1 = n1 ? 2 * first_lane(n1) : 0;
             const uint8_t *c0 = w.low + p + d0 + 2, *c1 = w.low + p + 1 + d1 + 2;
-            const uint32_t e0 = (uint32_t)c0[0] << 8 | (uint32_t)c0[1] << 16 | (uint32_t)c0[2] << 24;
-            const uint32_t e1 = (uint32_t)c1[0] << 8 | (uint32_t)c1[1] << 16 | (uint32_t)c1[2] << 24;
-            if (lane() < kWin / 2)
-                *reinterpret_cast<uint2*>(w.rec + p) = make_uint2(e0 | (n0 ? (uint32_t)d0 : kNone), e1 | (n1 ? (uint32_t)d1 : kNone));
+            const uint32_t h = hop(l2, d0, c0, n0 != 0) | hop(l2 + 1, d1, c1, n1 != 0) << 16;
+            if (lane() < kWin / 2) *reinterpret_cast<uint32_t*>(w.hop + p) = h;
         }
         post(w.ready, win);
     }
 }
-
-__device__ __forceinline__ uint32_t smear(uint32_t x) { return x ? 0xffffffffu >> __clz((int)x) : 0u; }
 
 // A room's pairs and shuffle draws, from the stream wavefront to its applier:
 // in LDS up to `cap` of them, the rest in HBM. pr[i]: cell | candidate << 16
@@ -1075,76 +1085,84 @@ __device__ __forceinline__ int slot_wait(int* flag, bool full) {
     return v;
 }
 
+__device__ int writelane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 // The room's pairs from the stream; returns their count. The walk is at word
-// x of a window; the record there holds the distance to the next swapping
-// cell and the first words of its candidate draw (low bytes: a cell has at
-// most 255 candidates). drift: what x is ahead of two words a cell from the
-// window's first cell. The walk is a chain of scalar instructions at about
-// five cycles each, so the common swap (a draw that ends in the window after
-// one or two words) is as few of them as possible.
-template <bool LDS>
-__device__ void room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n, int& m, int& j) {
+// x of a window; drift is what x is ahead of two words a cell from the window's
+// first cell. The walk is a chain of scalar instructions, one wavefront's at
+// seven to ten cycles each, so a swap is as few of them as possible: a cell of
+// the commonest candidate count takes its whole swap from the record (87% of
+// the 205K-cell building's cells), and the window's pairs gather in a register,
+// one a lane, stored together. Every swap from the draw's words instead, 40
+// instructions each: 3.8 ms a plan at 256 envs, 3.4 ms so. (One hop without a
+// branch or with one instead of two took the same time.)
+__device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n) {
     // the window's first word, its place in the ring, its number, the walk's
     // word in it, and what that is ahead of two words a cell from cell j
+    int m = 0, j = 0;
+    if (n == 0) return 0;
     int win = S.pos / kWin, x0 = win * kWin, ring = x0 % kRingWords;
     int x = S.pos - x0, drift = x;
     for (;;) {
         S.need_window(win, x0);
-        const uint2 rec = *reinterpret_cast<const uint2*>(S.w.rec + ring + 2 * min(lane(), kWin / 2 - 1));
+        uint32_t hops = *reinterpret_cast<const uint32_t*>(S.w.hop + ring + 2 * min(lane(), kWin / 2 - 1));
         const int nc = ncand[min(j + lane(), n - 1)];
         // each cell's candidate draw: mask << 16 | largest value; where it
         // draws nothing a value no byte is below (one candidate: -1, none, or
         // past the room: -2)
         const int rule = j + lane() >= n || nc == 0 ? 0xfffe
                          : nc > 1 ? (int)(smear((uint32_t)nc - 1u) << 16) | (nc - 1) : 0xffff;
+        // bit c: the window's cell c (of 48 at most) has the commonest count
+        const unsigned long long usual = ballot(j + lane() < n && nc == S.usual);
+        asm volatile("" : "+v"(hops));   // (arrived: no wait among the swaps)
+        int pairs = 0, cnt = 0;          // lane i: the window's pair i, its cell from j on
+        int ahead = drift + 2;
         while (x < kWin) {
-            uint32_t rc;
-            int xs, c, ru, at;
-            do {
-                uint32_t ra = lane_u32(rec.x, x >> 1), rb = lane_u32(rec.y, x >> 1);
-                asm volatile("" : "+s"(ra), "+s"(rb));   // (both read: a select, not a branch)
-                rc = (x & 1) ? rb : ra;
-                xs = x + (int)(rc & 0xffu);
-                c = (xs - drift) >> 1;
-                ru = (int)lane_u32((uint32_t)rule, c & 63);
-                const int mask = ru >> 16, mx = (int)(int16_t)ru;
-                const int v1 = (int)(rc >> 8) & mask, v2 = (int)(rc >> 16) & mask;
-                const int v = v1 <= mx ? v1 : v2;
-                at = v1 <= mx ? xs + 3 : xs + 4;
-                at = v <= mx ? at : kWin;
-                // (stored whether or not it is a swap: the next one overwrites it)
-                if (LDS) R.pr[m] = (uint32_t)(j + c) | ((uint32_t)v << 16);
-                else R.set_pair(m, (uint32_t)(j + c) | ((uint32_t)v << 16));
-                const bool ok = at < kWin;
-                m += ok ? 1 : 0;
-                drift = ok ? at - 2 * (c + 1) : drift;
-                x = ok ? at : x;
-            } while (at < kWin);
-            // any other swap, or none in the rest of the window
-            if ((rc & 0xffu) == kNone) break;
-            x = xs + 2;
-            const int mask = ru >> 16, mx = (int)(int16_t)ru;
+            uint32_t h;
+            int xs, c;
+            for (;;) {
+                h = lane_u32(hops, x >> 1) >> (16 * x & 31);
+                xs = x + (int)((h >> 1) & 0x7fu);
+                c = (xs - ahead) >> 1;
+                if (!((uint32_t)(usual >> (c & 63)) & h & 1u)) break;
+                pairs = writelane(c | (int)((h >> 10) & 0x3fu) << 16, cnt++, pairs);
+                const int k = (int)(h >> 8) & 3;
+                ahead += k;
+                x = xs + k;
+            }
+            if ((h & kNoHop) == kNoHop) break;
+            // any other swap
+            const int ru = (int)lane_u32((uint32_t)rule, c & 63), mask = ru >> 16, mx = (int)(int16_t)ru;
+            // its draw's first bytes (the records of the window are made from them)
+            const int low = S.w.low[ring + xs + (lane() & 1)];
+            x = xs;
             if (mx == -2) continue;
             int v = 0;
-            while (mx >= 0) {
+            if (mx >= 0) {
+                v = (int)lane_u32((uint32_t)low, 0) & mask;
+                x++;
+                if (v > mx) {
+                    v = (int)lane_u32((uint32_t)low, 1) & mask;
+                    x++;
+                }
+            }
+            while (v > mx && mx >= 0) {
                 S.need_window((x0 + x) / kWin, x0 + x);
                 v = __builtin_amdgcn_readfirstlane((int)S.w.low[(x0 + x) % kRingWords]) & mask;
                 x++;
-                if (v <= mx) break;
             }
-            if (LDS) R.pr[m] = (uint32_t)(j + c) | ((uint32_t)v << 16);
-            else R.set_pair(m, (uint32_t)(j + c) | ((uint32_t)v << 16));
-            m++;
-            drift = x - 2 * (c + 1);
+            pairs = writelane(c | v << 16, cnt++, pairs);
+            ahead = x - 2 * c;
         }
+        drift = ahead - 2;
+        if (lane() < cnt) R.set_pair(m + lane(), (uint32_t)(pairs + j));
+        m += cnt;
         // the cells up to the window's end; the room may end before (the cells
-        // past it draw nothing), or the pairs may be about to outgrow the slot
+        // past it draw nothing)
         const int xe = max(x, kWin + (x & 1)), ce = (xe - drift) >> 1;
-        if (ce >= n - j || (LDS && m + kWin / 2 >= R.cap)) {
-            const int cells = min(ce, n - j);
-            S.pos = x0 + 2 * cells + drift;
-            j += cells;
-            return;
+        if (ce >= n - j) {
+            S.pos = x0 + 2 * (n - j) + drift;
+            return m;
         }
         j += ce;
         x = xe;
@@ -1156,14 +1174,6 @@ __device__ void room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, i
         } while (x >= kWin);
         drift = x;
     }
-}
-
-// Every pair of the room: in the slot's LDS, then in HBM should they outgrow it.
-__device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, int n) {
-    int m = 0, j = 0;
-    while (j < n && m + kWin / 2 < R.cap) room_pairs<true>(S, R, ncand, n, m, j);
-    if (j < n) room_pairs<false>(S, R, ncand, n, m, j);
-    return m;
 }
 
 // The shuffle's draws (draw t below t + 1, t = m - 1 .. 1, into R's draw t):
@@ -1248,8 +1258,8 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
     };
     Words w;
     w.raw = reinterpret_cast<uint32_t*>(lds);
-    w.rec = w.raw + kRingWords;
-    w.low = reinterpret_cast<uint8_t*>(w.rec + kRingWords);
+    w.hop = reinterpret_cast<uint16_t*>(w.raw + kRingWords);
+    w.low = reinterpret_cast<uint8_t*>(w.hop + kRingWords);
     uint8_t* nbuf = w.low + kRingWords + kRingPad + 8;   // [cv_max_room + 32]
     w.ready = &ready;
     w.used = &used;
@@ -1264,6 +1274,7 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
         __builtin_amdgcn_s_setprio(3);   // the field step's wavefronts share the SIMD
         Stream S;
         S.w = w;
+        S.usual = t.cv_usual;
         S.pos = __builtin_amdgcn_readfirstlane(*gidx);
         S.ready = 0;
         S.used = 0;
@@ -1291,7 +1302,7 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
         wsync();
         post(&used, -1);
     } else if (wave == 1) {
-        produce(w, ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo, t.cv_thr_hi == 0xFFFFFFFFu);
+        produce(w, ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo, t.cv_thr_hi == 0xFFFFFFFFu, t.cv_usual);
     } else {
         unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
         for (int rm = 0; rm < t.cv_rooms; rm++) {

@@ -254,3 +254,24 @@ def test_walk_equals_sequential_draws():
         words = [int(x) for x in rng.integers(0, 2 ** 32, size=7 * n + 1000, dtype=np.uint64)]
         start = int(rng.integers(0, 700))
         assert walk_pairs(words, start, ncand, thr) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
+
+
+def test_hop_records_equal_sequential_draws():
+    """A record's whole swap (csrc/field_env_kernel.hip, produce): for a cell of
+    `usual` candidates the distance to the next swap of the word's parity, the
+    draw's words (at most three, inside the window) and its candidate are those
+    of the sequential draws, at every word of a window; whole numbers, so equal."""
+    rng = np.random.default_rng(41)
+    for trial in range(60):
+        usual = int(rng.choice([2, 3, 8, 19, 24, 33, 64]))
+        thr = int(np.floor(float(rng.choice([0.0, 0.1, 0.6, 1.0])) * 2.0 ** 53))
+        w = [int(x) for x in rng.integers(0, 2 ** 32, size=CHUNK + 700, dtype=np.uint64)]
+        for x in range(CHUNK):
+            at = [q for q in range(x, CHUNK, 2) if (((w[q] >> 5) << 26) | (w[q + 1] >> 6)) <= thr]
+            vs = [(w[at[0] + 2 + i] & 0xFF) & smear(usual - 1) for i in range(3)] if at else []
+            k = next((i + 1 for i, v in enumerate(vs) if v <= usual - 1), 0)
+            whole = k > 0 and at[0] + 2 + k < CHUNK
+            pairs, end = sequential_pairs(w, x, [usual] * ((at[0] - x) // 2 + 1 if at else (CHUNK + 1 - x) // 2), thr)
+            assert len(pairs) == (1 if at else 0)
+            if whole:
+                assert pairs[0] == ((at[0] - x) // 2, vs[k - 1]) and end == at[0] + 2 + k, (trial, x)
