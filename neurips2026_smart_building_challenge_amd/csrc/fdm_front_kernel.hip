@@ -15,7 +15,7 @@
 // l / 16 + 4 q, env l % 16.
 // What bounds it: the vectors' HBM traffic at 256 envs and more, the chain of
 // 2 x 17 dependent launches at a tile or two. Measured on the 205K-cell plan:
-// a step of 256 envs 13.1 -> 2.0 ms, of 16 envs 10.2 -> 0.45 ms against level
+// a step of 256 envs 13.1 -> 1.9 ms, of 16 envs 10.2 -> 0.45 ms against level
 // by level row solves, whose 4,577 dependent levels were the whole time.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
