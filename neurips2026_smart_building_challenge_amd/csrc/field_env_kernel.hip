@@ -948,7 +948,11 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 // 103 us, and two env steps went from 13.3 to 9.7 ms.
 namespace {
 
-constexpr int kWin = 96;             // words of a walk window
+// Words of a walk window: the most that tile the ring and fit a record's seven
+// bits and two words a lane. A window costs the walk as much as several swaps,
+// so the fewer the better: two env steps at 256 envs 9.7 ms with 64 words, 7.31
+// with 96, 7.09 with 104 (the small building's eight 2.71, 2.06 and 2.02).
+constexpr int kWin = 104;
 constexpr int kRing = 4;             // MT blocks in LDS
 constexpr int kRingWords = kRing * SBE_MT_N;
 constexpr int kRingPad = 8;          // the ring's first words again, so that reads past a window need no wrap
@@ -1112,7 +1116,7 @@ __device__ int room_pairs(Stream& S, const RoomSlot& R, const uint8_t* ncand, in
         // past the room: -2)
         const int rule = j + lane() >= n || nc == 0 ? 0xfffe
                          : nc > 1 ? (int)(smear((uint32_t)nc - 1u) << 16) | (nc - 1) : 0xffff;
-        // bit c: the window's cell c (of 48 at most) has the commonest count
+        // bit c: the window's cell c (of 52 at most) has the commonest count
         const unsigned long long usual = ballot(j + lane() < n && nc == S.usual);
         asm volatile("" : "+v"(hops));   // (arrived: no wait among the swaps)
         int pairs = 0, cnt = 0;          // lane i: the window's pair i, its cell from j on

@@ -204,11 +204,11 @@ def test_draws_by_fixed_point_equal_sequential_draws():
         assert got == want and gpos == pos, m
 
 
-CHUNK = 96
+CHUNK = 104
 
 
 def walk_pairs(words: list, pos: int, ncand, thr: int):
-    """The plan kernel's walk: windows are the stream's chunks of 96 words,
+    """The plan kernel's walk: windows are the stream's chunks of 104 words,
     entered at any word; the next swapping cell is the next swap bit of the
     walk's parity (a cell's swap draw is words x and x + 1)."""
     n, pairs, j = len(ncand), [], 0
