@@ -37,9 +37,10 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
 // acc[r][e] += A (row tile r) B (env tile e) over the steps [k0, k1): A from
 // the operator's tiles, B through load(step, e). U steps' loads are issued
 // before their products; the last U may run past k1 with zeros for A (a step
-// at a time there would be a memory latency each).
-template <int RT, int NE, int U, class Load>
-__device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE]) {
+// at a time there would be a memory latency each). `before(k)` runs ahead of step k's products.
+template <int RT, int NE, int U, class Load, class Before>
+__device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE],
+                                        Before before) {
     for (int k = k0; k < k1; k += U) {
         double a[RT][U], b[NE][U];
 #pragma unroll
@@ -51,14 +52,20 @@ __device__ __forceinline__ void product(const double* const (&A)[RT], int k0, in
             for (int r = 0; r < RT; r++) a[r][u] = A[r][(size_t)q * 64];
         }
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++) {
+            if (k + u < k1) before(k + u);
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 const double x = k + u < k1 ? a[r][u] : 0.0;
 #pragma unroll
                 for (int e = 0; e < NE; e++) acc[r][e] = mfma(x, b[e][u], acc[r][e]);
             }
+        }
     }
+}
+template <int RT, int NE, int U, class Load>
+__device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE]) {
+    product<RT, NE, U>(A, k0, k1, load, acc, [](int) {});
 }
 
 // The leaves, a wavefront per (RT row tiles of a front, NE env tiles): up
@@ -147,9 +154,14 @@ __global__ __launch_bounds__(256) void assemble_kernel(sbf::FrontTab t, int task
                                                                + gathered(t, f.arow + row, Cb);
 }
 
+// Column shares of a front's product above the leaves. Every form of
+// front_kernel sums the same shares in the same order, ((0 + 1) + (2 + 3)) +
+// ..., so an env's result does not depend on the form its batch takes.
+constexpr int kShares = 8;
+
 // A height above the leaves, one workgroup per (RT row tiles of a front, NE
-// env tiles), its KW wavefronts taking an equal share of the columns each,
-// summed in LDS in wavefront order. Down: x = K [b'; x_B]. Up: c = the
+// env tiles), its KW wavefronts taking kShares / KW neighbouring shares of the
+// columns each, summed in LDS. Down: x = K [b'; x_B]. Up: c = the
 // children's contributions on B + F b', with b' from Y (assemble_kernel), or,
 // FUSED, assembled into LDS by every workgroup of the front (its first tile's
 // writes it to Y).
@@ -161,11 +173,16 @@ __global__ __launch_bounds__(256) void assemble_kernel(sbf::FrontTab t, int task
 // height (the lowest three) assembled by every workgroup took 188 us at 256
 // envs, from Y 47: there it
 // is bound by the products' operand traffic: 2 x 2 tiles.
+//
+// Four wavefronts a SIMD: left alone, the compiler takes registers for three
+// (the same two env steps 9.74 ms).
 template <bool DOWN, bool FUSED, int RT, int NE, int KW, int U>
-__global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+__global__ __launch_bounds__(64 * KW, 4) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
                                                         const double* __restrict__ W, double* __restrict__ Y,
                                                         double* C, double* X) {
-    static_assert(!FUSED || (RT == 1 && NE == 1), "the fused form takes single tiles");
+    static_assert(!FUSED || (RT == 1 && NE == 1 && KW == kShares), "the fused form takes single tiles and shares");
+    static_assert(KW == kShares || 2 * KW == kShares, "a wavefront takes one share or a pair");
+    constexpr int SH = kShares / KW;
     extern __shared__ double lds[];
     const int neg = (nt + NE - 1) / NE;
     const int eg = (int)(blockIdx.x % (unsigned)neg), task = (int)(blockIdx.x / (unsigned)neg) * RT;
@@ -192,9 +209,13 @@ __global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int tas
             Xb[e] = X + te * n * E + j;
         }
         d4 acc[RT][NE] = {};
+        // partial sums: [wavefront][row tile][env tile][register][lane]
+        double* red = lds;
+        auto slot = [&](int w, int r, int e, int q) { return (((w * RT + r) * NE + e) * 4 + q) * 64 + lane; };
         const int rows = DOWN ? f.w : f.r;
         // the shares cut where the columns are (none for a front without rows)
-        const int q0 = rows > 0 ? ks * wave / KW : 0, q1 = rows > 0 ? ks * (wave + 1) / KW : 0;
+        auto cut = [&](int share) { return rows > 0 ? ks * share / kShares : 0; };
+        const int mid = cut(wave * SH + 1);   // the second share of a pair
         // the output's own gathered part, final before this height (up)
         double own[RT][NE] = {};
         if (!DOWN && wave < 4) {
@@ -216,6 +237,7 @@ __global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int tas
             double* Yw = Y + ((size_t)eg * ny + (f.off - t.n_leaf)) * E + col;
             // this wavefront's share of F, loaded meanwhile (a share has at most kFrontCols / 4 / KW steps)
             constexpr int AU = (sbf::kFrontCols / 4 + KW - 1) / KW;
+            const int q0 = cut(wave), q1 = cut(wave + 1);
             double a[AU];
 #pragma unroll
             for (int k = 0; k < AU; k++) a[k] = A[0][(size_t)min(q0 + k, max(q1 - 1, 0)) * 64 * (rows > 0 ? 1 : 0)];
@@ -253,22 +275,44 @@ __global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int tas
                 if (q0 + k < q1) acc[0][0] = mfma(a[k], lds[(4 * (q0 + k) + kk) * E + j], acc[0][0]);
             __syncthreads();
         } else {
+            // one run over the wavefront's columns; at its second share the first
+            // one's sums go to LDS (two env steps at 512 envs of the 205K-cell
+            // building 9.36 ms; a run a share 9.55; registers for both shares 9.53)
+            const int q0 = cut(wave * SH), q1 = cut(wave * SH + SH);
+            auto keep = [&](int k) {
+                if (SH == 1 || k != mid) return;
+#pragma unroll
+                for (int r = 0; r < RT; r++)
+#pragma unroll
+                    for (int e = 0; e < NE; e++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            red[slot(wave, r, e, q)] = acc[r][e][q];
+                            acc[r][e][q] = 0.0;
+                        }
+            };
             product<RT, NE, U>(A, min(q0, kw), min(q1, kw),
-                               [&](int k, int e) { return Yb[e][min(4 * k + kk, f.w - 1) * E]; }, acc);
+                               [&](int k, int e) { return Yb[e][min(4 * k + kk, f.w - 1) * E]; }, acc, keep);
             if (DOWN) {
                 const int* br = t.brow + f.brow + kk - 4 * kw;
                 product<RT, NE, U>(A, max(q0, kw), max(q1, kw),
-                                   [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc);
+                                   [&](int k, int e) { return Xb[e][(size_t)br[4 * k] * E]; }, acc, keep);
+            }
+            if (SH == 2 && mid < q1) {
+#pragma unroll
+                for (int r = 0; r < RT; r++)
+#pragma unroll
+                    for (int e = 0; e < NE; e++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) acc[r][e][q] = red[slot(wave, r, e, q)] + acc[r][e][q];
             }
         }
-        // [wavefront][row tile][env tile][register][lane]
-        double* red = lds;
 #pragma unroll
         for (int r = 0; r < RT; r++)
 #pragma unroll
             for (int e = 0; e < NE; e++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) red[(((wave * RT + r) * NE + e) * 4 + q) * 64 + lane] = acc[r][e][q];
+                for (int q = 0; q < 4; q++) red[slot(wave, r, e, q)] = acc[r][e][q];
         __syncthreads();
         // wavefront q finishes register q of every tile
         if (wave < 4) {
@@ -282,7 +326,11 @@ __global__ __launch_bounds__(64 * KW) void front_kernel(sbf::FrontTab t, int tas
                     if ((int)te >= nt) continue;
                     double v = 0.0;
 #pragma unroll
-                    for (int w = 0; w < KW; w++) v += red[(((w * RT + r) * NE + e) * 4 + wave) * 64 + lane];
+                    for (int w = 0; w < KW; w += KW / 4) {
+                        double pair = red[slot(w, r, e, wave)];
+                        if (SH == 1) pair += red[slot(w + 1, r, e, wave)];
+                        v += pair;
+                    }
                     if (DOWN) X[(te * n + f.off + row) * E + j] = v;
                     else C[(te * (t.n_c + 1) + f.c + row) * E + j] = v + own[r][e];
                 }

@@ -245,6 +245,35 @@ def test_gpu_fdm_full_size_batch_properties(full):
     g2.close()
 
 
+def test_gpu_fdm_default_independent_of_batch(full):
+    """An env's field and interior mass are the same bit for bit whether it is
+    stepped alone or in a group of 33 or 300 (default mode, full-size plan): the
+    heights of the tree of fronts take their narrow form everywhere at 1 env,
+    their wide form at one height from 33 envs on and at several at 300, with
+    the same sums in the same order."""
+    import torch
+
+    plan, path, _ = full
+    say("full-size plan: envs alone, among 33 and among 300")
+    big, pick = 300, [0, 17, 32, 255, 299]
+    inputs = [F.step_inputs(plan, big, 61, s) for s in range(3)]
+
+    def run(envs):
+        f = gpu_group(path, len(envs), 0, exact=False)
+        for inp in inputs:
+            f.step(*device_inputs({k: (np.ascontiguousarray(v[envs]) if v.ndim else v) for k, v in inp.items()}))
+        torch.cuda.synchronize()
+        T, M = f.state()
+        f.close()
+        return T, M
+
+    T, M = run(list(range(big)))
+    for envs in [[g] for g in pick] + [pick + list(range(28))]:
+        Ts, Ms = run(envs)
+        for i, g in enumerate(envs):
+            assert np.array_equal(Ts[i], T[g]) and np.array_equal(Ms[i], M[g]), (len(envs), g)
+
+
 @pytest.mark.parametrize("G", [40, 300])
 def test_gpu_fdm_full_size_default_every_cell(full, G):
     """The default configuration (envs_per_block 0, default mode) at
