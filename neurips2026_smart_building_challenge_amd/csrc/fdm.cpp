@@ -173,8 +173,8 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     g->pw = (double*)dalloc(f, sizeof(double) * G * k);
     g->mat = fields ? (double*)dalloc(f, sizeof(double) * G * k * k) : nullptr;
     g->eact = (int*)dalloc(f, sizeof(int) * G);
-    g->bact = (int*)dalloc(f, sizeof(int) * g->nblk);
-    if (!g->W1 || !g->pw || !g->eact || !g->bact || (w2 && !g->W2) || (fields && (!g->T || !g->M || !g->mat))
+    g->bact = fronts ? nullptr : (int*)dalloc(f, sizeof(int) * g->nblk);
+    if (!g->W1 || !g->pw || !g->eact || (!fronts && !g->bact) || (w2 && !g->W2) || (fields && (!g->T || !g->M || !g->mat))
         || (fronts && (!g->X || !g->Y || !g->C)))
         return fail("hipMalloc failed for the field buffers");
     // C's zero rows (the contributions are written before they are read)

@@ -153,7 +153,7 @@ struct Group {
     double* pw;             // [G][k] air-side power, then the dense solve's result
     double* mat;            // [G][k][k] I + diag(g) S
     int* eact;              // [G] env has a nonzero air-side conductance this step
-    int* bact;              // [nblk] some env of the block has
+    int* bact;              // [nblk] some env of the block has (exact mode; null in the default one)
 };
 
 // One batched step's inputs (device): input_q [G][n_cvs], ambient / h [G],

@@ -481,8 +481,7 @@ __device__ __forceinline__ double base_of(double ambient) { return isfinite(ambi
 // Forcing (sb_fdm.c:147-151, exposure :126-140) less base x row sum: a workgroup takes 64 solved
 // cells of one env tile, computes with lanes over cells (the field, the heat
 // and the mass are read in the cells' order) and stores rows of 16 envs
-// through LDS. Lanes past the group's envs get zeros. Clears the blocks'
-// air-side flags.
+// through LDS. Lanes past the group's envs get zeros.
 __global__ __launch_bounds__(256) void front_forcing_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
     __shared__ double fs[64][E + 1];
     const int te = (int)(blockIdx.x % (unsigned)g.nt), t0 = (int)(blockIdx.x / (unsigned)g.nt) * 64;
@@ -520,8 +519,6 @@ __global__ __launch_bounds__(256) void front_forcing_kernel(sbf::Tables t, sbf::
         const int c = q * 16 + (threadIdx.x >> 4);
         if (t0 + c < n) Wt[(size_t)t.ft.rf[t0 + c] * E + (threadIdx.x & 15)] = fs[c][threadIdx.x & 15];
     }
-    const size_t x = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (x < (size_t)g.nblk) g.bact[x] = 0;
 }
 
 // Per sensed row and env tile: the sensed temperature of the solution and the

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64) void dense_kernel(sbf::Tables t, sbf::Group g, 
     any = __any(any);
     if (lane == 0) {
         g.eact[env] = any;
-        if (any) atomicOr(&g.bact[env / g.Gl], 1);
+        if (any && g.bact) atomicOr(&g.bact[env / g.Gl], 1);
     }
     if (!any) return;
     double* M = g.mat + (size_t)env * k * k;
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_lds_kernel(sbf::Tables t,
     any = __syncthreads_or(any);
     if (tid == 0) {
         g.eact[env] = any;
-        if (any) atomicOr(&g.bact[env / g.Gl], 1);
+        if (any && g.bact) atomicOr(&g.bact[env / g.Gl], 1);
     }
     if (!any) return;   // workgroup-uniform
     double* bv = M + k * k;
