@@ -151,6 +151,33 @@ bool hip_check(hipError_t e, const char* what) {
     return fail(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// The default mode's vectors W1, X, Y and C in one allocation: for every env
+// tile, or, past kVectorBytes (some 2,500 envs of a 205K-cell plan), for an
+// equal share of them at a time; for fewer where the device has no room left.
+constexpr size_t kVectorBytes = (size_t)8 << 30;
+
+bool make_vectors(SbxFdm* f, sbf::Group* g) {
+    const sbf::Tables& t = f->tab;
+    const size_t n = t.n, ny = t.n - t.ft.n_leaf, nc = (size_t)t.ft.n_c + 1;
+    const size_t tile = sizeof(double) * sbf::kEnvTile * (2 * n + ny + nc);
+    const int most = (int)std::min<size_t>(g->nt, std::max<size_t>(kVectorBytes / tile, 1));
+    const int passes = (g->nt + most - 1) / most;
+    double* p = nullptr;
+    for (g->tiles = (g->nt + passes - 1) / passes;; g->tiles = (g->tiles + 1) / 2) {
+        p = (double*)dalloc(f, tile * g->tiles);
+        if (p || g->tiles == 1) break;
+        (void)hipGetLastError();   // (not the next launch's)
+    }
+    if (!p) return false;
+    const size_t rows = (size_t)g->tiles * sbf::kEnvTile;
+    g->W1 = p;
+    g->X = g->W1 + rows * n;
+    g->Y = g->X + rows * n;
+    g->C = g->Y + rows * ny;
+    // C's zero rows (the contributions are written before they are read)
+    return hip_check(hipMemset(g->C, 0, sizeof(double) * rows * nc), "clear the front contributions");
+}
+
 // Device buffers of a group of G envs in blocks of Gl lanes.
 bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     const sbf::Tables& t = f->tab;
@@ -160,13 +187,11 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     const size_t lanes = (size_t)g->nblk * Gl;
     const bool fronts = fields && t.fast;   // the default mode's vectors, in tiles of envs
     g->nt = (G + sbf::kEnvTile - 1) / sbf::kEnvTile;
-    const size_t tl = (size_t)g->nt * sbf::kEnvTile, c_rows = (size_t)t.ft.n_c + 1;
-    g->W1 = (double*)dalloc(f, sizeof(double) * (fronts ? tl : lanes) * t.n);
+    g->t0 = 0;
+    g->tiles = g->nt;
+    g->W1 = fronts ? nullptr : (double*)dalloc(f, sizeof(double) * lanes * t.n);
     const bool w2 = fields && !t.fast;   // the second solve's vector (exact mode)
     g->W2 = w2 ? (double*)dalloc(f, sizeof(double) * lanes * t.n) : nullptr;
-    g->X = fronts ? (double*)dalloc(f, sizeof(double) * tl * t.n) : nullptr;
-    g->Y = fronts ? (double*)dalloc(f, sizeof(double) * tl * std::max(t.n - t.ft.n_leaf, 1)) : nullptr;
-    g->C = fronts ? (double*)dalloc(f, sizeof(double) * tl * c_rows) : nullptr;
     g->T = fields ? (double*)dalloc(f, sizeof(double) * lanes * t.n_cvs) : nullptr;
     g->M = fields ? (double*)dalloc(f, sizeof(double) * lanes * t.n) : nullptr;
     const size_t k = std::max(t.k, 1);
@@ -174,11 +199,10 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     g->mat = fields ? (double*)dalloc(f, sizeof(double) * G * k * k) : nullptr;
     g->eact = (int*)dalloc(f, sizeof(int) * G);
     g->bact = fronts ? nullptr : (int*)dalloc(f, sizeof(int) * g->nblk);
-    if (!g->W1 || !g->pw || !g->eact || (!fronts && !g->bact) || (w2 && !g->W2) || (fields && (!g->T || !g->M || !g->mat))
-        || (fronts && (!g->X || !g->Y || !g->C)))
+    if ((!fronts && (!g->W1 || !g->bact)) || !g->pw || !g->eact || (w2 && !g->W2)
+        || (fields && (!g->T || !g->M || !g->mat)) || (fronts && !make_vectors(f, g)))
         return fail("hipMalloc failed for the field buffers");
-    // C's zero rows (the contributions are written before they are read)
-    return !fronts || hip_check(hipMemset(g->C, 0, sizeof(double) * tl * c_rows), "clear the front contributions");
+    return true;
 }
 
 bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {

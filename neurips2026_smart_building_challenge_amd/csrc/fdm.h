@@ -140,16 +140,17 @@ struct Tables {
 
 struct Group {
     int G, Gl, nblk;
-    int nt;                 // env tiles of the default mode's vectors
+    int nt;                 // env tiles, of the group or (in a launch of the default mode) of the pass
+    int t0, tiles;          // default mode: the pass's first env tile; the tiles that W1, X, Y and C hold
     double* T;              // [nblk][n_cvs][Gl]
     double* M;              // [nblk][n][Gl]
     // exact mode: the forcing solve in place, [nblk][n][Gl]; default mode: the
-    // right-hand side in front order, [nt][n][kEnvTile]
+    // right-hand side in front order, [tiles][n][kEnvTile]
     double* W1;
     double* W2;             // [nblk][n][Gl] the air-side correction (exact mode)
-    double* X;              // [nt][n][kEnvTile] the solution less the ambient temperature (default mode)
-    double* Y;              // [nt][n - n_leaf][kEnvTile] assembled right-hand sides above the leaves (default mode)
-    double* C;              // [nt][n_c + 1][kEnvTile] the fronts' contributions, then a zero row (default mode)
+    double* X;              // [tiles][n][kEnvTile] the solution less the ambient temperature (default mode)
+    double* Y;              // [tiles][n - n_leaf][kEnvTile] assembled right-hand sides above the leaves (default mode)
+    double* C;              // [tiles][n_c + 1][kEnvTile] the fronts' contributions, then a zero row (default mode)
     double* pw;             // [G][k] air-side power, then the dense solve's result
     double* mat;            // [G][k][k] I + diag(g) S
     int* eact;              // [G] env has a nonzero air-side conductance this step
@@ -173,6 +174,6 @@ struct StepIn {
 static_assert(sizeof(Tri) == 56 && sizeof(Front) == 40 && sizeof(AsmRow) == 32 && sizeof(FrontTab) == 104,
               "Tri / Front / FrontTab layout");
 static_assert(sizeof(Tables) == 440 && offsetof(Tables, S) == 408 && offsetof(Tables, nz) == 432, "Tables layout");
-static_assert(sizeof(Group) == 104 && sizeof(StepIn) == 48, "Group / StepIn layout");
+static_assert(sizeof(Group) == 112 && sizeof(StepIn) == 48, "Group / StepIn layout");
 
 }  // namespace sbf

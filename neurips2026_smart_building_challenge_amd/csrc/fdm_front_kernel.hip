@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void front_forcing_kernel(sbf::Tables t, sbf::
     const int z = in.q ? -1 : t.czone[tt];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const int l = wave * 4 + q, env = te * E + l;
+        const int l = wave * 4 + q, env = (g.t0 + te) * E + l;
         double v = 0.0;
         if (env < g.G) {
             const size_t b = env / Gl, gl = env % Gl;
@@ -531,7 +531,8 @@ __global__ __launch_bounds__(kSensedThreads) void front_sensed_kernel(sbf::Table
     const int te = (int)(blockIdx.x % (unsigned)g.nt), i = (int)(blockIdx.x / (unsigned)g.nt);
     const int j = threadIdx.x % E, s = threadIdx.x / E;
     const double* Xb = g.X + (size_t)te * t.n * E + j;
-    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
+    const int env = (g.t0 + te) * E + j;
+    const double base = base_of(in.amb[min(env, g.G - 1)]);
     double acc = 0.0;
 #pragma unroll 8
     for (int p = t.sn_p[i] + s; p < t.sn_p[i + 1]; p += R) acc += t.sn_x[p] * (base + Xb[(size_t)t.ft.sn_w[p] * E]);
@@ -541,7 +542,6 @@ __global__ __launch_bounds__(kSensedThreads) void front_sensed_kernel(sbf::Table
         if (s < h) part[s][j] += part[s + h][j];
         __syncthreads();
     }
-    const int env = te * E + j;
     if (s == 0 && env < g.G) {
         const size_t x = (size_t)env * t.k + i;
         g.pw[x] = in.g[x] * (in.airT[x] - part[0][j]);
@@ -561,13 +561,13 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
     const int j = lane & 15, kk = lane >> 4;
     const int n = t.n, k = t.k, Gl = g.Gl;
     const double* Xb = g.X + (size_t)te * n * E + j;
-    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
+    const int e0 = (g.t0 + te) * E, ej = min(e0 + j, g.G - 1);
+    const double base = base_of(in.amb[ej]);
     double y[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) y[q] = Xb[(size_t)t.ft.rx[min(t0 + wave * 16 + kk + 4 * q, n - 1)] * E];
     if (t.R) {
-        const int env = min(te * E + j, g.G - 1);
-        const double* qv = g.pw + (size_t)env * k;
+        const double* qv = g.pw + (size_t)ej * k;
         const double* Rb = t.R + min(t0 + wave * 16 + j, n - 1);   // A: row (cell) lane % 16
         d4 acc = {};
 #pragma unroll 5
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
             const double a = col < k ? Rb[(size_t)min(col, k - 1) * n] : 0.0;
             acc = mfma(a, qv[min(col, k - 1)], acc);
         }
-        const bool on = g.eact[env] != 0;
+        const bool on = g.eact[ej] != 0;
 #pragma unroll
         for (int q = 0; q < 4; q++) y[q] = on ? y[q] + acc[q] : y[q];
     }
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
         const double mr = t.mret[tt], mg = t.mgain[tt];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int l = wave * 4 + q, env = te * E + l;
+            const int l = wave * 4 + q, env = e0 + l;
             if (env >= g.G) break;
             const size_t b = env / Gl, gl = env % Gl, mi = (b * n + tt) * Gl + gl;
             const double v = ys[l][lane];
@@ -597,6 +597,7 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
             g.T[(b * t.n_cvs + cell) * Gl + gl] = v;
         }
     }
+    if (g.t0 != 0) return;   // the first pass writes every env's other cells
     const size_t tu = (size_t)g.nblk * t.n_unsolved * Gl;
     for (size_t x = (size_t)blockIdx.x * 256 + threadIdx.x; x < tu; x += (size_t)gridDim.x * 256) {
         const size_t bu = x / Gl;
@@ -652,9 +653,9 @@ void launch_level(const sbf::Tables& t, const sbf::Group& g, int h, hipStream_t 
 
 extern "C" int sbf_launch_dense(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s);
 
-// One batched step of a group in the default mode.
-extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in,
-                                     hipStream_t s) {
+namespace {
+
+int launch_pass(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s) {
     const unsigned tiles = (unsigned)((t->n + 63) / 64) * (unsigned)g->nt;
     hipLaunchKernelGGL(front_forcing_kernel, dim3(tiles), dim3(256), 0, s, *t, *g, *in);
     for (int h = 0; h < t->ft.n_levels; h++) launch_level<false>(*t, *g, h, s);
@@ -666,6 +667,21 @@ extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* g, 
     }
     hipLaunchKernelGGL(front_update_kernel, dim3(tiles), dim3(256), 0, s, *t, *g, *in);
     return (int)hipGetLastError();
+}
+
+}  // namespace
+
+// One batched step of a group in the default mode, in passes over the env
+// tiles that the vectors hold (an env's result does not depend on its pass).
+extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* group, const sbf::StepIn* in,
+                                     hipStream_t s) {
+    for (int t0 = 0; t0 < group->nt; t0 += group->tiles) {
+        sbf::Group pass = *group;
+        pass.t0 = t0;
+        pass.nt = std::min(group->tiles, group->nt - t0);
+        if (int e = launch_pass(t, &pass, in, s)) return e;
+    }
+    return 0;
 }
 
 // The fronts' operators from the factors (rows scheduled in L and U: nl, nu;
