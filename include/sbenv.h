@@ -466,8 +466,10 @@ typedef struct {
  * elimination tree into dense fronts, whose inverses and couplings are formed
  * at open; a step's solve is one matrix product per front up the tree and one
  * down it, so row sums are formed in another order and results agree with the
- * reference to rounding, far inside 1e-9 relative. SBX_FDM_EXACT: every level
- * in the reference's order, bit-identical results. envs_per_block (envs that
+ * reference to rounding, far inside 1e-9 relative; factors for which the
+ * fronts are not that accurate (checked at open: a solve whose solution is
+ * all ones, within 1e-12) run as with SBX_FDM_EXACT. SBX_FDM_EXACT: every
+ * level in the reference's order, bit-identical results. envs_per_block (envs that
  * share a block of the field's layout) 0 picks 1 (default) or up to 64
  * (exact). The default mode also takes the air-side correction from the
  * responses of the applied columns (sbx_fdm_air_responses) instead of a

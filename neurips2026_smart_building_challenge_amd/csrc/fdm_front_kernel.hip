@@ -655,11 +655,15 @@ extern "C" int sbf_launch_dense(const sbf::Tables* t, const sbf::Group* g, const
 
 namespace {
 
+void launch_solve(const sbf::Tables& t, const sbf::Group& g, hipStream_t s) {
+    for (int h = 0; h < t.ft.n_levels; h++) launch_level<false>(t, g, h, s);
+    for (int h = t.ft.n_levels; h-- > 0;) launch_level<true>(t, g, h, s);
+}
+
 int launch_pass(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s) {
     const unsigned tiles = (unsigned)((t->n + 63) / 64) * (unsigned)g->nt;
     hipLaunchKernelGGL(front_forcing_kernel, dim3(tiles), dim3(256), 0, s, *t, *g, *in);
-    for (int h = 0; h < t->ft.n_levels; h++) launch_level<false>(*t, *g, h, s);
-    for (int h = t->ft.n_levels; h-- > 0;) launch_level<true>(*t, *g, h, s);
+    launch_solve(*t, *g, s);
     if (t->k > 0) {
         hipLaunchKernelGGL(front_sensed_kernel, dim3((unsigned)t->k * (unsigned)g->nt), dim3(kSensedThreads), 0, s,
                            *t, *g, *in);
@@ -682,6 +686,34 @@ extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* gro
         if (int e = launch_pass(t, &pass, in, s)) return e;
     }
     return 0;
+}
+
+// Worst error of a solve whose solution is all ones: the largest |x - 1| over
+// the rows, as the bits of a double that is not negative (a NaN's lie above).
+namespace {
+
+__global__ void check_fill_kernel(sbf::Tables t, double* W, unsigned long long* worst) {
+    const size_t x = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int tt = (int)(x / E);
+    if (x == 0) *worst = 0;
+    if (tt < t.n) W[(size_t)t.ft.rf[tt] * E + x % E] = (t.ft.rowsum[tt] + t.mcoup[tt]) + t.cap[tt];
+}
+
+__global__ void check_max_kernel(int n, const double* X, unsigned long long* worst) {
+    const int row = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (row < n) atomicMax(worst, (unsigned long long)__double_as_longlong(fabs(X[(size_t)row * E] - 1.0)));
+}
+
+}  // namespace
+
+extern "C" int sbf_launch_front_check(const sbf::Tables* t, const sbf::Group* group, unsigned long long* worst) {
+    sbf::Group g = *group;
+    g.nt = 1;
+    hipLaunchKernelGGL(check_fill_kernel, dim3((unsigned)(((size_t)t->n * E + 255) / 256)), dim3(256), 0, nullptr, *t,
+                       g.W1, worst);
+    launch_solve(*t, g, nullptr);
+    hipLaunchKernelGGL(check_max_kernel, dim3((unsigned)((t->n + 255) / 256)), dim3(256), 0, nullptr, t->n, g.X, worst);
+    return (int)hipGetLastError();
 }
 
 // The fronts' operators from the factors (rows scheduled in L and U: nl, nu;

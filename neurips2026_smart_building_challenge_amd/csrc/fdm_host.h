@@ -17,6 +17,7 @@ struct SbxFdm {
     double* d_mass_init = nullptr;
     std::vector<sbf::FrontLevel> front_levels;   // (tab.ft.levels points here)
     std::vector<void*> owned;     // device buffers of the group
+    bool inaccurate = false;      // the fronts' operators failed their check at open
 };
 
 extern "C" int sbf_launch_step(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s);
