@@ -475,12 +475,11 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     for (auto& e : fix) *e.first = f->d_tables + e.second;
     if (T.fast) {
         // the fronts' operators, formed on the device from the factors' rows
-        double *dense = nullptr, *sol = nullptr, *ops = (double*)dalloc(f, 8 * fp.ops);
+        double *dense = nullptr, *ops = (double*)dalloc(f, 8 * fp.ops);
         const int leaf_fronts = (int)(std::partition_point(fp.fronts.begin(), fp.fronts.end(),
                                                            [&](const sbf::Front& q) { return q.off < fp.n_leaf; })
                                       - fp.fronts.begin());
-        bool ok = ops && hip_check(hipMalloc(&dense, 8 * dense_n), "hipMalloc(front blocks)")
-                  && hip_check(hipMalloc(&sol, 8 * sol_n), "hipMalloc(front solutions)")
+        bool ok = ops && hip_check(hipMalloc(&dense, 8 * (dense_n + sol_n)), "hipMalloc(front blocks)")
                   && hip_check(hipMemset(dense, 0, 8 * dense_n), "clear front blocks");
         T.ft.ops = ops;
         auto at = [&](size_t off) { return (const void*)(f->d_tables + off); };
@@ -488,11 +487,10 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
              && hip_check((hipError_t)sbf_launch_front_ops(&T, (int)L.rows.size(), (int)U.rows.size(), leaf_fronts,
                                                            (const int*)at(o_front), (const int*)at(o_local),
                                                            (const int*)at(o_bperm), (const long long*)at(o_d0),
-                                                           (const long long*)at(o_s0), dense, sol, ops),
+                                                           (const long long*)at(o_s0), dense, dense + dense_n, ops),
                           "front operators")
              && hip_check(hipDeviceSynchronize(), "front operators");
         (void)hipFree(dense);
-        (void)hipFree(sol);
         if (!ok) return ops ? false : fail("hipMalloc failed for the front operators");
     }
     if (!hip_check(hipMalloc(&f->d_temp_init, 8 * (size_t)n_cvs), "hipMalloc(temp_init)")) return false;

@@ -365,24 +365,27 @@ __device__ int b_index(const sbf::Front& f, const int* bperm, int i) {
     return lo;
 }
 
-// One thread per scheduled row of a factor: its terms into the dense blocks.
+// kRowLanes lanes per scheduled row of a factor: its terms into the dense blocks
+// (one lane a row: 0.8 ms for the 120 x 90 building's L).
+constexpr int kRowLanes = 16;
+
 template <bool UPPER>
 __global__ void ops_scatter_kernel(sbf::Tri tri, int nrows, const sbf::Front* fronts, OpsTab o) {
-    const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int q = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kRowLanes), l = (int)(threadIdx.x % kRowLanes);
     if (q >= nrows) return;
     const int i = tri.rows[q], fi = o.front_of[i];
     if (UPPER) {
         const sbf::Front f = fronts[fi];
         double* D = o.dense + o.d0[fi];
         const int li = o.local[i];
-        D[(size_t)f.w * f.w + (size_t)li * f.w + li] = tri.diag[q];
-        for (int e = tri.ptr[q]; e < tri.ptr[q + 1]; e++) {
+        if (l == 0) D[(size_t)f.w * f.w + (size_t)li * f.w + li] = tri.diag[q];
+        for (int e = tri.ptr[q] + l; e < tri.ptr[q + 1]; e += kRowLanes) {
             const int c = tri.col[e];
             if (o.front_of[c] == fi) D[(size_t)f.w * f.w + (size_t)li * f.w + o.local[c]] = tri.val[e];
             else D[2 * (size_t)f.w * f.w + (size_t)f.w * f.r + (size_t)li * f.r + b_index(f, o.bperm, c)] = tri.val[e];
         }
     } else {
-        for (int e = tri.ptr[q]; e < tri.ptr[q + 1]; e++) {
+        for (int e = tri.ptr[q] + l; e < tri.ptr[q + 1]; e += kRowLanes) {
             const int c = tri.col[e], fc = o.front_of[c], lc = o.local[c];
             const sbf::Front f = fronts[fc];
             double* D = o.dense + o.d0[fc];
@@ -395,8 +398,10 @@ __global__ void ops_scatter_kernel(sbf::Tri tri, int nrows, const sbf::Front* fr
 // One lane per column of a front's operators: column c < w of K solves
 // L U x = e_c, the next r solve U x = -U_CB, the last r (rows of F) z L = -L_BC.
 // A wavefront's 64 columns are kept in LDS; a row's coefficients are the same
-// for every lane (scalar loads), eight products a trip in four sums (columns
-// in global memory and one chain a row: 32 ms for a 205K-cell plan, 5 so).
+// for every lane (scalar loads), in four sums. What bounds it is the latency of
+// a row's trips over its coefficients: 32 products a trip, and what is left
+// over loaded at once. A 205K-cell plan: columns in global memory and one chain
+// a row 32 ms, eight products a trip and the rest one by one 7.3 ms, 5.3 ms so.
 struct OpsCol {
     double (*x)[64];
     int lane;
@@ -404,10 +409,23 @@ struct OpsCol {
     __device__ double dot(const double* M, size_t stride, int q0, int q1) const {
         double s[4] = {0.0, 0.0, 0.0, 0.0};
         int q = q0;
+        for (; q + 32 <= q1; q += 32)
+#pragma unroll
+            for (int u = 0; u < 32; u++) s[u & 3] = fma(M[(size_t)(q + u) * stride], x[q + u][lane], s[u & 3]);
         for (; q + 8 <= q1; q += 8)
 #pragma unroll
             for (int u = 0; u < 8; u++) s[u & 3] = fma(M[(size_t)(q + u) * stride], x[q + u][lane], s[u & 3]);
-        for (; q < q1; q++) s[0] = fma(M[(size_t)q * stride], x[q][lane], s[0]);
+        if (q < q1) {   // the loads of the rest at once too
+            double m[8], y[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int p = min(q + u, q1 - 1);
+                m[u] = M[(size_t)p * stride];
+                y[u] = x[p][lane];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) s[0] = q + u < q1 ? fma(m[u], y[u], s[0]) : s[0];
+        }
         return (s[0] + s[1]) + (s[2] + s[3]);
     }
 };
@@ -455,7 +473,7 @@ __global__ void ops_pack_kernel(const sbf::Front* fronts, int n_fronts, OpsTab o
         const int w = f.w, r = f.r, ld = w + 2 * r, kw = (w + 3) / 4, ks = kw + (r + 3) / 4;
         const double* S = o.sol + o.s0[fi];
         const size_t nF = (size_t)((r + 15) / 16) * kw * 64, nK = (size_t)((w + 15) / 16) * ks * 64;
-        for (size_t x = threadIdx.x; x < nF + nK; x += blockDim.x) {
+        for (size_t x = blockIdx.y * blockDim.x + threadIdx.x; x < nF + nK; x += gridDim.y * blockDim.x) {
             const bool up = x < nF;
             const size_t y = up ? x : x - nF;
             const int lane = (int)(y & 63), step = (int)((y >> 6) % (size_t)(up ? kw : ks));
@@ -726,9 +744,11 @@ extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, int le
     const OpsTab o{front_of, local, bperm, d0, dense, sol, s0};
     const sbf::Front* fr = t->ft.fronts;
     const int nf = t->ft.n_fronts;
+    constexpr int rows = 256 / kRowLanes;   // a workgroup's
     if (nl > 0)
-        hipLaunchKernelGGL((ops_scatter_kernel<false>), dim3((nl + 255) / 256), dim3(256), 0, nullptr, t->L, nl, fr, o);
-    hipLaunchKernelGGL((ops_scatter_kernel<true>), dim3((nu + 255) / 256), dim3(256), 0, nullptr, t->U, nu, fr, o);
+        hipLaunchKernelGGL((ops_scatter_kernel<false>), dim3((nl + rows - 1) / rows), dim3(256), 0, nullptr, t->L, nl,
+                           fr, o);
+    hipLaunchKernelGGL((ops_scatter_kernel<true>), dim3((nu + rows - 1) / rows), dim3(256), 0, nullptr, t->U, nu, fr, o);
     int wmax = 1;
     for (int h = 0; h < t->ft.n_levels; h++) wmax = std::max(wmax, t->ft.levels[h].wmax);
     const size_t lds = sizeof(double) * 64 * (size_t)wmax;
@@ -747,6 +767,6 @@ extern "C" int sbf_launch_front_ops(const sbf::Tables* t, int nl, int nu, int le
         up.s0 += leaves;
         hipLaunchKernelGGL(ops_solve_kernel, dim3(nf - leaves, 16), dim3(64), lds, nullptr, fr + leaves, up);
     }
-    hipLaunchKernelGGL(ops_pack_kernel, dim3(nf), dim3(256), 0, nullptr, fr, nf, o, ops);
+    hipLaunchKernelGGL(ops_pack_kernel, dim3(nf, 4), dim3(256), 0, nullptr, fr, nf, o, ops);
     return (int)hipGetLastError();
 }
