@@ -944,8 +944,8 @@ __global__ __launch_bounds__(W) void fe_post_kernel(Args a) {
 // whole swaps in the producer's records. One applier
 // keeps up with the walk, and its LDS is what the field step running beside
 // the plan is left with: at 512 envs (two workgroups per CU) four appliers on
-// 64 KB each held the wide up heights at 531 us, one on 51 KB leaves them
-// 103 us, and two env steps went from 13.3 to 9.7 ms.
+// 64 KB each held the wide up heights at 531 us, one on 51 KB (46 since) leaves
+// them 103 us, and two env steps went from 13.3 to 9.7 ms.
 namespace {
 
 // Words of a walk window: the most that tile the ring and fit a record's seven
@@ -1089,7 +1089,9 @@ __device__ __forceinline__ int slot_wait(int* flag, bool full) {
     return v;
 }
 
-__device__ int writelane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+// v_writelane_b32 (the compiler has an intrinsic for it, but no builtin; under
+// another name than an intrinsic's the device code does not link).
+__device__ int writelane(int v, int lane, int old) __asm("llvm.amdgcn.writelane");
 
 // The room's pairs from the stream; returns their count. The walk is at word
 // x of a window; drift is what x is ahead of two words a cell from the window's
@@ -1251,7 +1253,7 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
     const Tabs& t = a.t;
     extern __shared__ __align__(16) unsigned char lds[];
     // flag: the slot's pairs, or -1 where it is free
-    __shared__ int flag[2], total, ready, used;
+    __shared__ int flag[2], ready, used;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / W));
     const ConvLds L = conv_lds(t.cv_max_room, a.cv_lds_pairs, a.cv_nc_lds);
     auto slot = [&](int i) {
@@ -1272,7 +1274,7 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
     int* gidx = reinterpret_cast<int*>(gmt + SBE_MT_N);   // the stream's position in its block
     for (int i = (int)threadIdx.x; i < SBE_MT_N; i += (int)blockDim.x) w.raw[i] = gmt[i];
     if (threadIdx.x < 2) flag[threadIdx.x] = -1;
-    if (threadIdx.x == 0) total = ready = used = 0;
+    if (threadIdx.x == 0) ready = used = 0;
     __syncthreads();
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(3);   // the field step's wavefronts share the SIMD
@@ -1309,6 +1311,7 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
         produce(w, ((uint64_t)t.cv_thr_hi << 32) | t.cv_thr_lo, t.cv_thr_hi == 0xFFFFFFFFu, t.cv_usual);
     } else {
         unsigned long long* moves = a.cv_moves + (size_t)s * t.cv_cells;
+        int total = 0;   // moves of the rooms so far
         for (int rm = 0; rm < t.cv_rooms; rm++) {
             const RoomSlot R = slot(rm & 1);
             const int b0 = t.cv_off[rm], n = t.cv_off[rm + 1] - b0;
@@ -1327,36 +1330,28 @@ __global__ __launch_bounds__(3 * W) void fe_conv_plan_kernel(Args a) {
             else room_shuffle<false>(R, m);
             post(&flag[rm & 1], -1);
             // moves: cell i's value goes to cell q[i] (convection-cell indices;
-            // the move kernels map them to field cells), in any order: each
-            // reads and writes cells of its own
+            // the move kernels map them to field cells)
             for (int i0 = 0; i0 < n; i0 += 4 * W) {
                 int q[4];
                 unsigned long long mm[4];
-                int cnt = 0;
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int i = i0 + u * W + lane();
                     q[u] = i < n ? (int)R.qinv[i] : i;
                     mm[u] = ballot(q[u] != i);
-                    cnt += __popcll(mm[u]);
                 }
-                if (cnt == 0) continue;
-                int at = 0;
-                if (lane() == 0) at = atomicAdd(&total, cnt);
-                at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int i = i0 + u * W + lane();
                     if (q[u] != i)
-                        moves[at + below_me(mm[u])] = ((unsigned long long)(unsigned)(b0 + q[u]) << 32) | (unsigned)(b0 + i);
-                    at += __popcll(mm[u]);
+                        moves[total + below_me(mm[u])] = ((unsigned long long)(unsigned)(b0 + q[u]) << 32) | (unsigned)(b0 + i);
+                    total += __popcll(mm[u]);
                 }
             }
             wsync();
         }
+        if (lane() == 0) a.cv_count[s] = total;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) a.cv_count[s] = total;
 }
 
 // The moves of the step, read then written (two launches: every value is read
