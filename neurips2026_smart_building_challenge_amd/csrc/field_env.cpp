@@ -620,9 +620,9 @@ bool field_attach(FieldScen* f, const std::string& path, const std::vector<sbe::
         const double expect = 1.5 * std::min(std::max(f->conv_p, 0.0), 1.0) * mr_lds;
         f->lds_pairs = std::max(512, (int)expect);
         const size_t all = 160 * 1024 - 64;   // (a few words are the kernel's own)
-        if (4 * 4 * SBE_MT_N + 3 * mr_lds + 16 > 154 * 1024)
+        if (mr_lds > sbe::kConvRoomCells)
             return (*err = "a convection room is too large for the plan kernel's LDS"), false;
-        f->nc_lds = sbe::conv_lds(mr_lds, 512, 1).bytes <= all;   // (rooms of up to some 46,000 cells)
+        f->nc_lds = sbe::conv_lds(mr_lds, 512, 1).bytes <= all;   // (rooms of up to 46,703 cells)
         while (sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes > all) f->lds_pairs -= 64;
         lds = std::max(lds, (int)sbe::conv_lds(mr_lds, f->lds_pairs, f->nc_lds).bytes);
         const size_t cells = (size_t)std::max(f->t.cv_cells, 1), mr = (size_t)std::max(f->t.cv_max_room, 1);

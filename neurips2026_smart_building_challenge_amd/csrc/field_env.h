@@ -187,6 +187,10 @@ struct Slot {
 
 enum { FE_STEP = 0, FE_RESET = 1 };
 
+// The largest convection room that is taken: its permutation (two bytes a cell),
+// 512 pairs a slot and the stream's blocks fit the 160 KB of LDS with room to spare.
+constexpr int kConvRoomCells = 49232;
+
 // The convection plan kernel's LDS for rooms of up to `room` cells: four MT
 // blocks, a record and the low byte of each of their words, with nc_lds the
 // room's candidate counts (and up to 15 cells before and after it; else they
