@@ -1,20 +1,20 @@
 """The field scenarios' convection plan (csrc/field_env_kernel.hip,
-fe_conv_plan_kernel) restated step for step in Python and checked against
-the reference core's sequential algorithm (complete_port/csim/sb_convect.c:
-39-73 with sb_rng.c's masked-rejection interval draw), on the CPU:
+fe_conv_plan_kernel) restated in Python and checked against the reference
+core's sequential algorithm (complete_port/csim/sb_convect.c:39-73 with
+sb_rng.c's masked-rejection interval draw), on the CPU:
 
-  - window rounds: lane i of a 64-lane window holds the stream words at
-    offsets 2i, 2i + 1, 2i + 2; the two parities' swap bits (P0, P1) shifted
-    by half the drift give every cell's decision, and each swap's candidate
-    draw reads its words from the same window's first 128 words (or, past
-    them, from the stream):
-    the pairs and the stream position after the room equal the sequential
-    draws, over random rooms (sizes 1..700, p from 0.05 to 1, cells without
-    or with one candidate);
-  - the shuffle composed into the room's inverse permutation q from the top
-    (q <- q o (a b) as each pair becomes final) and applied as moves
-    T_new[q[i]] = T_old[i] equals the reference's Fisher-Yates shuffle then
-    swaps in order.
+  - the producer's records (`hops`) and the walk over them (`room_pairs`), as
+    the kernel has them: windows of 104 words entered at any word, whole swaps
+    of the commonest candidate count from the records, other counts from the
+    first two bytes, longer draws past the window's end, cells without or with
+    one candidate. The pairs and the stream position after the room equal the
+    sequential draws, over random rooms and one of 46,900 cells, for every
+    kind of commonest count (none, up to 64) and counts up to 255; and a
+    record alone, at every word of a window;
+  - the shuffle's draws as the fixed point over 64 words, and the shuffle
+    composed into the room's inverse permutation q from the top (q <- q o (a b)
+    as each pair becomes final) and applied as moves T_new[q[i]] = T_old[i],
+    equal to the reference's Fisher-Yates shuffle then swaps in order.
 """
 from __future__ import annotations
 
@@ -52,80 +52,6 @@ def sequential_pairs(words: list, pos: int, ncand, thr: int):
         pick, pos = interval(words, pos, int(ncand[j]) - 1)
         pairs.append((j, pick))
     return pairs, pos
-
-
-def window_pairs(words: list, pos: int, ncand, thr: int):
-    """The plan kernel's window rounds."""
-    n = len(ncand)
-    pairs, j = [], 0
-    full = (1 << 64) - 1
-    while j < n:
-        w0 = [words[pos + 2 * i] for i in range(W)]
-        w1 = [words[pos + 2 * i + 1] for i in range(W)]
-        w2 = [words[pos + 2 * i + 2] for i in range(W)]
-        nc = [int(ncand[j + i]) if j + i < n else 0 for i in range(W)]
-        P0 = sum(1 << i for i in range(W) if (((w0[i] >> 5) << 26) | (w1[i] >> 6)) <= thr)
-        P1 = sum(1 << i for i in range(W) if (((w1[i] >> 5) << 26) | (w2[i] >> 6)) <= thr)
-        HC = sum(1 << i for i in range(W) if nc[i] > 0)
-
-        def wreg(q):
-            return w1[q >> 1] if q & 1 else w0[q >> 1]
-
-        c, drift, slow, smax = 0, 0, False, 0
-        while True:
-            tt, par = drift >> 1, drift & 1
-            if c + tt >= W:
-                break
-            cand = ((P1 if par else P0) >> tt) & HC & ((full << c) & full)
-            if cand == 0:
-                c = W - tt
-                break
-            cc = (cand & -cand).bit_length() - 1
-            mx = nc[cc] - 1
-            q = 2 * (cc + tt) + par + 2
-            pick = 0
-            if mx:
-                mask = smear(mx)
-                while True:
-                    if q >= 2 * W:
-                        slow = True
-                        break
-                    v = wreg(q) & mask
-                    q += 1
-                    if v <= mx:
-                        pick = v
-                        break
-            if slow:
-                pos += q
-                j += cc
-                smax = mx
-                break
-            pairs.append((j + cc, pick))
-            drift = q - 2 * (cc + 1)
-            c = cc + 1
-        if slow:
-            pick, pos = interval(words, pos, smax)
-            pairs.append((j, pick))
-            j += 1
-            continue
-        ce = min(c, n - j)
-        pos += 2 * ce + drift
-        j += ce
-    return pairs, pos
-
-
-def test_window_rounds_equal_sequential_draws():
-    rng = np.random.default_rng(20261202)
-    for trial in range(200):
-        n = int(rng.integers(1, 700))
-        p = float(rng.choice([0.05, 0.1, 0.3, 0.6, 0.95, 1.0]))
-        thr = (1 << 53) if p >= 1 else int(np.floor(p * 2.0 ** 53))
-        ncand = rng.integers(0, 25, size=n)
-        ncand[rng.random(n) < 0.1] = 0
-        ncand[rng.random(n) < 0.1] = 1
-        words = [int(x) for x in rng.integers(0, 2 ** 32, size=6 * n + 1000, dtype=np.uint64)]
-        start = int(rng.integers(0, 50))
-        assert window_pairs(words, start, ncand, thr) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
 
 
 def test_composed_moves_equal_shuffled_swaps():
@@ -204,56 +130,123 @@ def test_draws_by_fixed_point_equal_sequential_draws():
         assert got == want and gpos == pos, m
 
 
-CHUNK = 104
+CHUNK = 104          # words of a window (kWin)
+NO_HOP = 0xFE        # kNoHop
 
 
-def walk_pairs(words: list, pos: int, ncand, thr: int):
-    """The plan kernel's walk: windows are the stream's chunks of 104 words,
-    entered at any word; the next swapping cell is the next swap bit of the
-    walk's parity (a cell's swap draw is words x and x + 1)."""
+def hops(w: list, thr: int, usual: int) -> list:
+    """produce(): the records of the window whose first word is w[0], and the words past it."""
+    swap = [(((w[i] >> 5) << 26) | (w[i + 1] >> 6)) <= thr for i in range(CHUNK)]
+    umax, umask = usual - 1, smear(max(usual - 1, 0))
+    out = []
+    for x in range(CHUNK):
+        d = next((q - x for q in range(x, CHUNK, 2) if swap[q]), None)
+        if d is None:
+            out.append(NO_HOP)
+            continue
+        v = [w[x + d + 2 + i] & 0xFF & umask for i in range(3)]
+        k = 1 if v[0] <= umax else 2 if v[1] <= umax else 3
+        ok = v[k - 1] <= umax and x + d + 2 + k < CHUNK
+        out.append((d + 2) << 1 | (1 | k << 8 | v[k - 1] << 10 if ok else 0))
+    return out
+
+
+def room_pairs(words: list, pos: int, ncand, thr: int, usual: int):
+    """room_pairs(): the walk of one room from stream word pos; the pairs and the position after it."""
     n, pairs, j = len(ncand), [], 0
-    while j < n:
-        x0 = pos // CHUNK * CHUNK
-        w = words[x0:]
-        swap = [(((w[i] >> 5) << 26) | (w[i + 1] >> 6)) <= thr for i in range(CHUNK)]
-        nc = [int(ncand[j + i]) if j + i < n else 0 for i in range(W)]
-        x = drift = pos - x0
+    if n == 0:
+        return pairs, pos
+    x0 = pos // CHUNK * CHUNK
+    x = drift = pos - x0
+    while True:
+        rec = hops(words[x0:x0 + CHUNK + 8], thr, usual)
+        rule, is_usual = [], []
+        for i in range(W):
+            nc = int(ncand[min(j + i, n - 1)])
+            mx = -2 if j + i >= n or nc == 0 else nc - 1 if nc > 1 else -1
+            rule.append((smear(nc - 1) if mx >= 0 else 0, mx))
+            is_usual.append(j + i < n and nc == usual)
+        got, ahead = [], drift + 2
         while x < CHUNK:
-            nxt = [q for q in range(x, CHUNK, 2) if swap[q]]
-            if not nxt:
-                break
-            c = (nxt[0] - drift) >> 1
-            x = nxt[0] + 2
-            v = 0
-            if nc[c] == 0:
-                continue
-            while nc[c] > 1:
-                v = (w[x] & 0xFF) & smear(nc[c] - 1)
-                x += 1
-                if v <= nc[c] - 1:
+            while True:
+                h = rec[x]
+                xs = x + ((h >> 1) & 0x7F)
+                c = (xs - ahead) >> 1
+                if not (is_usual[c & 63] and h & 1):
                     break
-            pairs.append((j + c, v))
-            drift = x - 2 * (c + 1)
-        ce = min((max(x, CHUNK + (x & 1)) - drift) >> 1, n - j)
-        pos = x0 + 2 * ce + drift
+                got.append((c, (h >> 10) & 0x3F))
+                k = (h >> 8) & 3
+                ahead += k
+                x = xs + k      # (a whole swap ends before its window does)
+                assert x < CHUNK
+            if h & NO_HOP == NO_HOP:
+                break
+            mask, mx = rule[c & 63]
+            x = xs
+            if mx == -2:
+                continue
+            v = 0
+            if mx >= 0:
+                v = words[x0 + x] & 0xFF & mask
+                x += 1
+                if v > mx:
+                    v = words[x0 + x] & 0xFF & mask
+                    x += 1
+            while mx >= 0 and v > mx:
+                v = words[x0 + x] & 0xFF & mask
+                x += 1
+            got.append((c, v))
+            ahead = x - 2 * c
+        assert len(got) <= W and all(c < W for c, _ in got)
+        drift = ahead - 2
+        pairs += [(j + c, v) for c, v in got]
+        xe = max(x, CHUNK + (x & 1))
+        ce = (xe - drift) >> 1
+        if ce >= n - j:
+            return pairs, x0 + 2 * (n - j) + drift
         j += ce
-    return pairs, pos
+        x = xe
+        while True:
+            x -= CHUNK
+            x0 += CHUNK
+            if x < CHUNK:
+                break
+        drift = x
 
 
-def test_walk_equals_sequential_draws():
+def test_walk_over_records_equals_sequential_draws():
     rng = np.random.default_rng(77)
-    for trial in range(300):
-        n = int(rng.integers(1, 500))
-        p = float(rng.choice([0.0, 0.05, 0.1, 0.3, 0.6, 0.95, 1.0]))
+    for trial in range(400):
+        usual = int(rng.choice([0, 2, 3, 8, 24, 33, 48, 63, 64]))
+        n = int(rng.integers(0, 500)) if trial else 46900
+        p = float(rng.choice([0.0, 0.05, 0.1, 0.3, 0.6, 0.95, 1.0])) if trial else 0.6
         thr = (1 << 53) if p >= 1 else int(np.floor(p * 2.0 ** 53))
-        ncand = rng.integers(0, 25, size=n)
-        ncand[rng.random(n) < 0.1] = 0
-        ncand[rng.random(n) < 0.1] = 1
-        if trial % 3 == 0:
-            ncand[:] = rng.choice([1, 2, 24, 129, 255])
-        words = [int(x) for x in rng.integers(0, 2 ** 32, size=7 * n + 1000, dtype=np.uint64)]
+        others = np.concatenate([[0, 1], rng.integers(2, 65, 4), rng.integers(65, 256, 4)])
+        if trial % 4 == 1:   # a draw that rejects often: 129 of 256 values
+            others = np.array([129])
+        ncand = rng.choice(others, size=n)
+        if usual:
+            ncand[rng.random(n) < float(rng.choice([0.1, 0.87, 1.0]))] = usual
+        elif n:
+            ncand[(ncand >= 2) & (ncand <= 64)] = 0   # the host sets 0 only where no count is in 2..64
+        words = [int(x) for x in rng.integers(0, 2 ** 32, size=8 * n + 1000, dtype=np.uint64)]
         start = int(rng.integers(0, 700))
-        assert walk_pairs(words, start, ncand, thr) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
+        assert room_pairs(words, start, ncand, thr, usual) == sequential_pairs(words, start, ncand, thr), (trial, n, p)
+
+
+def test_walk_where_draws_run_past_whole_windows():
+    """A candidate draw whose words are all rejected over two windows and more."""
+    rng = np.random.default_rng(78)
+    for trial in range(40):
+        n, usual = int(rng.integers(1, 200)), int(rng.choice([0, 24, 64]))
+        ncand = rng.choice([1, 0, 129, 129], size=n) if usual == 0 else rng.choice([usual, 129], size=n)
+        words = [int(x) for x in rng.integers(0, 2 ** 32, size=8 * n + 3000, dtype=np.uint64)]
+        start = int(rng.integers(0, 300))
+        a = start + int(rng.integers(0, 4 * n))
+        for q in range(a, a + int(rng.integers(100, 400))):
+            words[q] |= 0xFF
+        for thr in (1 << 53, 1 << 52):
+            assert room_pairs(words, start, ncand, thr, usual) == sequential_pairs(words, start, ncand, thr), trial
 
 
 def test_hop_records_equal_sequential_draws():

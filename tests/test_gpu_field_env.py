@@ -274,6 +274,32 @@ def test_gpu_field_env_conv_big_room(tmp_path):
     vec.close()
 
 
+@pytest.mark.parametrize("name,field,conv,usual,most", [
+    ("counts past 64", SMALL, (0.6, 7, 5), 63, 224),
+    ("all counts past 64", dict(rows=24, cols=36, rooms=2, margin=4, seed=4), (0.9, 8, 5), 0, 179),
+    ("usual count of six bits", SMALL, (0.6, 3, 5), 48, 48),
+    ("distance 1", SMALL, (0.3, 1, 5), 8, 8),
+    ("counts read from HBM", dict(rows=310, cols=268, rooms=2, margin=6, seed=4), (0.6, 2, 9), 24, 24),
+])
+def test_gpu_field_env_conv_counts(tmp_path, name, field, conv, usual, most):
+    """The plan kernel's walk by candidate counts: whole swaps recorded for the
+    commonest count of 2 to 64 (here with six-bit candidates, or none), other
+    counts up to 224 (eight-bit draws), and a room of 46,872 cells, past the
+    46,703 whose counts fit in LDS. Exact mode, bit-identical to the oracle."""
+    blob = field_blob(tmp_path, field, 2 if field["rooms"] > 2 else 1, 2, conv=conv)
+    d = read_sbb(blob)
+    counts = np.diff(d["conv_cand_offsets"])
+    small = np.bincount(counts[(counts >= 2) & (counts <= 64)], minlength=65)
+    assert counts.max() == most and (int(small.argmax()) if small.any() else 0) == usual
+    room = int(np.diff(d["conv_room_offsets"]).max())
+    assert (room > 46703) == ("HBM" in name)
+    say(f"{name}: 3 envs, rooms of up to {room} cells, convection {conv}, exact field mode, 6 steps")
+    vec = E.VecEnv(3, blob=str(blob), max_steps=100, field_exact=1)
+    twins = [Twin(vec, i, 100) for i in range(3)]
+    run_against_oracle(vec, twins, 6, True, name)
+    vec.close()
+
+
 def test_gpu_field_env_default_mode_full_size(tmp_path):
     """building_train_1's size (205,434 cells) with the shipped buildings'
     convection, default field mode, 300 envs (the field group then runs two
