@@ -456,8 +456,9 @@ typedef struct {
     int n_envs, envs_per_block, n_blocks;
     int levels_l, levels_u;       /* level-schedule depth of the two sweeps */
     long long nnz_l, nnz_u;       /* off-diagonal factor entries */
-    double bytes_per_step;        /* algorithmic HBM bytes of one batched step */
-    double flops_per_step;        /* multiply-adds x 2 of the solves and the air-side combination */
+    double bytes_per_step;        /* HBM bytes of one batched step as its mode computes it, each table read once */
+    double flops_per_step;        /* its multiply-adds x 2: the fronts' dense products and the air-side
+                                     combination (default), or the factors' terms in two solves (exact) */
     int tail_rows_l, tail_rows_u;       /* rows in fronts above the leaves (0: exact mode) */
     int tail_levels_l, tail_levels_u;   /* heights of the tree of fronts above the leaves (0: exact mode) */
     int chunked_levels_l, chunked_levels_u;   /* always 0 */

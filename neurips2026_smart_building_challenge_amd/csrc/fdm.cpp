@@ -557,20 +557,30 @@ bool build(SbxFdm* f, const char* path, int G, int epb, int flags) {
     I.tail_rows_l = I.tail_rows_u = T.fast ? n - T.ft.n_leaf : 0;
     I.tail_levels_l = I.tail_levels_u = T.fast ? T.ft.n_levels - 1 : 0;
     I.chunked_levels_l = I.chunked_levels_u = 0;
-    // algorithmic HBM bytes of one batched step: both factors read once per
-    // solve for the whole group (value + column per term, U's diagonal, row
-    // ids and row pointers: shared by every env, however the blocks re-read
-    // them); per env the heat input, the field read (solved cells) and
-    // written (all cells), the mass read and written, and each solve's vector
-    // read and written once per sweep
-    // (two solves in exact mode; in the default mode one, plus R read once and
-    // its k-term combination per env and solved cell)
-    const double solves = T.R ? 1.0 : 2.0;
-    const double per_solve = 12.0 * (double)(L.nnz + U.nnz) + 8.0 * n + 2.0 * 8.0 * n;
-    const double per_env = 8.0 * ((double)n_cvs + n + n_cvs + 2.0 * n) + solves * (2.0 * 2.0 * 8.0 * n);
-    const double r_bytes = T.R ? 8.0 * (double)k * n : 0.0;
-    I.bytes_per_step = solves * per_solve + r_bytes + (double)G * per_env;
-    I.flops_per_step = (double)G * (solves * 2.0 * (double)(L.nnz + U.nnz) + (T.R ? 2.0 * (double)k * n : 0.0));
+    // algorithmic HBM bytes and multiply-adds x 2 of one batched step. Per env
+    // the heat input, the field read (solved cells) and written (all cells) and
+    // the mass read and written, in both modes
+    const double cells = 8.0 * ((double)n_cvs + n + n_cvs + 2.0 * n);
+    if (T.fast) {
+        // the operators (zeros past a front's rows and columns included) and R
+        // once; per env W written and read up the tree (the leaves' rows down it
+        // too), Y, C and X written and read, X at the fronts' boundaries as well.
+        // Multiply-adds: the operators' own entries and R's
+        const double ny = n - T.ft.n_leaf, nc = T.ft.n_c;
+        double entries = 0.0;
+        for (const sbf::Front& q : fp.fronts) entries += (double)q.w * (q.w + 2.0 * q.r);
+        const double vectors = 8.0 * (4.0 * n + T.ft.n_leaf + 2.0 * ny + 3.0 * nc);
+        I.bytes_per_step = 8.0 * (double)fp.ops + 8.0 * (double)k * n + (double)G * (cells + vectors);
+        I.flops_per_step = 2.0 * (double)G * (entries + (double)k * n);
+    } else {
+        // two solves: both factors read once for the whole group (value + column
+        // per term, U's diagonal, row ids and row pointers: shared by every env,
+        // however the blocks re-read them), each solve's vector read and written
+        // once per sweep
+        const double per_solve = 12.0 * (double)(L.nnz + U.nnz) + 8.0 * n + 2.0 * 8.0 * n;
+        I.bytes_per_step = 2.0 * per_solve + (double)G * (cells + 2.0 * (2.0 * 2.0 * 8.0 * n));
+        I.flops_per_step = (double)G * 2.0 * 2.0 * (double)(L.nnz + U.nnz);
+    }
     return true;
 }
 
