@@ -12,11 +12,13 @@
 //               the boiler update (it reads only pre-step values), and the
 //               field step's inputs: heat per room cell of each zone, air-side
 //               conductance and supply temperature per column, ambient, h;
-//   conv plan   (stochastic convection on) one wavefront per env: the
-//               convection stream's swap decisions of the step, which depend
-//               on no temperature, composed per room into a permutation and
-//               listed as (cell, source cell) moves;
-//   field       the FDM step on the whole group (fdm_kernel.hip);
+//   conv plan   (stochastic convection on) one workgroup of three wavefronts
+//               per env, on a side stream: the convection stream's swap
+//               decisions of the step, which depend on no temperature,
+//               composed per room into a permutation and listed as (cell,
+//               source cell) moves;
+//   field       the FDM step on the whole group (fdm_front_kernel.hip; in
+//               exact mode fdm_kernel.hip);
 //   conv apply  the listed moves, gathered then scattered;
 //   means       each zone's mean over its room's cells, lane per (zone, env);
 //   hvac(post)  one wavefront per env: observation (lanes over fields),

@@ -1,16 +1,19 @@
-"""The building-scale field step on the GPU (sbx_fdm_*, csrc/fdm_kernel.hip)
-against the oracle (oracle/sbo_fdm.c, itself bit-identical to the reference
-core) and the reference core's fixture (tests/golden/fdm.json), in both
-modes: exact (every level in the reference's order) and the default one (the
-deep end of each sweep solved in LDS with reassociated sums):
+"""The building-scale field step on the GPU (sbx_fdm_*, csrc/fdm_kernel.hip
+and csrc/fdm_front_kernel.hip) against the oracle (oracle/sbo_fdm.c, itself
+bit-identical to the reference core) and the reference core's fixture
+(tests/golden/fdm.json), in both modes: exact (every level in the reference's
+order) and the default one (dense fronts along the elimination tree, their
+products on the matrix cores, sums in another order):
 
   - exact mode: bit-identical fields and interior mass after every step, on
     the small plan and on the plan at building_train_1's size (205,434 cells,
     152,334 solved, 39 rooms), for blocks of 1, 2 and 64 envs and a last block
     that is only partly filled;
   - default mode: the same runs within RTOL = 1e-9 relative (the north star's
-    per-step state bar) of the oracle and of the fixture's probe cells, with a
-    nonempty LDS tail on both plans;
+    per-step state bar) of the oracle and of the fixture's probe cells, with
+    fronts above the leaves on both plans; an env the same bit for bit alone
+    and in a batch, and where the solve takes the env tiles in passes; factors
+    whose fronts would be inaccurate run as in exact mode;
   - the sensed response S (solved on the device at open) and the factor solve
     of the baker's reference right-hand side, bit-identical to the oracle's;
   - the default mode's air-side responses (the applied columns solved at
@@ -381,12 +384,14 @@ def test_gpu_fdm_default_where_memory_is_short(full):
         assert np.array_equal(T[g], T0[g % small]) and np.array_equal(M[g], M0[g % small]), g
 
 
-@pytest.mark.parametrize("G", [40, 300])
+@pytest.mark.parametrize("G", [17, 40, 300])
 def test_gpu_fdm_full_size_default_every_cell(full, G):
     """The default configuration (envs_per_block 0, default mode) at
-    building_train_1's size: one env per block at 40 envs, two per block at
-    300 (more envs than the GPU's compute units). Every cell of the field and
-    of the interior mass of seven envs (the first block, the middle, the last
+    building_train_1's size, in tiles of 16 envs: two tiles with one env in the
+    last (the leaves' two-tile kernel, every height above them narrow), three
+    with 8 in the last (an odd tile without a mate, the lowest height wide) and
+    nineteen with 12 (several heights wide). Every cell of the field and
+    of the interior mass of seven envs (the first ones, the middle, the last
     ones) within 1e-9 of the oracle after each of 3 steps with air sides on;
     envs are independent, so the oracle steps just those envs."""
     import torch

@@ -302,8 +302,8 @@ def test_gpu_field_env_conv_counts(tmp_path, name, field, conv, usual, most):
 
 def test_gpu_field_env_default_mode_full_size(tmp_path):
     """building_train_1's size (205,434 cells) with the shipped buildings'
-    convection, default field mode, 300 envs (the field group then runs two
-    envs per block), episodes of 3 steps: four envs against their oracle twins
+    convection, default field mode, 300 envs (nineteen tiles of the field solve,
+    the last of 12 envs), episodes of 3 steps: four envs against their oracle twins
     every step through two auto-resets: state within 1e-9, observations within
     float32 quantisation of the physics fields, rewards within 2 float32 ulps."""
     blob = field_blob(tmp_path, {}, 3, 3, conv=SHIPPED_CONV)
