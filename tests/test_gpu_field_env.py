@@ -300,6 +300,48 @@ def test_gpu_field_env_conv_counts(tmp_path, name, field, conv, usual, most):
     vec.close()
 
 
+def test_gpu_field_env_default_mode_inaccurate_fronts(tmp_path):
+    """The same building with its system factored after swapping the rows of 30 %
+    of its cells with a neighbour's and without pivoting back to the diagonal:
+    factors of the same solve that the default mode's fronts would serve to
+    about 1e-10. The field group then keeps the reference's order (blocks of
+    envs of its own default width) under an env that runs in default mode."""
+    import scipy.sparse.linalg as spla
+
+    from neurips2026_smart_building_challenge_amd.fdm import FieldGroup
+
+    A = F.make_plan(F.FdmSpec(**SMALL)).A.tocsr()
+    n, rng = A.shape[0], np.random.default_rng(0)
+    p, used = np.arange(n), np.zeros(n, bool)
+    for i in rng.permutation(n)[:int(0.3 * n)]:
+        near = [j for j in A.indices[A.indptr[i]:A.indptr[i + 1]] if j != i and not used[j]]
+        if not used[i] and near:
+            p[i], p[near[0]] = near[0], i
+            used[i] = used[near[0]] = True
+    lu = spla.splu(A[p].tocsc(), permc_spec="MMD_AT_PLUS_A", diag_pivot_thresh=0.0, options=dict(SymmetricMode=False))
+    spec = G.FieldEnvSpec(F.FdmSpec(**SMALL), 2)
+    w = G.field_env_writer(spec, G.climates()[1], G.EPISODE_STEPS + 256, 17321, G.ConvSpec(*SHIPPED_CONV))
+    new = {"lu_perm_r": (lu.perm_r[np.argsort(p)], "i32"), "lu_perm_c": (lu.perm_c, "i32")}
+    for name, M in (("lu_L", lu.L.tocsc()), ("lu_U", lu.U.tocsc())):
+        M.sort_indices()
+        new.update({f"{name}_indptr": (M.indptr, "i32"), f"{name}_indices": (M.indices, "i32"),
+                    f"{name}_data": (M.data, "f64")})
+    w._items = [it for it in w._items if it[0] not in new]
+    w._seen -= new.keys()
+    for name, (a, dtype) in new.items():
+        w.add(name, a, dtype)
+    blob = tmp_path / "swapped.sbb"
+    w.write(blob)
+    f = FieldGroup(blob, 3)
+    assert f.info.tail_rows_l == 0 and f.info.envs_per_block == 4
+    f.close()
+    say("3 envs, 7-room plan with swapped rows, default field mode, 30 steps")
+    vec = E.VecEnv(3, blob=str(blob), max_steps=20)
+    twins = [Twin(vec, i, 20) for i in range(3)]
+    run_against_oracle(vec, twins, 30, False, "swapped rows")
+    vec.close()
+
+
 def test_gpu_field_env_default_mode_full_size(tmp_path):
     """building_train_1's size (205,434 cells) with the shipped buildings'
     convection, default field mode, 300 envs (nineteen tiles of the field solve,
