@@ -154,7 +154,8 @@ bool hip_check(hipError_t e, const char* what) {
 
 // The default mode's vectors W1, X, Y and C in one allocation: for every env
 // tile, or, past kVectorBytes (some 2,500 envs of a 205K-cell plan), for an
-// equal share of them at a time; for fewer where the device has no room left.
+// equal share of them at a time; for fewer where the device has no room left
+// (whole blocks of Gl envs in any case).
 constexpr size_t kVectorBytes = (size_t)8 << 30;
 
 bool make_vectors(SbxFdm* f, sbf::Group* g) {
@@ -162,11 +163,12 @@ bool make_vectors(SbxFdm* f, sbf::Group* g) {
     const size_t n = t.n, ny = t.n - t.ft.n_leaf, nc = (size_t)t.ft.n_c + 1;
     const size_t tile = sizeof(double) * sbf::kEnvTile * (2 * n + ny + nc);
     const int most = (int)std::min<size_t>(g->nt, std::max<size_t>(kVectorBytes / tile, 1));
-    const int passes = (g->nt + most - 1) / most;
+    const int passes = (g->nt + most - 1) / most, unit = std::max(g->Gl / sbf::kEnvTile, 1);
+    auto whole = [&](int tiles) { return std::min((tiles + unit - 1) / unit * unit, g->nt); };
     double* p = nullptr;
-    for (g->tiles = (g->nt + passes - 1) / passes;; g->tiles = (g->tiles + 1) / 2) {
+    for (g->tiles = whole((g->nt + passes - 1) / passes);; g->tiles = whole((g->tiles + 1) / 2)) {
         p = (double*)dalloc(f, tile * g->tiles);
-        if (p || g->tiles == 1) break;
+        if (p || g->tiles <= unit) break;
         (void)hipGetLastError();   // (not the next launch's)
     }
     if (!p) return false;
@@ -188,7 +190,6 @@ bool make_group(SbxFdm* f, int G, int Gl, bool fields, sbf::Group* g) {
     const size_t lanes = (size_t)g->nblk * Gl;
     const bool fronts = fields && t.fast;   // the default mode's vectors, in tiles of envs
     g->nt = (G + sbf::kEnvTile - 1) / sbf::kEnvTile;
-    g->t0 = 0;
     g->tiles = g->nt;
     g->W1 = fronts ? nullptr : (double*)dalloc(f, sizeof(double) * lanes * t.n);
     const bool w2 = fields && !t.fast;   // the second solve's vector (exact mode)

@@ -140,8 +140,7 @@ struct Tables {
 
 struct Group {
     int G, Gl, nblk;
-    int nt;                 // env tiles, of the group or (in a launch of the default mode) of the pass
-    int t0, tiles;          // default mode: the pass's first env tile; the tiles that W1, X, Y and C hold
+    int nt;                 // env tiles
     double* T;              // [nblk][n_cvs][Gl]
     double* M;              // [nblk][n][Gl]
     // exact mode: the forcing solve in place, [nblk][n][Gl]; default mode: the
@@ -155,6 +154,7 @@ struct Group {
     double* mat;            // [G][k][k] I + diag(g) S
     int* eact;              // [G] env has a nonzero air-side conductance this step
     int* bact;              // [nblk] some env of the block has (exact mode; null in the default one)
+    int tiles, pad;         // the tiles that W1, X, Y and C hold (default mode)
 };
 
 // One batched step's inputs (device): input_q [G][n_cvs], ambient / h [G],

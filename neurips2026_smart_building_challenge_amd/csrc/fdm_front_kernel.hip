@@ -21,6 +21,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "fdm.h"
 
@@ -37,10 +38,13 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
 // acc[r][e] += A (row tile r) B (env tile e) over the steps [k0, k1): A from
 // the operator's tiles, B through load(step, e). U steps' loads are issued
 // before their products; the last U may run past k1 with zeros for A (a step
-// at a time there would be a memory latency each). `before(k)` runs ahead of step k's products.
-template <int RT, int NE, int U, class Load, class Before>
+// at a time there would be a memory latency each). `before(k)`, if given, runs ahead of step k's products.
+struct Nothing {
+    __device__ void operator()(int) const {}
+};
+template <int RT, int NE, int U, class Load, class Before = Nothing>
 __device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE],
-                                        Before before) {
+                                        Before before = {}) {
     for (int k = k0; k < k1; k += U) {
         double a[RT][U], b[NE][U];
 #pragma unroll
@@ -53,7 +57,7 @@ __device__ __forceinline__ void product(const double* const (&A)[RT], int k0, in
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            if (k + u < k1) before(k + u);
+            if (!std::is_same<Before, Nothing>::value && k + u < k1) before(k + u);
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 const double x = k + u < k1 ? a[r][u] : 0.0;
@@ -62,10 +66,6 @@ __device__ __forceinline__ void product(const double* const (&A)[RT], int k0, in
             }
         }
     }
-}
-template <int RT, int NE, int U, class Load>
-__device__ __forceinline__ void product(const double* const (&A)[RT], int k0, int k1, Load load, d4 (&acc)[RT][NE]) {
-    product<RT, NE, U>(A, k0, k1, load, acc, [](int) {});
 }
 
 // The leaves, a wavefront per (RT row tiles of a front, NE env tiles): up
@@ -174,10 +174,10 @@ constexpr int kShares = 8;
 // envs, from Y 47: there it
 // is bound by the products' operand traffic: 2 x 2 tiles.
 //
-// Four wavefronts a SIMD: left alone, the compiler takes registers for three
-// (the same two env steps 9.74 ms).
+// The wide form with four wavefronts a SIMD: left alone, the compiler takes
+// registers for three (the same two env steps 9.74 ms).
 template <bool DOWN, bool FUSED, int RT, int NE, int KW, int U>
-__global__ __launch_bounds__(64 * KW, 4) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
+__global__ __launch_bounds__(64 * KW, KW == kShares ? 1 : 4) void front_kernel(sbf::FrontTab t, int task0, int ntask, int n, int nt,
                                                         const double* __restrict__ W, double* __restrict__ Y,
                                                         double* C, double* X) {
     static_assert(!FUSED || (RT == 1 && NE == 1 && KW == kShares), "the fused form takes single tiles and shares");
@@ -512,7 +512,7 @@ __global__ __launch_bounds__(256) void front_forcing_kernel(sbf::Tables t, sbf::
     const int z = in.q ? -1 : t.czone[tt];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const int l = wave * 4 + q, env = (g.t0 + te) * E + l;
+        const int l = wave * 4 + q, env = te * E + l;
         double v = 0.0;
         if (env < g.G) {
             const size_t b = env / Gl, gl = env % Gl;
@@ -549,8 +549,7 @@ __global__ __launch_bounds__(kSensedThreads) void front_sensed_kernel(sbf::Table
     const int te = (int)(blockIdx.x % (unsigned)g.nt), i = (int)(blockIdx.x / (unsigned)g.nt);
     const int j = threadIdx.x % E, s = threadIdx.x / E;
     const double* Xb = g.X + (size_t)te * t.n * E + j;
-    const int env = (g.t0 + te) * E + j;
-    const double base = base_of(in.amb[min(env, g.G - 1)]);
+    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
     double acc = 0.0;
 #pragma unroll 8
     for (int p = t.sn_p[i] + s; p < t.sn_p[i + 1]; p += R) acc += t.sn_x[p] * (base + Xb[(size_t)t.ft.sn_w[p] * E]);
@@ -560,6 +559,7 @@ __global__ __launch_bounds__(kSensedThreads) void front_sensed_kernel(sbf::Table
         if (s < h) part[s][j] += part[s + h][j];
         __syncthreads();
     }
+    const int env = te * E + j;
     if (s == 0 && env < g.G) {
         const size_t x = (size_t)env * t.k + i;
         g.pw[x] = in.g[x] * (in.airT[x] - part[0][j]);
@@ -579,13 +579,13 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
     const int j = lane & 15, kk = lane >> 4;
     const int n = t.n, k = t.k, Gl = g.Gl;
     const double* Xb = g.X + (size_t)te * n * E + j;
-    const int e0 = (g.t0 + te) * E, ej = min(e0 + j, g.G - 1);
-    const double base = base_of(in.amb[ej]);
+    const double base = base_of(in.amb[min(te * E + j, g.G - 1)]);
     double y[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) y[q] = Xb[(size_t)t.ft.rx[min(t0 + wave * 16 + kk + 4 * q, n - 1)] * E];
     if (t.R) {
-        const double* qv = g.pw + (size_t)ej * k;
+        const int env = min(te * E + j, g.G - 1);
+        const double* qv = g.pw + (size_t)env * k;
         const double* Rb = t.R + min(t0 + wave * 16 + j, n - 1);   // A: row (cell) lane % 16
         d4 acc = {};
 #pragma unroll 5
@@ -594,7 +594,7 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
             const double a = col < k ? Rb[(size_t)min(col, k - 1) * n] : 0.0;
             acc = mfma(a, qv[min(col, k - 1)], acc);
         }
-        const bool on = g.eact[ej] != 0;
+        const bool on = g.eact[env] != 0;
 #pragma unroll
         for (int q = 0; q < 4; q++) y[q] = on ? y[q] + acc[q] : y[q];
     }
@@ -607,7 +607,7 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
         const double mr = t.mret[tt], mg = t.mgain[tt];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int l = wave * 4 + q, env = e0 + l;
+            const int l = wave * 4 + q, env = te * E + l;
             if (env >= g.G) break;
             const size_t b = env / Gl, gl = env % Gl, mi = (b * n + tt) * Gl + gl;
             const double v = ys[l][lane];
@@ -615,7 +615,6 @@ __global__ __launch_bounds__(256) void front_update_kernel(sbf::Tables t, sbf::G
             g.T[(b * t.n_cvs + cell) * Gl + gl] = v;
         }
     }
-    if (g.t0 != 0) return;   // the first pass writes every env's other cells
     const size_t tu = (size_t)g.nblk * t.n_unsolved * Gl;
     for (size_t x = (size_t)blockIdx.x * 256 + threadIdx.x; x < tu; x += (size_t)gridDim.x * 256) {
         const size_t bu = x / Gl;
@@ -694,14 +693,29 @@ int launch_pass(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in
 }  // namespace
 
 // One batched step of a group in the default mode, in passes over the env
-// tiles that the vectors hold (an env's result does not depend on its pass).
+// tiles that the vectors hold: a pass is a group of its own envs, its arrays
+// and inputs from its first env on (an env's result does not depend on its pass).
 extern "C" int sbf_launch_front_step(const sbf::Tables* t, const sbf::Group* group, const sbf::StepIn* in,
                                      hipStream_t s) {
-    for (int t0 = 0; t0 < group->nt; t0 += group->tiles) {
-        sbf::Group pass = *group;
-        pass.t0 = t0;
-        pass.nt = std::min(group->tiles, group->nt - t0);
-        if (int e = launch_pass(t, &pass, in, s)) return e;
+    const size_t k = t->k, Gl = group->Gl;
+    for (int e0 = 0; e0 < group->G; e0 += group->tiles * E) {   // (a multiple of Gl)
+        sbf::Group p = *group;
+        p.G = std::min(group->G - e0, group->tiles * E);
+        p.nblk = (p.G + p.Gl - 1) / p.Gl;
+        p.nt = (p.G + E - 1) / E;
+        p.T += e0 / Gl * t->n_cvs * Gl;
+        p.M += e0 / Gl * t->n * Gl;
+        p.pw += e0 * k;
+        p.mat += e0 * k * k;
+        p.eact += e0;
+        sbf::StepIn q = *in;
+        if (q.q) q.q += (size_t)e0 * t->n_cvs;
+        if (q.qz) q.qz += (size_t)e0 * t->nz;
+        if (q.g) q.g += e0 * k;
+        if (q.airT) q.airT += e0 * k;
+        q.amb += e0;
+        q.h += e0;
+        if (int e = launch_pass(t, &p, &q, s)) return e;
     }
     return 0;
 }

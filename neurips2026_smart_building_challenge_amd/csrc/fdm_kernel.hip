@@ -150,7 +150,7 @@ __global__ void sensed_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
 // back-substitutes.
 __global__ __launch_bounds__(64) void dense_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
     __shared__ int s_piv, s_sing;
-    const int env = g.t0 * sbf::kEnvTile + (int)blockIdx.x, k = t.k, lane = threadIdx.x;
+    const int env = blockIdx.x, k = t.k, lane = threadIdx.x;
     const double* gv = in.g + (size_t)env * k;
     int any = 0;
     for (int i = lane; i < k; i += 64) any |= gv[i] != 0.0;
@@ -259,7 +259,7 @@ constexpr size_t dense_lds_bytes(int k) { return sizeof(double) * ((size_t)k * (
 template <bool EXACT, int RW>
 __global__ __launch_bounds__(kDenseThreads) void dense_lds_kernel(sbf::Tables t, sbf::Group g, sbf::StepIn in) {
     extern __shared__ __align__(16) double M[];   // [k + 1][k], then the pivots [k]
-    const int env = g.t0 * sbf::kEnvTile + (int)blockIdx.x, k = t.k, tid = threadIdx.x, lane = tid & 63;
+    const int env = blockIdx.x, k = t.k, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int NW = kDenseThreads / 64;
     const double* gv = in.g + (size_t)env * k;
@@ -514,17 +514,16 @@ int solve(const sbf::Tables& t, const sbf::Group& g, double* W, const int* bact,
 // Whether each env's air side is on and, where it is, its power row solved.
 extern "C" int sbf_launch_dense(const sbf::Tables* t, const sbf::Group* g, const sbf::StepIn* in, hipStream_t s) {
     const size_t lds = dense_lds_bytes(t->k);
-    const int envs = std::min(g->G - g->t0 * sbf::kEnvTile, g->nt * sbf::kEnvTile);   // (all of them, or the pass's)
     if (t->k <= 64 && t->fast)
-        hipLaunchKernelGGL((dense_lds_kernel<false, 1>), dim3(envs), dim3(kDenseThreads), lds, s, *t, *g, *in);
+        hipLaunchKernelGGL((dense_lds_kernel<false, 1>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
     else if (t->k <= 64)
-        hipLaunchKernelGGL((dense_lds_kernel<true, 1>), dim3(envs), dim3(kDenseThreads), lds, s, *t, *g, *in);
+        hipLaunchKernelGGL((dense_lds_kernel<true, 1>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
     else if (t->k <= kDenseLdsK && t->fast)
-        hipLaunchKernelGGL((dense_lds_kernel<false, 2>), dim3(envs), dim3(kDenseThreads), lds, s, *t, *g, *in);
+        hipLaunchKernelGGL((dense_lds_kernel<false, 2>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
     else if (t->k <= kDenseLdsK)
-        hipLaunchKernelGGL((dense_lds_kernel<true, 2>), dim3(envs), dim3(kDenseThreads), lds, s, *t, *g, *in);
+        hipLaunchKernelGGL((dense_lds_kernel<true, 2>), dim3(g->G), dim3(kDenseThreads), lds, s, *t, *g, *in);
     else
-        hipLaunchKernelGGL(dense_kernel, dim3(envs), dim3(64), 0, s, *t, *g, *in);
+        hipLaunchKernelGGL(dense_kernel, dim3(g->G), dim3(64), 0, s, *t, *g, *in);
     return (int)hipGetLastError();
 }
 

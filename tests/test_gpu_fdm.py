@@ -346,16 +346,18 @@ def test_gpu_fdm_default_independent_of_batch(full):
             assert np.array_equal(Ts[i], T[g]) and np.array_equal(Ms[i], M[g]), (len(envs), g)
 
 
-def test_gpu_fdm_default_where_memory_is_short(full):
+@pytest.mark.parametrize("epb", [0, 64])
+def test_gpu_fdm_default_where_memory_is_short(full, epb):
     """A group whose field fits the device, the solve's vectors for all of its
     envs not: 1,000 envs of the full-size plan beside an allocation that leaves
     about 1.2 GB for vectors of 3.4 GB. The steps then take a share of the env
-    tiles at a time: every env equals its twin of a group of 24 bit for bit."""
+    tiles at a time (whole blocks of envs_per_block): every env equals its twin
+    of a group of 24 bit for bit."""
     import torch
 
     plan, path, _ = full
     G, small = 1000, 24
-    say(f"full-size plan, {G} envs with little device memory left")
+    say(f"full-size plan, {G} envs, envs_per_block {epb}, with little device memory left")
     inputs = [device_inputs(F.step_inputs(plan, small, 83, s)) for s in range(2)]
     f = gpu_group(path, small, 0, exact=False)
     for inp in inputs:
@@ -371,7 +373,7 @@ def test_gpu_fdm_default_where_memory_is_short(full):
     rest = torch.empty(torch.cuda.mem_get_info()[0] - (state + tables + (1200 << 20)), dtype=torch.uint8, device="cuda")
     assert torch.cuda.mem_get_info()[0] < state + tile * ((G + 15) // 16)
     try:
-        f = gpu_group(path, G, 0, exact=False)
+        f = gpu_group(path, G, epb, exact=False)
         for inp in inputs:
             f.step(*inp)
         torch.cuda.synchronize()
